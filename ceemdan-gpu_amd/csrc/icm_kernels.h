@@ -203,6 +203,48 @@ template <typename real>
 hipError_t launch_adj_input(int nchan, const int* chan_len, const int64_t* chan_off, const real* y,
                             const real* gxt, real* gy, hipStream_t st);
 
+// ------------------------------------------------- whole stages (icm_resident.hip)
+// Knot structure of one pass written by a stage that keeps records.
+struct StageRec {
+    uint64_t* mask;
+    int *left, *right, *cnt, *pre, *n, *fixf;
+    int* winlist;
+    unsigned* wincount;
+};
+
+template <typename real>
+struct StageArgs {
+    SeriesDev sd;           // sd.len == nullptr: equal series of uniform_len samples, back to back
+    int uniform_len;
+    int nseries;
+    InitArgs<real> ia;
+    real *hA, *hB;          // sample buffers of the phase (series offsets)
+    real* out;              // FIXED: the stage output (series offsets)
+    int passes;             // FIXED: subtractions; RILLING: cap
+    int nak;
+    int rilling;
+    int need_out;           // 0: only the records are wanted
+    int* nk_out;            // optional [nseries][2] knot counts of the first pass input
+    const StageRec* rec;    // optional [passes]
+    int *stop_pass, *subs;  // RILLING
+    char* scratch;          // knot rows of every workgroup that do not fit LDS
+    int64_t slot_bytes;
+    int lds_bytes;
+};
+
+// Launch shape of a phase: waves per workgroup, one tile per wave or more,
+// workgroups, their LDS, and the scratch of each for passes whose knot rows
+// do not fit it.  ok = false: the series are too long.
+struct StageGeom {
+    bool ok, hold;
+    int nwv;
+    size_t lds, slot;
+    int64_t grid;
+};
+StageGeom stage_geometry(int real_size, int64_t max_len, int64_t nseries);
+template <typename real>
+hipError_t launch_stage(const StageArgs<real>& a, const StageGeom& g, hipStream_t st);
+
 // host-side launchers (icm_kernels.hip)
 // loop = true: the grid-stride instance even where one wavefront per run of
 // tiles fits a launch (for testing that instance)

@@ -262,6 +262,17 @@ struct PlanBase {
     bool overlap_on = true;
     bool sift_queue = false;          // every sift pass from a work queue (ICM_SIFT_QUEUE=1)
     bool grid_loop = false;           // grid-stride start / adjoint tile (ICM_GRID_LOOP=1)
+    // whole stages of short series, one workgroup per series
+    StageGeom sgeom[2] = {};
+    char* sscratch[2] = {nullptr, nullptr};
+    bool geometry_set = false;        // icm_set_tuning chose the sift geometry
+    // The stage kernel runs unless a caller asks for what only the
+    // launch-per-step path has: sift geometries being timed or set, traces,
+    // per-kernel times.
+    bool whole_stages(int phase) const
+    {
+        return sgeom[phase].ok && !tuning && !geometry_set && !trace_passes && !prof;
+    }
     int* h_err = nullptr;             // pinned
     // rilling
     int *active = nullptr, *stop_pass = nullptr, *subs = nullptr, *sx_cnt = nullptr,
@@ -409,6 +420,8 @@ struct PlanBase {
         tune_left = n;
         if (n > 0 && tune_table_get(tkey[0], choice[0]) && tune_table_get(tkey[1], choice[1]))
             tune_left = 0;
+        else if (sgeom[0].ok && sgeom[1].ok)
+            tune_left = 0;   // nothing to choose: no sift launches
         else if (tune_left > 0)
             for (int ph = 0; ph < 2; ++ph) choice[ph].assign(M - 1, -1);
     }
@@ -422,6 +435,7 @@ struct PlanBase {
         }
         tune_left = forwards;
         tune_round = 0;
+        geometry_set = false;
         drop_graphs();
         return ICM_OK;
     }
@@ -439,6 +453,7 @@ struct PlanBase {
         for (int64_t k = 0; k < count; ++k)
             if (in[k] < -1 || in[k] >= kNCand) return ICM_ERR_INVALID_ARG;
         for (int64_t k = 0; k < count; ++k) choice[phase][k] = in[k];
+        geometry_set = true;
         tune_left = 0;
         drop_graphs();
         return ICM_OK;
@@ -559,6 +574,17 @@ struct PlanBase {
         if (h_n_active) (void)hipHostFree(h_n_active);
         if (h_err) (void)hipHostFree(h_err);
         if (own) (void)hipStreamDestroy(own);
+        drop_stage_scratch();
+    }
+    void drop_stage_scratch()
+    {
+        for (int ph = 0; ph < 2; ++ph)
+            if (sscratch[ph]) {
+                (void)hipFree(sscratch[ph]);
+                bytes -= (int64_t)sgeom[ph].slot * sgeom[ph].grid;
+                sscratch[ph] = nullptr;
+                sgeom[ph].ok = false;
+            }
     }
 };
 
@@ -696,6 +722,8 @@ struct Plan : PlanBase {
     int64_t sparse_dense_max = -1;     // over-full tiles tolerated by them (-1: tiles / 64)
     std::vector<Rec> rec;                  // re-sift records of one stage (backward)
     std::vector<std::vector<Rec>> krec;    // per stage, kept by the forward (keep_records)
+    StageRec* rec_dev = nullptr;           // the same as device tables [passes]
+    std::vector<StageRec*> krec_dev;
     std::vector<char> krec_valid;
     real *mu = nullptr, *mom = nullptr, *edge = nullptr, *ga = nullptr, *gr = nullptr,
          *gacc = nullptr, *dots = nullptr, *gy = nullptr;
@@ -744,8 +772,9 @@ struct Plan : PlanBase {
         }
         if (cfg.keep_records && cfg.stop_mode == ICM_STOP_FIXED) {
             krec.resize(M - 1);
+            krec_dev.assign(M - 1, nullptr);
             for (int k = 0; k < M - 1; ++k)
-                if ((rc = alloc_recs(krec[k]))) return rc;
+                if ((rc = alloc_recs(krec[k], &krec_dev[k]))) return rc;
             krec_valid.assign(M - 1, 0);
         }
         if (hipHostMalloc((void**)&h_n_active, 2 * sizeof(unsigned), hipHostMallocDefault) !=
@@ -773,8 +802,39 @@ struct Plan : PlanBase {
         // grid-stride loops (else only where one wavefront per item would
         // exceed a launch's 2^32 work-items)
         if (const char* env = std::getenv("ICM_GRID_LOOP")) grid_loop = std::atoi(env) != 0;
+        setup_whole_stages();
         tune_init();
         return ICM_OK;
+    }
+
+    // Launch shapes of the stage kernel, and its scratch where the knot rows
+    // do not fit LDS.  The scratch is an extra: a plan that leaves little
+    // memory goes without (and keeps the launch-per-step path).
+    // ICM_WHOLE_STAGES=0 turns the stage kernel off.
+    void setup_whole_stages()
+    {
+        if (const char* env = std::getenv("ICM_WHOLE_STAGES"))
+            if (std::atoi(env) == 0) return;
+        for (int ph = 0; ph < 2; ++ph) {
+            const DevSeries& d = ph == ICM_PHASE_NOISE ? dn : dsig;
+            StageGeom g = stage_geometry((int)sizeof(real), d.max_len, d.nseries);
+            // a stage of a few passes does not repay the allocation
+            const int passes = ph == ICM_PHASE_NOISE ? cfg.noise_max_sifts : cfg.max_sifts;
+            if (g.slot && passes < 4) g.ok = false;
+            if (g.ok && g.slot) {
+                const int64_t need = (int64_t)g.slot * g.grid;
+                size_t fr = 0, tot = 0;
+                if (hipMemGetInfo(&fr, &tot) != hipSuccess || need > (int64_t)fr / 16 ||
+                    hipMalloc((void**)&sscratch[ph], (size_t)need) != hipSuccess) {
+                    (void)hipGetLastError();
+                    sscratch[ph] = nullptr;
+                    g.ok = false;
+                } else {
+                    bytes += need;
+                }
+            }
+            sgeom[ph] = g;
+        }
     }
 
     int alloc_lane(Lane& L, const HostSeries& h)
@@ -905,6 +965,20 @@ struct Plan : PlanBase {
         return ICM_OK;
     }
 
+    StageArgs<real> stage_args(int phase, const DevSeries& d, const InitArgs<real>& ia)
+    {
+        StageArgs<real> a{};
+        a.sd = d.view(ln[phase].kstride, cap);
+        a.nseries = d.nseries;
+        a.ia = ia;
+        a.hA = ln[phase].hA;
+        a.hB = ln[phase].hB;
+        a.nak = cfg.boundary == ICM_BOUNDARY_NOT_A_KNOT;
+        a.need_out = 1;
+        a.scratch = sscratch[phase];
+        return a;
+    }
+
     // Sift one stage of a phase, FIXED mode: init + S x (solve, sift).
     // The stage output (h after S subtractions) ends in `out` if given
     // (series offsets), else in buffer S % 2.
@@ -913,11 +987,24 @@ struct Plan : PlanBase {
     // h_out: the first pass reads the noise residual itself); null = L.hA.
     int stage_fixed(int phase, int stage, const DevSeries& d, const InitArgs<real>& ia, int S,
                     real* out, hipStream_t st, Rec* record = nullptr, bool full = false,
-                    real* h0 = nullptr)
+                    real* h0 = nullptr, int* nk_out = nullptr)
     {
         Lane& L = ln[phase];
         const SeriesDev sd = d.view(L.kstride, cap);
         int rc;
+        if (whole_stages(phase)) {
+            StageArgs<real> a = stage_args(phase, d, ia);
+            a.passes = S;
+            a.out = out ? out : (S & 1 ? L.hB : L.hA);
+            a.need_out = !record || full;
+            a.nk_out = nk_out;
+            if (record) {
+                a.rec = record == rec.data() ? rec_dev : krec_dev[stage];
+                ICM_TRY(launch_fill_u32((uint32_t*)record[0].wincount, 0u, S, st));
+            }
+            ICM_TRY(launch_stage<real>(a, sgeom[phase], st));
+            return ICM_OK;
+        }
         if (L.epoch + (uint32_t)S + 8 >= kEpochs - 1 && (rc = reset_control(L, st))) return rc;
         const int64_t pass_bytes = 2 * (int64_t)sizeof(real) * d.samples;
         real* in0 = h0 ? h0 : L.hA;
@@ -998,6 +1085,18 @@ struct Plan : PlanBase {
     {
         Lane& L = ln[phase];
         const SeriesDev sd = d.view(L.kstride, cap);
+        if (whole_stages(phase)) {
+            StageArgs<real> sa = stage_args(phase, d, ia);
+            sa.rilling = 1;
+            sa.passes = max_pass;
+            sa.stop_pass = stop_pass;
+            sa.subs = subs;
+            ICM_TRY(launch_stage<real>(sa, sgeom[phase], st));
+            if (stops[phase])
+                ICM_TRY(launch_copy<float>((float*)(stops[phase] + (int64_t)stage * d.nseries),
+                                           (const float*)subs, d.nseries, st));
+            return ICM_OK;
+        }
         ICM_TRY(launch_fill_u32((uint32_t*)active, 1u, d.nseries, st));
         ICM_TRY(launch_fill_u32((uint32_t*)subs, 0u, d.nseries, st));
         ICM_TRY(launch_fill_u32((uint32_t*)stop_pass, 0u, d.nseries, st));
@@ -1521,11 +1620,13 @@ struct Plan : PlanBase {
         return ICM_OK;
     }
 
-    int alloc_recs(std::vector<Rec>& out)
+    int alloc_recs(std::vector<Rec>& out, StageRec** table)
     {
         const int S = cfg.max_sifts;
         int rc;
         std::vector<Rec> rr(S);
+        unsigned* wc = nullptr;
+        if ((rc = alloc(&wc, S))) return rc;
         for (int j = 0; j < S; ++j) {
             if ((rc = alloc(&rr[j].mask, 8 * (int64_t)dsig.ntiles))) return rc;
             if ((rc = alloc(&rr[j].left, 2 * (int64_t)dsig.ntiles))) return rc;
@@ -1535,25 +1636,41 @@ struct Plan : PlanBase {
             if ((rc = alloc(&rr[j].n, 2 * (int64_t)dsig.nseries))) return rc;
             if ((rc = alloc(&rr[j].fixf, 4 * (int64_t)dsig.nseries))) return rc;
             if ((rc = alloc(&rr[j].winlist, (int64_t)kWinItem * dsig.maxwin))) return rc;
-            if ((rc = alloc(&rr[j].wincount, 1))) return rc;
+            rr[j].wincount = wc + j;
         }
+        std::vector<StageRec> dev(S);
+        for (int j = 0; j < S; ++j)
+            dev[j] = StageRec{rr[j].mask, rr[j].left, rr[j].right, rr[j].cnt, rr[j].pre,
+                              rr[j].n, rr[j].fixf, rr[j].winlist, rr[j].wincount};
+        if ((rc = upload(table, dev))) return rc;
         out.swap(rr);
         return ICM_OK;
     }
 
     int backward_alloc()
     {
-        if (mu) return ICM_OK;
+        int rc = backward_buffers();
+        if (rc == ICM_ERR_OUT_OF_MEMORY && (sscratch[0] || sscratch[1])) {
+            // the stage kernel's scratch makes room
+            (void)hipGetLastError();
+            drop_stage_scratch();
+            drop_graphs();
+            rc = backward_buffers();
+        }
+        return rc;
+    }
+    int backward_buffers()
+    {
         const int M = cfg.num_imfs;
         int rc;
-        if ((rc = alloc(&mu, dsig.samples))) return rc;
-        if ((rc = alloc(&mom, 8 * ln[ICM_PHASE_SIGNAL].kstride))) return rc;
-        if ((rc = alloc(&edge, 16 * (int64_t)dsig.ntiles))) return rc;
-        if ((rc = alloc(&ga, 2 * ln[ICM_PHASE_SIGNAL].kstride))) return rc;
-        if ((rc = alloc(&gr, (int64_t)M * chan_total))) return rc;
-        if ((rc = alloc(&gacc, chan_total))) return rc;
-        if ((rc = alloc(&dots, (int64_t)dsig.nseries))) return rc;
-        if ((rc = alloc(&gy, chan_total))) return rc;
+        if (!mu && (rc = alloc(&mu, dsig.samples))) return rc;
+        if (!mom && (rc = alloc(&mom, 8 * ln[ICM_PHASE_SIGNAL].kstride))) return rc;
+        if (!edge && (rc = alloc(&edge, 16 * (int64_t)dsig.ntiles))) return rc;
+        if (!ga && (rc = alloc(&ga, 2 * ln[ICM_PHASE_SIGNAL].kstride))) return rc;
+        if (!gr && (rc = alloc(&gr, (int64_t)M * chan_total))) return rc;
+        if (!gacc && (rc = alloc(&gacc, chan_total))) return rc;
+        if (!dots && (rc = alloc(&dots, (int64_t)dsig.nseries))) return rc;
+        if (!gy && (rc = alloc(&gy, chan_total))) return rc;
         return ICM_OK;
     }
 
@@ -1601,7 +1718,7 @@ struct Plan : PlanBase {
             if (!krec.empty() && krec_valid[k]) {
                 R = krec[k].data();   // kept by the forward
             } else {
-                if (rec.empty() && (rc = alloc_recs(rec))) return rc;
+                if (rec.empty() && (rc = alloc_recs(rec, &rec_dev))) return rc;
                 R = rec.data();
                 if ((rc = stage_fixed(ICM_PHASE_SIGNAL, k, dsig, ia, S, nullptr, st, R))) return rc;
             }
@@ -1674,8 +1791,10 @@ struct Plan : PlanBase {
         InitArgs<real> ia{};
         ia.mode = INIT_COPY;
         ia.src = h;
-        if ((rc = stage_fixed(ICM_PHASE_NOISE, 0, dn, ia, 1, hn, st))) return rc;
-        if (nk_out)
+        const bool whole = whole_stages(ICM_PHASE_NOISE);
+        if ((rc = stage_fixed(ICM_PHASE_NOISE, 0, dn, ia, 1, hn, st, nullptr, false, nullptr, nk_out)))
+            return rc;
+        if (nk_out && !whole)
             ICM_TRY(launch_copy<float>((float*)nk_out, (const float*)ln[ICM_PHASE_NOISE].nk[0],
                                        2 * dn.nseries, st));
         ICM_TRY(hipMemcpyAsync(h_err, err, sizeof(int), hipMemcpyDeviceToHost, st));
