@@ -194,11 +194,13 @@ hipError_t launch_adj_span_knot(const AdjArgs<real>& a, int solve_grid, hipStrea
 template <typename real>
 hipError_t launch_adj_seed(const real* gimf, int M, int64_t N, int64_t stride, real* gr,
                            hipStream_t st);
+// mean_k, sq_k: mean and std of r_k per channel (not read at stage 0)
 template <typename real>
 hipError_t launch_adj_stage(int stage, int nchan, int I, int max_len, const int* chan_len,
                             const int64_t* chan_off, const SeriesDev& sd, const real* gr_next,
-                            const real* mu, const real* E, const real* r_k, real eps0, real* gr_k,
-                            real* gacc, real* dots, hipStream_t st);
+                            const real* mu, const real* E, const real* r_k, const real* mean_k,
+                            const double* sq_k, real eps0, real* gr_k, real* gacc, real* dots,
+                            real* coef, hipStream_t st);
 template <typename real>
 hipError_t launch_adj_input(int nchan, const int* chan_len, const int64_t* chan_off, const real* y,
                             const real* gxt, real* gy, hipStream_t st);
@@ -265,26 +267,53 @@ hipError_t launch_rilling_decide(const SeriesDev& sd, const int* nk, const int* 
                                  const int* sx_mark, int* active, int* stop_pass, int* subs,
                                  int pass, int cap, const unsigned* run, unsigned* n_active,
                                  hipStream_t st);
+enum StatScale : int { SCALE_INV = 0, SCALE_STD = 1 };
 template <typename real>
-hipError_t launch_series_var(const real* base, const int64_t* off, int64_t stride,
-                             const int* len, int nser, real* var_out, hipStream_t st);
+hipError_t launch_series_var(const real* base, const int64_t* off, int64_t stride, const int* len,
+                             int nser, real* var_out, real* mean_out, double* scale_out, int scale,
+                             hipStream_t st);
 template <typename real>
-hipError_t launch_noise(uint64_t seed, int I, int64_t N, real* out, int64_t row_stride,
-                        hipStream_t st);
+hipError_t launch_noise(uint64_t seed, int I, int64_t N, real* out, hipStream_t st);
 template <typename real>
-hipError_t launch_ensemble(int stage, int nchan, int I, int max_len, const int* chan_len,
-                           const int64_t* chan_off, const int64_t* ser_off,
-                           const int64_t* ser_eoff, const int* ser_nidx, const real* hA, const real* hB,
-                           const int* mode_parity, int fixed_parity, const real* E,
-                           const double* inv, const double* sq, real eps0, const real* xt,
-                           real* r, real* imf_base, const int64_t* chan_imf_off, hipStream_t st);
+hipError_t launch_noise_groups(uint64_t seed, int I, int ngroups, int64_t max_len, const int* len,
+                               const int64_t* row_off, real* out, hipStream_t st);
+
+// r_{k+1} and IMF_k of every channel from the stage's realizations
 template <typename real>
-hipError_t launch_standardize(const real* y, const real* var, real* xt, int64_t N,
-                              hipStream_t st);
+struct EnsembleArgs {
+    int stage, I;
+    int last;                 // the residue is row M - 1 as well
+    const int* chan_len;
+    const int64_t* chan_off;
+    const int64_t* chan_imf_off;
+    const int64_t *ser_off, *ser_eoff;
+    const int* ser_nidx;
+    const real *hA, *hB;
+    const int* mode_parity;   // RILLING: per series, the buffer of its result
+    int fixed_parity;
+    const real* E;
+    const double *inv, *sq;
+    real eps0;
+    const real* xt;
+    real* r;
+    real* r_next;             // optional second copy of r_{k+1} (the adjoint's history)
+    real* imf;
+};
 template <typename real>
-hipError_t launch_inv_sqrt(const real* var, double* out, int n, int take_sqrt, hipStream_t st);
+hipError_t launch_ensemble(const EnsembleArgs<real>& a, int nchan, int max_len, hipStream_t st);
 template <typename real>
-hipError_t launch_sub(real* w, const real* e, int64_t n, hipStream_t st);
+hipError_t launch_standardize(const real* y, const real* var, real* xt, int nchan, int max_len,
+                              const int* chan_len, const int64_t* chan_off, hipStream_t st);
+
+// caller buffers of all channels into (in) or out of the plan's, kPtrBatch
+// channels per launch
+constexpr int kPtrBatch = 64;
+struct PtrBatch {
+    void* p[kPtrBatch];
+};
+template <typename real>
+hipError_t launch_channels(bool in, void* const* ptr, int nchan, int rows, int64_t max_len,
+                           const int* chan_len, const int64_t* off, real* own, hipStream_t st);
 template <typename real>
 hipError_t launch_copy(real* dst, const real* src, int64_t n, hipStream_t st);
 template <typename real>

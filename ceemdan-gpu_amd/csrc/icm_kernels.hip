@@ -709,24 +709,6 @@ __global__ __launch_bounds__(kThreads) void k_knot_prefix_w(SeriesDev sd, KnotsD
 
 // ------------------------------------------------------------- stage init
 
-template <typename real>
-__device__ __forceinline__ real init_value(const InitArgs<real>& ia, const SeriesDev& sd, int s,
-                                           int p)
-{
-    using P = typename Promote<real>::type;
-    if (ia.mode == INIT_COPY) return ia.src[sd.off[s] + p];
-    if (ia.mode == INIT_RESID) return ia.src[sd.off[s] + p] - ia.E[sd.off[s] + p];
-    const int c = sd.chan[s];
-    const real base = ia.chan_sig[ia.chan_off[c] + p];
-    const real e = ia.E[sd.eoff[s] + p];
-    if (ia.mode == INIT_STAGE0) {
-        // x_i = x~ + eps0 * E_1(w^i) * (1 / std(E_1(w^i)))   (cudaICEEMDAN.cu:76)
-        return (real)((P)base + (P)(ia.eps0 * e) * (P)ia.scale[sd.nidx[s]]);
-    }
-    // x_i = r_k + eps0 * E_{k+1}(w^i) * std(r_k)           (cudaICEEMDAN.cu:88)
-    return base + (ia.eps0 * e) * (real)ia.scale[c];
-}
-
 // ---------------------------------------------------------------- sift pass
 
 // ------------------------------------------------------- windowed spline solve
@@ -1049,40 +1031,92 @@ __global__ void k_rilling_decide(SeriesDev sd, const int* nk, const int* sx_cnt,
 
 // Canonical sum: lane l of 1024 adds x[l], x[l+1024], ... in order, then a
 // pairwise tree (same order as the oracle).  One workgroup per series.
+// The tree: the first wave's lane t combines the 16 partial sums of stride
+// 64 itself (strides 512 .. 64), then six steps inside the wave: two
+// workgroup barriers instead of one per level.
 template <typename real>
-__device__ real canon_sum_block(real acc, real* sred)
+__device__ __forceinline__ real canon_sum_block(real acc, real* sred)
 {
     const int tid = threadIdx.x;
     sred[tid] = acc;
     __syncthreads();
-    for (int st = 512; st >= 1; st >>= 1) {
-        if (tid < st) sred[tid] = sred[tid] + sred[tid + st];
-        __syncthreads();
+    if (tid < kWave) {
+        real v[16];
+#pragma unroll
+        for (int q = 0; q < 16; ++q) v[q] = sred[tid + kWave * q];
+#pragma unroll
+        for (int st = 8; st >= 1; st >>= 1)
+#pragma unroll
+            for (int q = 0; q < st; ++q) v[q] = v[q] + v[q + st];
+        real r = v[0];
+#pragma unroll
+        for (int st = 32; st >= 1; st >>= 1) r = r + shfl_down(r, st);
+        if (tid == 0) sred[0] = r;
     }
+    __syncthreads();
     const real r = sred[0];
     __syncthreads();
     return r;
 }
 
+// Sum over p = tid, tid + 1024, ... < N of f(loaded values), in order, the
+// loads of kSumAhead terms requested before the first is added: a lane's
+// chain is N / 1024 dependent adds, which took one memory round trip each
+// (244032 FP32 samples: 114 us for both passes of the variance).
+constexpr int kSumAhead = 16;
+template <typename real, class Load, class Term>
+__device__ __forceinline__ real canon_lane_sum(int N, Load load, Term term)
+{
+    real acc = (real)0;
+    int p = threadIdx.x;
+    for (; p + 1024 * (kSumAhead - 1) < N; p += 1024 * kSumAhead) {
+        decltype(load(0)) v[kSumAhead];
+#pragma unroll
+        for (int q = 0; q < kSumAhead; ++q) v[q] = load(p + 1024 * q);
+#pragma unroll
+        for (int q = 0; q < kSumAhead; ++q) acc = acc + term(v[q]);
+    }
+    // the last terms at clamped indices, so that their loads go out together
+    if (p < N) {
+        decltype(load(0)) v[kSumAhead];
+#pragma unroll
+        for (int q = 0; q < kSumAhead; ++q) v[q] = load(min(p + 1024 * q, N - 1));
+#pragma unroll
+        for (int q = 0; q < kSumAhead; ++q)
+            if (p + 1024 * q < N) acc = acc + term(v[q]);
+    }
+    return acc;
+}
+
+// Mean and unbiased variance (two passes) of every series, one workgroup
+// each; optionally the scale a stage start multiplies the noise with, as
+// double: 1 / std (SCALE_INV) or std (SCALE_STD).
 template <typename real>
 __global__ __launch_bounds__(1024) void k_series_var(const real* base, const int64_t* off,
-                                                     int64_t stride, const int* len, real* var_out)
+                                                     int64_t stride, const int* len, real* var_out,
+                                                     real* mean_out, double* scale_out, int scale)
 {
     __shared__ real sred[1024];
     const int s = blockIdx.x;
     const int64_t o = off ? off[s] : (int64_t)s * stride;
     const real* x = base + o;
     const int N = len ? len[s] : (int)stride;
-    real acc = (real)0;
-    for (int p = threadIdx.x; p < N; p += 1024) acc = acc + x[p];
-    const real mu = canon_sum_block<real>(acc, sred) * (real)(1.0 / (double)N);
-    acc = (real)0;
-    for (int p = threadIdx.x; p < N; p += 1024) {
-        const real dv = x[p] - mu;
-        acc = acc + dv * dv;
+    auto at = [&](int p) { return x[p]; };
+    const real mu = canon_sum_block<real>(canon_lane_sum<real>(N, at, [](real v) { return v; }), sred) *
+                    (real)(1.0 / (double)N);
+    const real ss = canon_sum_block<real>(canon_lane_sum<real>(N, at, [&](real v) {
+                                              const real dv = v - mu;
+                                              return dv * dv;
+                                          }), sred);
+    if (threadIdx.x == 0) {
+        const real var = ss * (real)(1.0 / (double)(N - 1));
+        if (var_out) var_out[s] = var;
+        if (mean_out) mean_out[s] = mu;
+        if (scale_out) {
+            const real sd = sqrt(var);
+            scale_out[s] = scale == SCALE_STD ? (double)sd : 1.0 / (double)sd;
+        }
     }
-    const real ss = canon_sum_block<real>(acc, sred);
-    if (threadIdx.x == 0) var_out[s] = ss * (real)(1.0 / (double)(N - 1));
 }
 
 // ------------------------------------------------- sift pass, wave per tile
@@ -1506,8 +1540,7 @@ __global__ __launch_bounds__(kThreads) void k_sift_list(SiftArgs<real> a, int ns
         sift_segment<real, RILL, kWKC>(b, segs, sid, lane, s_tab[wv]);
 }
 
-// Stage start for 256-sample tiles: forms x_i (the same arithmetic as
-// init_value) and stores its knots as bitmasks.  MODE is ia.mode as a
+// Stage start for 256-sample tiles: forms x_i and stores its knots as bitmasks.  MODE is ia.mode as a
 // compile-time constant: one straight-line body per mode.
 //
 // Per-series pointers and scales of the tile being formed.
@@ -2089,6 +2122,11 @@ __global__ void k_adj_seed(const real* gimf, int M, int N, int64_t stride, real*
         gr[(int64_t)k * stride + p] = gimf[(int64_t)k * N + p] - gimf[(int64_t)(k - 1) * N + p];
 }
 
+// Realizations whose samples are requested before the first is added, in the
+// sums over i (one at a time, a channel of 4096 samples and 50 realizations
+// took 21 us).
+constexpr int kEnsAhead = 8;
+
 // stage level: mu of every realization starts as dL/dr_{k+1} of its channel
 // g_x_i = (lambda - mu_i) / I; gacc = sum_i g_x_i (sequential in i)
 template <typename real>
@@ -2097,13 +2135,21 @@ __global__ void k_adj_accum(int I, const int* chan_len, const int64_t* chan_off,
 {
     const int c = blockIdx.y;
     const int p = blockIdx.x * blockDim.x + threadIdx.x;
-    if (p >= chan_len[c]) return;
+    const int N = chan_len[c];
+    if (p >= N) return;
     const real lam = gr_next[chan_off[c] + p];
+    // the channel's series lie back to back
+    const real* m = mu + sd.off[c * I] + p;
     real acc = (real)0;
-    for (int i = 0; i < I; ++i) {
-        const int s = c * I + i;
-        acc = acc + (lam - mu[sd.off[s] + p]) / (real)I;
+    int i = 0;
+    for (; i + kEnsAhead <= I; i += kEnsAhead) {
+        real v[kEnsAhead];
+#pragma unroll
+        for (int q = 0; q < kEnsAhead; ++q) v[q] = m[(int64_t)(i + q) * N];
+#pragma unroll
+        for (int q = 0; q < kEnsAhead; ++q) acc = acc + (lam - v[q]) / (real)I;
     }
+    for (; i < I; ++i) acc = acc + (lam - m[(int64_t)i * N]) / (real)I;
     gacc[chan_off[c] + p] = acc;
 }
 
@@ -2119,43 +2165,42 @@ __global__ __launch_bounds__(1024) void k_adj_dot(int I, SeriesDev sd, const int
     const real* lam = gr_next + chan_off[sd.chan[s]];
     const real* m = mu + sd.off[s];
     const real* e = E + sd.eoff[s];
-    real acc = (real)0;
-    for (int p = threadIdx.x; p < N; p += 1024) acc = acc + ((lam[p] - m[p]) / (real)I) * e[p];
+    struct T3 { real l, m, e; };
+    const real acc = canon_lane_sum<real>(
+        N, [&](int p) { return T3{lam[p], m[p], e[p]}; },
+        [&](const T3& t) { return ((t.l - t.m) / (real)I) * t.e; });
     const real d = canon_sum_block<real>(acc, sred);
     if (threadIdx.x == 0) dots[s] = d;
 }
 
-// gr_k += gacc (+ eps0 * sum_i dots * (r_k - mean) / ((N-1) std(r_k)), k >= 1)
+// coef[c] = eps0 sum_i dots / ((N - 1) std(r_k)) (sequential in i), one wave
+// per channel
 template <typename real>
-__global__ __launch_bounds__(1024) void k_adj_stage(int stage, int I, const int* chan_len,
-                                                    const int64_t* chan_off, const real* gacc,
-                                                    const real* dots, const real* r_k, real eps0,
-                                                    real* gr_k)
+__global__ __launch_bounds__(kWave) void k_adj_coef(int I, const int* chan_len, const real* dots,
+                                                    const double* sq, real eps0, real* coef)
 {
-    __shared__ real sred[1024];
-    const int c = blockIdx.x;
-    const int N = chan_len[c];
-    const int64_t o = chan_off[c];
-    real coef = (real)0, mu_r = (real)0;
-    if (stage > 0) {
-        real acc = (real)0;
-        for (int p = threadIdx.x; p < N; p += 1024) acc = acc + r_k[o + p];
-        mu_r = canon_sum_block<real>(acc, sred) * (real)(1.0 / (double)N);
-        acc = (real)0;
-        for (int p = threadIdx.x; p < N; p += 1024) {
-            const real dv = r_k[o + p] - mu_r;
-            acc = acc + dv * dv;
-        }
-        const real sq = sqrt(canon_sum_block<real>(acc, sred) * (real)(1.0 / (double)(N - 1)));
-        real dsum = (real)0;
-        for (int i = 0; i < I; ++i) dsum = dsum + dots[c * I + i];
-        coef = eps0 * dsum / ((real)(N - 1) * sq);
+    const int c = blockIdx.x, lane = threadIdx.x;
+    real dsum = (real)0;
+    for (int i0 = 0; i0 < I; i0 += kWave) {
+        const real v = i0 + lane < I ? dots[c * I + i0 + lane] : (real)0;
+        const int m = min(kWave, I - i0);
+        for (int l = 0; l < m; ++l) dsum = dsum + lane_value(v, l);
     }
-    for (int p = threadIdx.x; p < N; p += 1024) {
-        real v = gr_k[o + p] + gacc[o + p];
-        if (stage > 0) v = v + coef * (r_k[o + p] - mu_r);
-        gr_k[o + p] = v;
-    }
+    if (lane == 0) coef[c] = eps0 * dsum / ((real)(chan_len[c] - 1) * (real)sq[c]);
+}
+
+// gr_k += gacc (+ coef (r_k - mean(r_k)), k >= 1: coef is null at stage 0)
+template <typename real>
+__global__ void k_adj_stage(const int* chan_len, const int64_t* chan_off, const real* gacc,
+                            const real* coef, const real* mean, const real* r_k, real* gr_k)
+{
+    const int c = blockIdx.y;
+    const int p = blockIdx.x * blockDim.x + threadIdx.x;
+    if (p >= chan_len[c]) return;
+    const int64_t o = chan_off[c] + p;
+    real v = gr_k[o] + gacc[o];
+    if (coef) v = v + coef[c] * (r_k[o] - mean[c]);
+    gr_k[o] = v;
 }
 
 // dL/dy from dL/dx~ with x~ = y / std(y)
@@ -2167,18 +2212,17 @@ __global__ __launch_bounds__(1024) void k_adj_input(const int* chan_len, const i
     const int c = blockIdx.x;
     const int N = chan_len[c];
     const int64_t o = chan_off[c];
-    real acc = (real)0;
-    for (int p = threadIdx.x; p < N; p += 1024) acc = acc + y[o + p];
-    const real mu = canon_sum_block<real>(acc, sred) * (real)(1.0 / (double)N);
-    acc = (real)0;
-    for (int p = threadIdx.x; p < N; p += 1024) {
-        const real dv = y[o + p] - mu;
-        acc = acc + dv * dv;
-    }
-    const real var = canon_sum_block<real>(acc, sred) * (real)(1.0 / (double)(N - 1));
-    acc = (real)0;
-    for (int p = threadIdx.x; p < N; p += 1024) acc = acc + gxt[o + p] * y[o + p];
-    const real dot = canon_sum_block<real>(acc, sred);
+    auto at = [&](int p) { return y[o + p]; };
+    const real mu = canon_sum_block<real>(canon_lane_sum<real>(N, at, [](real v) { return v; }), sred) *
+                    (real)(1.0 / (double)N);
+    const real var = canon_sum_block<real>(canon_lane_sum<real>(N, at, [&](real v) {
+                                               const real dv = v - mu;
+                                               return dv * dv;
+                                           }), sred) * (real)(1.0 / (double)(N - 1));
+    struct T2 { real g, y; };
+    const real dot = canon_sum_block<real>(
+        canon_lane_sum<real>(N, [&](int p) { return T2{gxt[o + p], y[o + p]}; },
+                             [](const T2& t) { return t.g * t.y; }), sred);
     const real sx = (real)1 / sqrt(var);
     for (int p = threadIdx.x; p < N; p += 1024)
         gy[o + p] = sx * gxt[o + p] - sx * sx * sx * dot * (y[o + p] - mu) / (real)(N - 1);
@@ -2188,11 +2232,14 @@ __global__ __launch_bounds__(1024) void k_adj_input(const int* chan_len, const i
 
 // value (i, p): Philox4x64-10 block q = p/4, counter (q, i, 0, 0), key (seed, 0);
 // u = ((bits >> 11) + 0.5) * 2^-53; Box-Muller on (u0,u1) and (u2,u3).
+// One launch for the rows of several lengths: length blockIdx.z of `len`
+// (its rows from row_off[z]), or the one length N.
 template <typename real>
-__global__ void k_noise(uint64_t seed, int I, int64_t N, real* out, int64_t row_stride)
+__global__ void k_noise(uint64_t seed, const int* len, const int64_t* row_off, int64_t N, real* out)
 {
     const int i = blockIdx.y;
     const int64_t q = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+    if (len) N = len[blockIdx.z];
     if (4 * q >= N) return;
     const u64x4 b = philox4x64_10((uint64_t)q, (uint64_t)i, 0, 0, seed, 0);
     const double TWO_PI = 6.283185307179586476925286766559;
@@ -2206,7 +2253,7 @@ __global__ void k_noise(uint64_t seed, int I, int64_t N, real* out, int64_t row_
     z[1] = r0 * sin(TWO_PI * u[1]);
     z[2] = r1 * cos(TWO_PI * u[3]);
     z[3] = r1 * sin(TWO_PI * u[3]);
-    real* row = out + (int64_t)i * row_stride;
+    real* row = out + (row_off ? row_off[blockIdx.z] : 0) + (int64_t)i * N;
 #pragma unroll
     for (int j = 0; j < 4; ++j)
         if (4 * q + j < N) row[4 * q + j] = (real)z[j];
@@ -2222,83 +2269,94 @@ __device__ __forceinline__ real acc_stage0(real tem, double invI, real d)
     return (real)((double)tem + invI * (double)d);
 }
 
-template <typename real>
-__global__ void k_ensemble(int stage, int I, const int* chan_len, const int64_t* chan_off,
-                           const int64_t* ser_off, const int64_t* ser_eoff, const int* ser_nidx,
-                           const real* hA,
-                           const real* hB, const int* mode_parity, int fixed_parity, const real* E,
-                           const double* inv, const double* sq, real eps0, const real* xt,
-                           real* r, real* imf_base, const int64_t* chan_imf_off)
+// The loads of kEnsAhead realizations go out before the first is added.
+template <typename real, bool STAGE0>
+__global__ void k_ensemble(EnsembleArgs<real> a)
 {
     using P = typename Promote<real>::type;
     const int c = blockIdx.y;
-    const int N = chan_len[c];
+    const int N = a.chan_len[c];
     const int p = blockIdx.x * blockDim.x + threadIdx.x;
     if (p >= N) return;
-    const int64_t co = chan_off[c];
+    const int I = a.I;
+    const int64_t co = a.chan_off[c];
     // row `stage` of channel c's [M][N] output
-    real* imf_k = imf_base + chan_imf_off[c] + (int64_t)stage * N;
+    real* imf_k = a.imf + a.chan_imf_off[c] + (int64_t)a.stage * N;
+    // the channel's series and its noise rows lie back to back
     const int s0 = c * I;
+    const int64_t ho = a.ser_off[s0] + p;
+    const real* hs[2] = {a.hA + ho, a.hB + ho};
+    const real* e = a.E + a.ser_eoff[s0] + p;
+    const int n0 = a.ser_nidx[s0];
+    const real base = STAGE0 ? a.xt[co + p] : a.r[co + p];
+    const double invI = 1.0 / (double)I;
+    const real sqc = STAGE0 ? (real)0 : (real)a.sq[c];
     real tem = (real)0;
-    if (stage == 0) {
-        const double invI = 1.0 / (double)I;
-        const real xv = xt[co + p];
-        for (int i = 0; i < I; ++i) {
-            const int s = s0 + i;
-            const int par = mode_parity ? (mode_parity[s] & 1) : fixed_parity;
-            const real hv = (par ? hB : hA)[ser_off[s] + p];
-            const real e = E[ser_eoff[s] + p];
-            const real x = (real)((P)xv + (P)(eps0 * e) * (P)inv[ser_nidx[s]]);
+    auto add = [&](int i, real hv, real ev) {
+        if (STAGE0) {
+            const real x = (real)((P)base + (P)(a.eps0 * ev) * (P)a.inv[n0 + i]);
             tem = acc_stage0<real>(tem, invI, x - hv);
-        }
-        r[co + p] = tem;
-        imf_k[p] = xv - tem;
-    } else {
-        const real rv = r[co + p];
-        const real sqc = (real)sq[c];
-        for (int i = 0; i < I; ++i) {
-            const int s = s0 + i;
-            const int par = mode_parity ? (mode_parity[s] & 1) : fixed_parity;
-            const real hv = (par ? hB : hA)[ser_off[s] + p];
-            const real e = E[ser_eoff[s] + p];
-            const real x = rv + (eps0 * e) * sqc;
+        } else {
+            const real x = base + (a.eps0 * ev) * sqc;
             tem = tem + (x - hv);
         }
-        imf_k[p] = rv - tem / (real)I;
-        r[co + p] = tem / (real)I;
+    };
+    int i = 0;
+    for (; i + kEnsAhead <= I; i += kEnsAhead) {
+        real hv[kEnsAhead], ev[kEnsAhead];
+#pragma unroll
+        for (int q = 0; q < kEnsAhead; ++q) {
+            const int par = a.mode_parity ? (a.mode_parity[s0 + i + q] & 1) : a.fixed_parity;
+            hv[q] = (par ? hs[1] : hs[0])[(int64_t)(i + q) * N];
+            ev[q] = e[(int64_t)(i + q) * N];
+        }
+#pragma unroll
+        for (int q = 0; q < kEnsAhead; ++q) add(i + q, hv[q], ev[q]);
     }
+    for (; i < I; ++i) {
+        const int par = a.mode_parity ? (a.mode_parity[s0 + i] & 1) : a.fixed_parity;
+        add(i, (par ? hs[1] : hs[0])[(int64_t)i * N], e[(int64_t)i * N]);
+    }
+    const real rn = STAGE0 ? tem : tem / (real)I;
+    imf_k[p] = base - rn;
+    a.r[co + p] = rn;
+    if (a.r_next) a.r_next[co + p] = rn;
+    // the last stage's residue is row M - 1 (cudaICEEMDAN.cu:1298)
+    if (a.last) imf_k[N + p] = rn;
 }
 
 // x~ = y * (1 / sqrt(var(y)))  (standardizeRunning, cudaICEEMDAN.cu:57-66)
 template <typename real>
-__global__ void k_standardize(const real* y, const real* var, real* xt, int64_t N)
+__global__ void k_standardize(const real* y, const real* var, real* xt, const int* chan_len,
+                              const int64_t* chan_off)
 {
     using P = typename Promote<real>::type;
-    const int64_t p = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (p >= N) return;
-    const P inv = 1.0 / (P)sqrt(var[0]);
-    xt[p] = (real)((P)y[p] * inv);
+    const int c = blockIdx.y;
+    const int p = blockIdx.x * blockDim.x + threadIdx.x;
+    if (p >= chan_len[c]) return;
+    const P inv = 1.0 / (P)sqrt(var[c]);
+    const int64_t o = chan_off[c] + p;
+    xt[o] = (real)((P)y[o] * inv);
 }
 
-// out = 1/sqrt(var) (take_sqrt = 0) or sqrt(var) (take_sqrt = 1), as double
-template <typename real>
-__global__ void k_inv_sqrt(const real* var, double* out, int n, int take_sqrt)
+// Caller buffers of up to kPtrBatch channels to (IN) or from the plan's:
+// channel c0 + blockIdx.y, rows * chan_len elements
+template <typename real, bool IN>
+__global__ void k_channels(PtrBatch ptr, int c0, int rows, const int* chan_len, const int64_t* off,
+                           real* own)
 {
-    const int i = blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= n) return;
-    const real sd = sqrt(var[i]);
-    out[i] = take_sqrt ? (double)sd : 1.0 / (double)sd;
+    const int c = c0 + blockIdx.y;
+    const int64_t n = (int64_t)rows * chan_len[c];
+    real* q = own + off[c];
+    real* u = (real*)ptr.p[blockIdx.y];
+    for (int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; i < n;
+         i += (int64_t)gridDim.x * blockDim.x) {
+        if (IN) q[i] = u[i];
+        else u[i] = q[i];
+    }
 }
 
 // elementwise kernels: grid-stride with 64-bit indices (capped grids)
-template <typename real>
-__global__ void k_sub(real* w, const real* e, int64_t n)
-{
-    for (int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; i < n;
-         i += (int64_t)gridDim.x * blockDim.x)
-        w[i] = w[i] - e[i];
-}
-
 template <typename real>
 __global__ void k_copy(real* dst, const real* src, int64_t n)
 {
@@ -2530,58 +2588,75 @@ hipError_t launch_rilling_decide(const SeriesDev& sd, const int* nk, const int* 
 
 template <typename real>
 hipError_t launch_series_var(const real* base, const int64_t* off, int64_t stride, const int* len,
-                             int nser, real* var_out, hipStream_t st)
+                             int nser, real* var_out, real* mean_out, double* scale_out, int scale,
+                             hipStream_t st)
 {
     hipLaunchKernelGGL((k_series_var<real>), dim3(nser), dim3(1024), 0, st, base, off, stride, len,
-                       var_out);
+                       var_out, mean_out, scale_out, scale);
     return hipGetLastError();
 }
 
 template <typename real>
-hipError_t launch_noise(uint64_t seed, int I, int64_t N, real* out, int64_t row_stride,
-                        hipStream_t st)
+hipError_t launch_noise(uint64_t seed, int I, int64_t N, real* out, hipStream_t st)
 {
     const int64_t nq = (N + 3) / 4;
-    hipLaunchKernelGGL((k_noise<real>), dim3(blocks_for(nq, 256), I), dim3(256), 0, st, seed, I, N,
-                       out, row_stride);
+    hipLaunchKernelGGL((k_noise<real>), dim3(blocks_for(nq, 256), I), dim3(256), 0, st, seed,
+                       (const int*)nullptr, (const int64_t*)nullptr, N, out);
+    return hipGetLastError();
+}
+
+// `ngroups` lengths of at most max_len samples, as many per launch as keep
+// it below 2^31 work-items
+template <typename real>
+hipError_t launch_noise_groups(uint64_t seed, int I, int ngroups, int64_t max_len, const int* len,
+                               const int64_t* row_off, real* out, hipStream_t st)
+{
+    const unsigned bx = blocks_for((max_len + 3) / 4, 256);
+    const int64_t per = (int64_t)bx * 256 * I;
+    const int most = (int)std::max<int64_t>(1, std::min<int64_t>(65535, ((int64_t)1 << 31) / per));
+    for (int g = 0; g < ngroups; g += most) {
+        hipLaunchKernelGGL((k_noise<real>), dim3(bx, I, std::min(most, ngroups - g)), dim3(256), 0, st,
+                           seed, len + g, row_off + g, (int64_t)0, out);
+        const hipError_t e = hipGetLastError();
+        if (e != hipSuccess) return e;
+    }
+    return hipSuccess;
+}
+
+template <typename real>
+hipError_t launch_ensemble(const EnsembleArgs<real>& a, int nchan, int max_len, hipStream_t st)
+{
+    const dim3 g(blocks_for(max_len, 256), nchan);
+    if (a.stage == 0) hipLaunchKernelGGL((k_ensemble<real, true>), g, dim3(256), 0, st, a);
+    else hipLaunchKernelGGL((k_ensemble<real, false>), g, dim3(256), 0, st, a);
     return hipGetLastError();
 }
 
 template <typename real>
-hipError_t launch_ensemble(int stage, int nchan, int I, int max_len, const int* chan_len,
-                           const int64_t* chan_off, const int64_t* ser_off,
-                           const int64_t* ser_eoff, const int* ser_nidx, const real* hA, const real* hB,
-                           const int* mode_parity, int fixed_parity, const real* E,
-                           const double* inv, const double* sq, real eps0, const real* xt,
-                           real* r, real* imf_base, const int64_t* chan_imf_off, hipStream_t st)
+hipError_t launch_standardize(const real* y, const real* var, real* xt, int nchan, int max_len,
+                              const int* chan_len, const int64_t* chan_off, hipStream_t st)
 {
-    hipLaunchKernelGGL((k_ensemble<real>), dim3(blocks_for(max_len, 256), nchan), dim3(256), 0, st,
-                       stage, I, chan_len, chan_off, ser_off, ser_eoff, ser_nidx, hA, hB, mode_parity,
-                       fixed_parity, E, inv, sq, eps0, xt, r, imf_base, chan_imf_off);
+    hipLaunchKernelGGL((k_standardize<real>), dim3(blocks_for(max_len, 256), nchan), dim3(256), 0, st,
+                       y, var, xt, chan_len, chan_off);
     return hipGetLastError();
 }
 
 template <typename real>
-hipError_t launch_standardize(const real* y, const real* var, real* xt, int64_t N, hipStream_t st)
+hipError_t launch_channels(bool in, void* const* ptr, int nchan, int rows, int64_t max_len,
+                           const int* chan_len, const int64_t* off, real* own, hipStream_t st)
 {
-    hipLaunchKernelGGL((k_standardize<real>), dim3(blocks_for(N, 256)), dim3(256), 0, st, y, var,
-                       xt, N);
-    return hipGetLastError();
-}
-
-template <typename real>
-hipError_t launch_inv_sqrt(const real* var, double* out, int n, int take_sqrt, hipStream_t st)
-{
-    hipLaunchKernelGGL((k_inv_sqrt<real>), dim3(blocks_for(n, 256)), dim3(256), 0, st, var, out, n,
-                       take_sqrt);
-    return hipGetLastError();
-}
-
-template <typename real>
-hipError_t launch_sub(real* w, const real* e, int64_t n, hipStream_t st)
-{
-    hipLaunchKernelGGL((k_sub<real>), dim3(capped_blocks(n, 256)), dim3(256), 0, st, w, e, n);
-    return hipGetLastError();
+    const unsigned bx = std::min(capped_blocks((int64_t)rows * max_len, 256), 4096u);
+    for (int c = 0; c < nchan; c += kPtrBatch) {
+        const int nc = std::min(kPtrBatch, nchan - c);
+        PtrBatch b{};
+        for (int q = 0; q < nc; ++q) b.p[q] = ptr[c + q];
+        const dim3 g(bx, nc);
+        if (in) hipLaunchKernelGGL((k_channels<real, true>), g, dim3(256), 0, st, b, c, rows, chan_len, off, own);
+        else hipLaunchKernelGGL((k_channels<real, false>), g, dim3(256), 0, st, b, c, rows, chan_len, off, own);
+        const hipError_t e = hipGetLastError();
+        if (e != hipSuccess) return e;
+    }
+    return hipSuccess;
 }
 
 template <typename real>
@@ -2636,18 +2711,25 @@ hipError_t launch_adj_seed(const real* gimf, int M, int64_t N, int64_t stride, r
 template <typename real>
 hipError_t launch_adj_stage(int stage, int nchan, int I, int max_len, const int* chan_len,
                             const int64_t* chan_off, const SeriesDev& sd, const real* gr_next,
-                            const real* mu, const real* E, const real* r_k, real eps0, real* gr_k,
-                            real* gacc, real* dots, hipStream_t st)
+                            const real* mu, const real* E, const real* r_k, const real* mean_k,
+                            const double* sq_k, real eps0, real* gr_k, real* gacc, real* dots,
+                            real* coef, hipStream_t st)
 {
-    hipLaunchKernelGGL((k_adj_accum<real>), dim3(blocks_for(max_len, 256), nchan), dim3(256), 0, st,
-                       I, chan_len, chan_off, sd, gr_next, mu, gacc);
+    const dim3 g(blocks_for(max_len, 256), nchan);
+    hipLaunchKernelGGL((k_adj_accum<real>), g, dim3(256), 0, st, I, chan_len, chan_off, sd, gr_next,
+                       mu, gacc);
     hipError_t e = hipGetLastError();
     if (e != hipSuccess) return e;
-    hipLaunchKernelGGL((k_adj_dot<real>), dim3(sd.nseries), dim3(1024), 0, st, I, sd, chan_off,
-                       gr_next, mu, E, dots);
-    if ((e = hipGetLastError()) != hipSuccess) return e;
-    hipLaunchKernelGGL((k_adj_stage<real>), dim3(nchan), dim3(1024), 0, st, stage, I, chan_len,
-                       chan_off, gacc, dots, r_k, eps0, gr_k);
+    if (stage > 0) {
+        hipLaunchKernelGGL((k_adj_dot<real>), dim3(sd.nseries), dim3(1024), 0, st, I, sd, chan_off,
+                           gr_next, mu, E, dots);
+        if ((e = hipGetLastError()) != hipSuccess) return e;
+        hipLaunchKernelGGL((k_adj_coef<real>), dim3(nchan), dim3(kWave), 0, st, I, chan_len, dots,
+                           sq_k, eps0, coef);
+        if ((e = hipGetLastError()) != hipSuccess) return e;
+    }
+    hipLaunchKernelGGL((k_adj_stage<real>), g, dim3(256), 0, st, chan_len, chan_off, gacc,
+                       stage > 0 ? coef : nullptr, mean_k, r_k, gr_k);
     return hipGetLastError();
 }
 
@@ -2704,18 +2786,15 @@ hipError_t launch_check_index(const int* d_x, int64_t N, int* err, hipStream_t s
                                                     const int*, int*, int*, int*, int, int,        \
                                                     const unsigned*, unsigned*, hipStream_t);      \
     template hipError_t launch_series_var<real>(const real*, const int64_t*, int64_t, const int*,  \
-                                                int, real*, hipStream_t);                          \
-    template hipError_t launch_noise<real>(uint64_t, int, int64_t, real*, int64_t, hipStream_t);  \
-    template hipError_t launch_ensemble<real>(int, int, int, int, const int*, const int64_t*,      \
-                                              const int64_t*, const int64_t*, const int*,          \
-                                              const real*,                                         \
-                                              const real*, const int*, int, const real*,           \
-                                              const double*, const double*, real, const real*,     \
-                                              real*, real*, const int64_t*, hipStream_t);          \
-    template hipError_t launch_standardize<real>(const real*, const real*, real*, int64_t,         \
-                                                 hipStream_t);                                     \
-    template hipError_t launch_inv_sqrt<real>(const real*, double*, int, int, hipStream_t);        \
-    template hipError_t launch_sub<real>(real*, const real*, int64_t, hipStream_t);                \
+                                                int, real*, real*, double*, int, hipStream_t);     \
+    template hipError_t launch_noise<real>(uint64_t, int, int64_t, real*, hipStream_t);            \
+    template hipError_t launch_noise_groups<real>(uint64_t, int, int, int64_t, const int*,         \
+                                                  const int64_t*, real*, hipStream_t);             \
+    template hipError_t launch_ensemble<real>(const EnsembleArgs<real>&, int, int, hipStream_t);   \
+    template hipError_t launch_standardize<real>(const real*, const real*, real*, int, int,        \
+                                                 const int*, const int64_t*, hipStream_t);         \
+    template hipError_t launch_channels<real>(bool, void* const*, int, int, int64_t, const int*,   \
+                                              const int64_t*, real*, hipStream_t);                 \
     template hipError_t launch_copy<real>(real*, const real*, int64_t, hipStream_t);               \
     template hipError_t launch_select_copy<real>(const SeriesDev&, int, const real*, const real*,  \
                                                  const int*, real*, hipStream_t);
@@ -2727,8 +2806,9 @@ hipError_t launch_check_index(const int* d_x, int64_t N, int* err, hipStream_t s
                                               hipStream_t);                                        \
     template hipError_t launch_adj_stage<real>(int, int, int, int, const int*, const int64_t*,     \
                                                const SeriesDev&, const real*, const real*,         \
-                                               const real*, const real*, real, real*, real*,       \
-                                               real*, hipStream_t);                                \
+                                               const real*, const real*, const real*,              \
+                                               const double*, real, real*, real*, real*, real*,    \
+                                               hipStream_t);                                       \
     template hipError_t launch_adj_input<real>(int, const int*, const int64_t*, const real*,       \
                                                const real*, real*, hipStream_t);
 

@@ -292,6 +292,8 @@ struct PlanBase {
     int64_t* d_chan_off = nullptr;
     int64_t* d_chan_imf_off = nullptr;
     int* d_chan_len = nullptr;
+    int* d_glen = nullptr;             // noise-group lengths and first samples
+    int64_t* d_group_off = nullptr;
     int max_chan_len = 0;
     bool noise_external = false;
     // per-kernel timing (HIP events around each init / solve / sift launch)
@@ -705,7 +707,7 @@ struct Plan : PlanBase {
     Lane ln[2];                            // [ICM_PHASE_NOISE], [ICM_PHASE_SIGNAL]
     real *modes = nullptr, *wres = nullptr, *wres2 = nullptr;
     real *y = nullptr, *xt = nullptr, *r = nullptr, *imf = nullptr;
-    real *var_chan = nullptr, *var_noise = nullptr;
+    real* var_chan = nullptr;   // per channel: var(x); in the backward, mean(r_k)
     double *inv_noise = nullptr, *sq_chan = nullptr;
     real* r_hist = nullptr;
     int stage_ = -1;            // next CEEMDAN stage of a staged forward (-1: none in progress)     // [M-1][chan_total]: rows 1 .. M-2 = r_1 .. r_{M-2} of the last forward
@@ -726,7 +728,7 @@ struct Plan : PlanBase {
     std::vector<StageRec*> krec_dev;
     std::vector<char> krec_valid;
     real *mu = nullptr, *mom = nullptr, *edge = nullptr, *ga = nullptr, *gr = nullptr,
-         *gacc = nullptr, *dots = nullptr, *gy = nullptr;
+         *gacc = nullptr, *dots = nullptr, *gcoef = nullptr, *gy = nullptr;
 
     int setup()
     {
@@ -757,12 +759,14 @@ struct Plan : PlanBase {
         if ((rc = alloc(&r_hist, chan_total * (M - 1)))) return rc;
         if ((rc = alloc(&var_chan, cfg.num_channels))) return rc;
         if ((rc = alloc(&sq_chan, cfg.num_channels))) return rc;
-        if ((rc = alloc(&var_noise, (int64_t)hn.len.size()))) return rc;
         if ((rc = alloc(&inv_noise, (int64_t)hn.len.size()))) return rc;
         if ((rc = upload(&d_chan_off, chan_off))) return rc;
         if ((rc = upload(&d_chan_imf_off, chan_imf_off))) return rc;
         std::vector<int> cl(lens.begin(), lens.end());
         if ((rc = upload(&d_chan_len, cl))) return rc;
+        std::vector<int> gl(glen.begin(), glen.end());
+        if ((rc = upload(&d_glen, gl))) return rc;
+        if ((rc = upload(&d_group_off, group_off))) return rc;
         if (cfg.stop_mode == ICM_STOP_RILLING) {
             if ((rc = alloc(&active, nser_max))) return rc;
             if ((rc = alloc(&stop_pass, nser_max))) return rc;
@@ -855,10 +859,10 @@ struct Plan : PlanBase {
         L.kstride = h.kcap;
         if ((rc = alloc(&L.kc, 2 * h.kcap))) return rc;
         if ((rc = alloc(&L.winlist, (int64_t)kWinItem * h.maxwin))) return rc;
-        if ((rc = alloc(&L.wincount, kEpochs))) return rc;
-        if ((rc = alloc(&L.ovfcount, kEpochs))) return rc;
-        if ((rc = alloc(&L.densecnt, kEpochs))) return rc;
-        if ((rc = alloc(&L.squeue, kEpochs))) return rc;
+        if ((rc = alloc(&L.wincount, 4 * (int64_t)kEpochs))) return rc;
+        L.ovfcount = L.wincount + kEpochs;
+        L.densecnt = L.ovfcount + kEpochs;
+        L.squeue = L.densecnt + kEpochs;
         if ((rc = alloc(&L.ovfsegs, nt))) return rc;
         return ICM_OK;
     }
@@ -896,20 +900,19 @@ struct Plan : PlanBase {
         if (e_ != hipSuccess) return hip_fail(e_, __LINE__); \
     } while (0)
 
+    // one fill for the lane's four arrays of control words (back to back)
     int reset_control(Lane& L, hipStream_t st)
     {
-        ICM_TRY(launch_fill_u32((uint32_t*)L.wincount, 0u, kEpochs, st));
-        ICM_TRY(launch_fill_u32((uint32_t*)L.ovfcount, 0u, kEpochs, st));
-        ICM_TRY(launch_fill_u32((uint32_t*)L.densecnt, 0u, kEpochs, st));
-        ICM_TRY(launch_fill_u32((uint32_t*)L.squeue, 0u, kEpochs, st));
+        ICM_TRY(launch_fill_u32((uint32_t*)L.wincount, 0u, 4 * (int64_t)kEpochs, st));
         L.epoch = 0;
         return ICM_OK;
     }
     int reset_controls(hipStream_t st)
     {
         int rc;
-        if ((rc = reset_control(ln[0], st))) return rc;
-        return reset_control(ln[1], st);
+        for (int ph = 0; ph < 2; ++ph)   // the stage kernel has no control words
+            if (!whole_stages(ph) && (rc = reset_control(ln[ph], st))) return rc;
+        return ICM_OK;
     }
     static uint32_t next_epoch(Lane& L) { return ++L.epoch; }
 
@@ -1222,12 +1225,11 @@ struct Plan : PlanBase {
     int signal_begin(hipStream_t st)
     {
         const int C = cfg.num_channels;
-        ICM_TRY(launch_series_var<real>(y, d_chan_off, 0, d_chan_len, C, var_chan, st));
-        for (int c = 0; c < C; ++c)
-            ICM_TRY(launch_standardize<real>(y + chan_off[c], var_chan + c, xt + chan_off[c],
-                                             lens[c], st));
-        ICM_TRY(launch_series_var<real>(modes, dn.off, 0, dn.len, dn.nseries, var_noise, st));
-        ICM_TRY(launch_inv_sqrt<real>(var_noise, inv_noise, dn.nseries, 0, st));
+        ICM_TRY(launch_series_var<real>(y, d_chan_off, 0, d_chan_len, C, var_chan, nullptr, nullptr,
+                                        0, st));
+        ICM_TRY(launch_standardize<real>(y, var_chan, xt, C, max_chan_len, d_chan_len, d_chan_off, st));
+        ICM_TRY(launch_series_var<real>(modes, dn.off, 0, dn.len, dn.nseries, nullptr, nullptr,
+                                        inv_noise, SCALE_INV, st));
         return ICM_OK;
     }
 
@@ -1247,8 +1249,8 @@ struct Plan : PlanBase {
             ia.chan_sig = xt;
             ia.scale = inv_noise;
         } else {
-            ICM_TRY(launch_series_var<real>(r, d_chan_off, 0, d_chan_len, C, var_chan, st));
-            ICM_TRY(launch_inv_sqrt<real>(var_chan, sq_chan, C, 1, st));
+            ICM_TRY(launch_series_var<real>(r, d_chan_off, 0, d_chan_len, C, nullptr, nullptr,
+                                            sq_chan, SCALE_STD, st));
             ia.mode = INIT_STAGEK;
             ia.chan_sig = r;
             ia.scale = sq_chan;
@@ -1266,18 +1268,36 @@ struct Plan : PlanBase {
             if ((rc = stage_rilling(ICM_PHASE_SIGNAL, k, dsig, ia, cfg.max_sifts, st))) return rc;
             parity = stop_pass;
         }
-        ICM_TRY(launch_ensemble<real>(k, C, I, max_chan_len, d_chan_len, d_chan_off, dsig.off,
-                                      dsig.eoff, dsig.nidx, ln[1].hA, ln[1].hB, parity,
-                                      fixed_parity, Ek,
-                                      inv_noise, sq_chan, eps0, xt, r, imf, d_chan_imf_off, st));
+        EnsembleArgs<real> ea{};
+        ea.stage = k;
+        ea.I = I;
+        ea.last = k == M - 2;
+        ea.chan_len = d_chan_len;
+        ea.chan_off = d_chan_off;
+        ea.chan_imf_off = d_chan_imf_off;
+        ea.ser_off = dsig.off;
+        ea.ser_eoff = dsig.eoff;
+        ea.ser_nidx = dsig.nidx;
+        ea.hA = ln[1].hA;
+        ea.hB = ln[1].hB;
+        ea.mode_parity = parity;
+        ea.fixed_parity = fixed_parity;
+        ea.E = Ek;
+        ea.inv = inv_noise;
+        ea.sq = sq_chan;
+        ea.eps0 = eps0;
+        ea.xt = xt;
+        ea.r = r;
         // residues kept for the adjoint (r_0 = x~ is xt)
-        if (k + 1 <= M - 2)
-            ICM_TRY(launch_copy<real>(r_hist + (int64_t)(k + 1) * chan_total, r, chan_total, st));
+        ea.r_next = k + 1 <= M - 2 ? r_hist + (int64_t)(k + 1) * chan_total : nullptr;
+        ea.imf = imf;
+        ICM_TRY(launch_ensemble<real>(ea, C, max_chan_len, st));
         return ICM_OK;
     }
 
-    // residue row M-1 (cudaICEEMDAN.cu:1298)
-    int signal_end(hipStream_t st)
+    // residue row M-1 of a staged forward (a state saved after the last stage
+    // may come from a library that wrote it only here)
+    int residue_row(hipStream_t st)
     {
         const int M = cfg.num_imfs, C = cfg.num_channels;
         for (int c = 0; c < C; ++c)
@@ -1297,7 +1317,7 @@ struct Plan : PlanBase {
             if (ready && k > 0) ICM_TRY(hipStreamWaitEvent(st, ready[k], 0));
             if ((rc = signal_stage(k, st))) return rc;
         }
-        return signal_end(st);
+        return ICM_OK;
     }
 
     // Both phases side by side (FIXED mode): the noise-mode phase on the
@@ -1417,8 +1437,7 @@ struct Plan : PlanBase {
             if ((rc = capture_or_run(1, st))) return rc;
         }
         ICM_TRY(hipEventRecord(ev[2], st));
-        for (int c = 0; c < C; ++c)
-            ICM_TRY(launch_copy<real>((real*)out[c], imf + chan_imf_off[c], (int64_t)M * lens[c], st));
+        ICM_TRY(launch_channels<real>(false, out, C, M, max_chan_len, d_chan_len, d_chan_imf_off, imf, st));
         ICM_TRY(hipEventRecord(ev[3], st));
         ICM_TRY(hipMemcpyAsync(h_err, err, sizeof(int), hipMemcpyDeviceToHost, st));
         ICM_TRY(hipStreamSynchronize(st));
@@ -1449,19 +1468,18 @@ struct Plan : PlanBase {
     {
         const int C = cfg.num_channels;
         if (sig) {
-            for (int c = 0; c < C; ++c) {
+            for (int c = 0; c < C; ++c)
                 if (!sig[c]) return ICM_ERR_INVALID_ARG;
-                ICM_TRY(launch_copy<real>(y + chan_off[c], (const real*)sig[c], lens[c], st));
-            }
+            ICM_TRY(launch_channels<real>(true, const_cast<void* const*>(sig), C, 1, max_chan_len,
+                                          d_chan_len, d_chan_off, y, st));
         }
         noise_external = (noise != nullptr);
         if (noise_external) {
             if (glen.size() != 1) return ICM_ERR_INVALID_ARG;
             ICM_TRY(launch_copy<real>(wres, (const real*)noise, hn.samples, st));
         } else {
-            for (size_t g = 0; g < glen.size(); ++g)
-                ICM_TRY(launch_noise<real>(cfg.seed, cfg.num_noise, glen[g], wres + group_off[g],
-                                           glen[g], st));
+            ICM_TRY(launch_noise_groups<real>(cfg.seed, cfg.num_noise, (int)glen.size(),
+                                              max_chan_len, d_glen, d_group_off, wres, st));
         }
         return ICM_OK;
     }
@@ -1512,9 +1530,8 @@ struct Plan : PlanBase {
         for (int c = 0; c < C; ++c)
             if (!out[c]) return ICM_ERR_INVALID_ARG;
         int rc;
-        if ((rc = signal_end(st))) return rc;
-        for (int c = 0; c < C; ++c)
-            ICM_TRY(launch_copy<real>((real*)out[c], imf + chan_imf_off[c], (int64_t)M * lens[c], st));
+        if ((rc = residue_row(st))) return rc;
+        ICM_TRY(launch_channels<real>(false, out, C, M, max_chan_len, d_chan_len, d_chan_imf_off, imf, st));
         if ((rc = sync_err(st))) return rc;
         stage_ = -1;
         have_forward = true;
@@ -1670,6 +1687,7 @@ struct Plan : PlanBase {
         if (!gr && (rc = alloc(&gr, (int64_t)M * chan_total))) return rc;
         if (!gacc && (rc = alloc(&gacc, chan_total))) return rc;
         if (!dots && (rc = alloc(&dots, (int64_t)dsig.nseries))) return rc;
+        if (!gcoef && (rc = alloc(&gcoef, cfg.num_channels))) return rc;
         if (!gy && (rc = alloc(&gy, chan_total))) return rc;
         return ICM_OK;
     }
@@ -1708,8 +1726,8 @@ struct Plan : PlanBase {
                 ia.chan_sig = xt;
                 ia.scale = inv_noise;
             } else {
-                ICM_TRY(launch_series_var<real>(rk, d_chan_off, 0, d_chan_len, C, var_chan, st));
-                ICM_TRY(launch_inv_sqrt<real>(var_chan, sq_chan, C, 1, st));
+                ICM_TRY(launch_series_var<real>(rk, d_chan_off, 0, d_chan_len, C, nullptr, var_chan,
+                                                sq_chan, SCALE_STD, st));
                 ia.mode = INIT_STAGEK;
                 ia.chan_sig = rk;
                 ia.scale = sq_chan;
@@ -1765,12 +1783,11 @@ struct Plan : PlanBase {
                 if (j >= 0) ICM_TRY(launch_adj_span_knot<real>(adj_args(j), solve_grid(), st));
             }
             ICM_TRY(launch_adj_stage<real>(k, C, I, max_chan_len, d_chan_len, d_chan_off, sd, lam,
-                                           mu, Ek, rk, eps0, gr + (int64_t)k * chan_total, gacc,
-                                           dots, st));
+                                           mu, Ek, rk, var_chan, sq_chan, eps0,
+                                           gr + (int64_t)k * chan_total, gacc, dots, gcoef, st));
         }
         ICM_TRY(launch_adj_input<real>(C, d_chan_len, d_chan_off, y, gr, gy, st));
-        for (int c = 0; c < C; ++c)
-            ICM_TRY(launch_copy<real>((real*)gsig[c], gy + chan_off[c], lens[c], st));
+        ICM_TRY(launch_channels<real>(false, gsig, C, 1, max_chan_len, d_chan_len, d_chan_off, gy, st));
         ICM_TRY(hipEventRecord(ev[3], st));
         ICM_TRY(hipMemcpyAsync(h_err, err, sizeof(int), hipMemcpyDeviceToHost, st));
         ICM_TRY(hipStreamSynchronize(st));
@@ -2133,9 +2150,9 @@ int icm_noise(int dtype, uint64_t seed, int64_t I, int64_t N, void* d_out, void*
     if (!d_out || I < 1 || N < 1 || I > 65535 || N > kMaxLen) return ICM_ERR_INVALID_ARG;
     hipError_t e;
     if (dtype == ICM_DTYPE_F64)
-        e = launch_noise<double>(seed, (int)I, N, (double*)d_out, N, (hipStream_t)stream);
+        e = launch_noise<double>(seed, (int)I, N, (double*)d_out, (hipStream_t)stream);
     else if (dtype == ICM_DTYPE_F32)
-        e = launch_noise<float>(seed, (int)I, N, (float*)d_out, N, (hipStream_t)stream);
+        e = launch_noise<float>(seed, (int)I, N, (float*)d_out, (hipStream_t)stream);
     else
         return ICM_ERR_INVALID_ARG;
     if (e != hipSuccess) return ICM_ERR_HIP;
