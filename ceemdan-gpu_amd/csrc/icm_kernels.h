@@ -47,6 +47,9 @@ struct KnotsDev {
     real* fix;   // [nseries][2][2] values of knots 0 and n-1 after the endpoint fix (k_solve)
     int* nbx;    // [ntiles][2][3] positions of the knots pre-1, pre-2 and pre+cnt of the
     real* nby;   //  tile (-1 = none) and their values (k_knot_prefix)
+    // a pass that is recorded for the adjoint (else null): [ntiles][2]
+    // positions of the knots pre-1 and pre+cnt again
+    int *left, *right;
 };
 
 // A run of consecutive tiles of one series, sifted by one workgroup that
@@ -64,7 +67,7 @@ constexpr int kWinItem = 3;
 struct PassCtl {
     uint32_t epoch;        // launch id (unique within one forward)
     int* winlist;          // [kWinItem * maxwin] window items for the next solve
-    unsigned* wincount;    // [epochs] number of window items
+    unsigned* wincount;    // number of window items (of this epoch)
     int K;                 // rows kept per window of the solve
     int H;                 // halo rows on each side of a window
     int* err;              // device error word
@@ -319,7 +322,6 @@ hipError_t launch_copy(real* dst, const real* src, int64_t n, hipStream_t st);
 template <typename real>
 hipError_t launch_select_copy(const SeriesDev& sd, int max_len, const real* hA, const real* hB,
                               const int* parity, real* dst, hipStream_t st);
-hipError_t launch_rec_left(const int* nbx, int* left, int* right, int ntiles, hipStream_t st);
 hipError_t launch_fill_u32(uint32_t* p, uint32_t v, int64_t n, hipStream_t st);
 hipError_t launch_knot_digest(const int* tile_series, const int* tile0, const uint64_t* mask,
                               int ntiles, uint64_t* out, int nseries, hipStream_t st);

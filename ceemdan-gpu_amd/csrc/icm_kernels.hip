@@ -255,6 +255,7 @@ __global__ __launch_bounds__(kPT) void k_knot_prefix_b(SeriesDev sd, KnotsDev<re
                 k.nby[o] = before.l1 >= 0 ? hs[before.l1] : (real)0;
                 k.nbx[o + 1] = before.l2 >= 0 ? (int)before.l2 : -1;
                 k.nby[o + 1] = before.l2 >= 0 ? hs[before.l2] : (real)0;
+                if (k.left) k.left[2 * (tb + t) + ty] = (int)before.l1;
             }
             carry += s_all;
             carry_lt = lt_combine(carry_lt, s_all_lt);
@@ -290,6 +291,7 @@ __global__ __launch_bounds__(kPT) void k_knot_prefix_b(SeriesDev sd, KnotsDev<re
                 }
                 k.nbx[o] = x3;
                 k.nby[o] = x3 >= 0 ? hs[x3] : (real)0;
+                if (k.right) k.right[2 * (tb + t) + ty] = x3;
             }
             carry_min = all;
         }
@@ -299,7 +301,7 @@ __global__ __launch_bounds__(kPT) void k_knot_prefix_b(SeriesDev sd, KnotsDev<re
     if (tid == 0) {
         k.n[2 * s] = ntot[0];
         k.n[2 * s + 1] = ntot[1];
-        s_wbase = atomicAdd(&pc.wincount[pc.epoch], (unsigned)(wmx + wmn));
+        s_wbase = atomicAdd(pc.wincount, (unsigned)(wmx + wmn));
     }
     __syncthreads();
     const unsigned wbase = s_wbase;
@@ -453,7 +455,7 @@ __global__ __launch_bounds__(kPT) void k_knot_prefix_1(SeriesDev sd, KnotsDev<re
             const int n0 = s_all[0], n1 = s_all[1];
             k.n[2 * s] = n0;
             k.n[2 * s + 1] = n1;
-            s_wbase = atomicAdd(&pc.wincount[pc.epoch],
+            s_wbase = atomicAdd(pc.wincount,
                                 (unsigned)((n0 + pc.K - 1) / pc.K + (n1 + pc.K - 1) / pc.K));
         }
 #pragma unroll
@@ -466,6 +468,10 @@ __global__ __launch_bounds__(kPT) void k_knot_prefix_1(SeriesDev sd, KnotsDev<re
                 k.nbx[o + w] = xs[ty][w];
                 k.nby[o + w] = xs[ty][w] >= 0 ? ys[ty][w] : (real)0;
             }
+            if (k.left) {
+                k.left[2 * (tb + t) + ty] = xs[ty][0];
+                k.right[2 * (tb + t) + ty] = xs[ty][2];
+            }
         }
     }
     const int n0 = s_all[0], n1 = s_all[1];
@@ -474,7 +480,7 @@ __global__ __launch_bounds__(kPT) void k_knot_prefix_1(SeriesDev sd, KnotsDev<re
     if (tid == 0 && nt == 0) {
         k.n[2 * s] = n0;
         k.n[2 * s + 1] = n1;
-        s_wbase = atomicAdd(&pc.wincount[pc.epoch], (unsigned)(wmx + wmn));
+        s_wbase = atomicAdd(pc.wincount, (unsigned)(wmx + wmn));
     }
     if (tid == 0) {
         unsigned d = 0;
@@ -646,6 +652,7 @@ __global__ __launch_bounds__(kThreads) void k_knot_prefix_w(SeriesDev sd, KnotsD
                 k.nby[o + 1] = xb[ty][1] >= 0 ? yb[ty][1] : (real)0;
                 // the tile's own first knot, read back by this lane below
                 k.nbx[o + 2] = fp[ty];
+                if (k.left) k.left[2 * gt + ty] = xb[ty][0];
             }
         }
         c[0] = cn[0];
@@ -683,6 +690,7 @@ __global__ __launch_bounds__(kThreads) void k_knot_prefix_w(SeriesDev sd, KnotsD
                 const int64_t o = 6 * gt + 3 * ty + 2;
                 k.nbx[o] = after[ty] == INF ? -1 : after[ty];
                 k.nby[o] = after[ty] == INF ? (real)0 : ya[ty];
+                if (k.right) k.right[2 * gt + ty] = after[ty] == INF ? -1 : after[ty];
             }
         }
     }
@@ -693,7 +701,7 @@ __global__ __launch_bounds__(kThreads) void k_knot_prefix_w(SeriesDev sd, KnotsD
     if (lane == 0) {
         k.n[2 * s] = n0;
         k.n[2 * s + 1] = n1;
-        wbase = atomicAdd(&pc.wincount[pc.epoch], (unsigned)(wmx + wmn));
+        wbase = atomicAdd(pc.wincount, (unsigned)(wmx + wmn));
         if (dense) atomicAdd(&pc.dense[pc.epoch], dense);
     }
     wbase = (unsigned)__builtin_amdgcn_readfirstlane((int)wbase);
@@ -2378,18 +2386,6 @@ __global__ void k_select_copy(SeriesDev sd, const real* hA, const real* hB, cons
     }
 }
 
-// left/right[2 t + ty] = positions of the last knot before tile t and of the
-// first knot after it (from the prefix's neighbour knots), for the
-// adjoint's pass records
-__global__ void k_rec_left(const int* nbx, int* left, int* right, int ntiles)
-{
-    const int i = blockIdx.x * blockDim.x + threadIdx.x;
-    if (i < 2 * ntiles) {
-        left[i] = nbx[6 * (int64_t)(i >> 1) + 3 * (i & 1)];
-        right[i] = nbx[6 * (int64_t)(i >> 1) + 3 * (i & 1) + 2];
-    }
-}
-
 __global__ void k_fill_u32(uint32_t* p, uint32_t v, int64_t n)
 {
     for (int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; i < n;
@@ -2739,13 +2735,6 @@ hipError_t launch_adj_input(int nchan, const int* chan_len, const int64_t* chan_
 {
     hipLaunchKernelGGL((k_adj_input<real>), dim3(nchan), dim3(1024), 0, st, chan_len, chan_off, y,
                        gxt, gy);
-    return hipGetLastError();
-}
-
-hipError_t launch_rec_left(const int* nbx, int* left, int* right, int ntiles, hipStream_t st)
-{
-    hipLaunchKernelGGL(k_rec_left, dim3(blocks_for(2 * (int64_t)ntiles, 256)), dim3(256), 0, st, nbx,
-                       left, right, ntiles);
     return hipGetLastError();
 }
 

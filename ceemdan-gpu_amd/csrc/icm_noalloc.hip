@@ -173,7 +173,7 @@ int sift_static(const real* h, int64_t N64, int64_t I64, real* h_new, int32_t* d
         PassCtl pc{};
         pc.epoch = epoch;
         pc.winlist = winlist;
-        pc.wincount = ctlw;
+        pc.wincount = ctlw + epoch;
         pc.K = solve_k<real>();
         pc.H = solve_h<real>();
         pc.err = err;

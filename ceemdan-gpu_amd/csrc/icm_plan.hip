@@ -867,28 +867,31 @@ struct Plan : PlanBase {
         return ICM_OK;
     }
 
-    PassCtl ctl(const Lane& L, uint32_t e)
+    // R: the record the pass's knot structure goes to instead of the lane
+    PassCtl ctl(const Lane& L, uint32_t e, const Rec* R = nullptr)
     {
         PassCtl pc{};
         pc.epoch = e;
-        pc.winlist = L.winlist;
-        pc.wincount = L.wincount;
+        pc.winlist = R ? R->winlist : L.winlist;
+        pc.wincount = R ? R->wincount : L.wincount + e;
         pc.K = solve_K(cfg.dtype);
         pc.H = solve_H(cfg.dtype);
         pc.err = err;
         pc.dense = L.densecnt;
         return pc;
     }
-    KnotsDev<real> knots(const Lane& L, int b)
+    KnotsDev<real> knots(const Lane& L, int b, const Rec* R = nullptr)
     {
         KnotsDev<real> k{};
-        k.cnt = L.kcnt[b];
-        k.pre = L.kpre[b];
-        k.n = L.nk[b];
+        k.cnt = R ? R->cnt : L.kcnt[b];
+        k.pre = R ? R->pre : L.kpre[b];
+        k.n = R ? R->n : L.nk[b];
         k.fix = L.kfix[b];
         k.nbx = L.knbx[b];
         k.nby = L.knby[b];
-        k.mask = L.kmask[b];
+        k.mask = R ? R->mask : L.kmask[b];
+        k.left = R ? R->left : nullptr;
+        k.right = R ? R->right : nullptr;
         return k;
     }
 
@@ -956,14 +959,15 @@ struct Plan : PlanBase {
         return prof_end(st);
     }
 
-    int trace_copy(int phase, int stage, int pass, const DevSeries& d, int b, hipStream_t st)
+    int trace_copy(int phase, int stage, int pass, const DevSeries& d, const KnotsDev<real>& k,
+                   hipStream_t st)
     {
         if (!trace_passes || pass >= trace_passes || !trace[phase]) return ICM_OK;
         const int64_t n = 2 * (int64_t)d.nseries;
         int32_t* dst = trace[phase] + ((int64_t)stage * trace_passes + pass) * n;
-        ICM_TRY(launch_copy<float>((float*)dst, (const float*)ln[phase].nk[b], n, st));
+        ICM_TRY(launch_copy<float>((float*)dst, (const float*)k.n, n, st));
         uint64_t* dh = trace_hash[phase] + ((int64_t)stage * trace_passes + pass) * d.nseries;
-        ICM_TRY(launch_knot_digest(d.tile_series, d.tile0, ln[phase].kmask[b], d.ntiles, dh,
+        ICM_TRY(launch_knot_digest(d.tile_series, d.tile0, k.mask, d.ntiles, dh,
                                    d.nseries, st));
         return ICM_OK;
     }
@@ -1012,37 +1016,30 @@ struct Plan : PlanBase {
         const int64_t pass_bytes = 2 * (int64_t)sizeof(real) * d.samples;
         real* in0 = h0 ? h0 : L.hA;
         uint32_t e_emit = next_epoch(L);
+        // a recorded pass's knots are written to its record in the first
+        // place (copies of them were 5 % of a forward and adjoint)
+        auto rec_of = [&](int j) { return record && j < S ? record + j : nullptr; };
+        if (record) ICM_TRY(launch_fill_u32((uint32_t*)record[0].wincount, 0u, S, st));
+        KnotsDev<real> kin = knots(L, 0, rec_of(0));
+        PassCtl pin = ctl(L, e_emit, rec_of(0));
         if ((rc = prof_begin(0, pass_bytes, st))) return rc;
-        ICM_TRY(launch_init<real>(sd, ia, h0 ? nullptr : L.hA, knots(L, 0), ctl(L, e_emit), st,
-                                  grid_loop));
+        ICM_TRY(launch_init<real>(sd, ia, h0 ? nullptr : L.hA, kin, pin, st, grid_loop));
         if ((rc = prof_end(st))) return rc;
-        ICM_TRY(launch_knot_prefix<real>(sd, knots(L, 0), in0, ctl(L, e_emit), nullptr, st));
-        if ((rc = trace_copy(phase, stage, 0, d, 0, st))) return rc;
+        ICM_TRY(launch_knot_prefix<real>(sd, kin, in0, pin, nullptr, st));
+        if ((rc = trace_copy(phase, stage, 0, d, kin, st))) return rc;
         for (int j = 0; j < S; ++j) {
             const int b = j & 1;
             SolveArgs<real> sa{};
             sa.sd = sd;
-            sa.k = knots(L, b);
+            sa.k = kin;
             sa.h = j == 0 ? in0 : (b ? L.hB : L.hA);
             sa.c = L.kc;
-            sa.winlist = L.winlist;
-            sa.wincount = L.wincount + e_emit;
+            sa.winlist = pin.winlist;
+            sa.wincount = pin.wincount;
             sa.active = nullptr;
             sa.err = err;
             sa.nak = cfg.boundary == ICM_BOUNDARY_NOT_A_KNOT;
-            if (record) {
-                // structure of pass j's input for the adjoint
-                const Rec& R = record[j];
-                sa.fixf = R.fixf;
-                ICM_TRY(launch_copy<float>((float*)R.mask, (const float*)L.kmask[b], 16 * (int64_t)d.ntiles, st));
-                ICM_TRY(launch_rec_left(L.knbx[b], R.left, R.right, d.ntiles, st));
-                ICM_TRY(launch_copy<float>((float*)R.cnt, (const float*)L.kcnt[b], 2 * (int64_t)d.ntiles, st));
-                ICM_TRY(launch_copy<float>((float*)R.pre, (const float*)L.kpre[b], 2 * (int64_t)d.ntiles, st));
-                ICM_TRY(launch_copy<float>((float*)R.n, (const float*)L.nk[b], 2 * (int64_t)d.nseries, st));
-                ICM_TRY(launch_copy<float>((float*)R.winlist, (const float*)L.winlist,
-                                           (int64_t)kWinItem * d.maxwin, st));
-                ICM_TRY(launch_copy<float>((float*)R.wincount, (const float*)(L.wincount + e_emit), 1, st));
-            }
+            if (record) sa.fixf = record[j].fixf;
             if ((rc = prof_begin(1, 0, st))) return rc;
             ICM_TRY(launch_solve<real>(sa, solve_grid(), st));
             if ((rc = prof_end(st))) return rc;
@@ -1052,21 +1049,23 @@ struct Plan : PlanBase {
             a.sd = sd;
             a.h_in = j == 0 ? in0 : (b ? L.hB : L.hA);
             a.h_out = (j == S - 1 && out) ? out : (b ? L.hA : L.hB);
-            a.kin = knots(L, b);
+            a.kin = kin;
             a.c = L.kc;
-            a.kout = knots(L, b ^ 1);
+            a.kout = knots(L, b ^ 1, rec_of(j + 1));
             a.emit = (j < S - 1) ? 1 : 0;
             const uint32_t e_in = e_emit;
             e_emit = next_epoch(L);
-            a.pc = ctl(L, e_emit);
+            a.pc = ctl(L, e_emit, rec_of(j + 1));
             a.active = nullptr;
             a.sx_cnt = nullptr;
             a.sx_mark = nullptr;
             if ((rc = sift_launch(a, phase, stage, j, d, e_in, e_emit, pass_bytes, st))) return rc;
             if (j < S - 1) {
-                ICM_TRY(launch_knot_prefix<real>(sd, knots(L, b ^ 1), a.h_out, ctl(L, e_emit), nullptr, st));
-                if ((rc = trace_copy(phase, stage, j + 1, d, b ^ 1, st))) return rc;
+                ICM_TRY(launch_knot_prefix<real>(sd, a.kout, a.h_out, a.pc, nullptr, st));
+                if ((rc = trace_copy(phase, stage, j + 1, d, a.kout, st))) return rc;
             }
+            kin = a.kout;
+            pin = a.pc;
         }
         return ICM_OK;
     }
@@ -1113,7 +1112,7 @@ struct Plan : PlanBase {
         ICM_TRY(launch_init<real>(sd, ia, L.hA, knots(L, 0), ctl(L, e_emit), st, grid_loop));
         ICM_TRY(launch_knot_prefix<real>(sd, knots(L, 0), L.hA, ctl(L, e_emit), nullptr, st));
         int rc;
-        if ((rc = trace_copy(phase, stage, 0, d, 0, st))) return rc;
+        if ((rc = trace_copy(phase, stage, 0, d, knots(L, 0), st))) return rc;
         int pending = -1;   // poll slot whose count the host has not read yet
         for (int j = 0; j < max_pass; ++j) {
             const int b = j & 1;
@@ -1155,7 +1154,7 @@ struct Plan : PlanBase {
             PassCtl pn = ctl(L, e_emit);
             pn.run = run_this;
             ICM_TRY(launch_knot_prefix<real>(sd, knots(L, b ^ 1), a.h_out, pn, active, st));
-            if ((rc = trace_copy(phase, stage, j + 1, d, b ^ 1, st))) return rc;
+            if ((rc = trace_copy(phase, stage, j + 1, d, knots(L, b ^ 1), st))) return rc;
             // early exit: results are identical to running every pass to the
             // cap with finished series masked (they never change again).
             // Not while a graph is being captured: it holds every pass.
