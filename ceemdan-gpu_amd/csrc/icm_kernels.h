@@ -250,6 +250,11 @@ StageGeom stage_geometry(int real_size, int64_t max_len, int64_t nseries);
 template <typename real>
 hipError_t launch_stage(const StageArgs<real>& a, const StageGeom& g, hipStream_t st);
 
+// One sift pass over I series of N samples, back to back, with whatever
+// memory it needs taken for the call (icm_noalloc.hip); synchronous.
+int sift_uniform(int dtype, const void* h, int64_t N, int64_t I, void* h_new, int32_t* nk,
+                 hipStream_t st);
+
 // host-side launchers (icm_kernels.hip)
 // loop = true: the grid-stride instance even where one wavefront per run of
 // tiles fits a launch (for testing that instance)

@@ -507,26 +507,75 @@ struct PlanBase {
     virtual int state_save(void* host, int64_t bytes, hipStream_t st) = 0;
     virtual int state_load(const void* host, int64_t bytes, const void* noise, hipStream_t st) = 0;
 
+    // Device memory is taken in batches: alloc and upload between
+    // batch_begin and batch_commit only note what is wanted; the commit makes
+    // one allocation, sets the pointers (which must live until then) and
+    // copies all uploads at once.  One by one, a small plan spent more time
+    // in its ~35 table copies (13 us each) than in a forward.
+    struct Piece {
+        void** where;
+        size_t bytes;
+        std::vector<char> src;
+    };
+    std::vector<Piece> batch;
+    bool batching = false;
+    void batch_begin()
+    {
+        batch.clear();
+        batching = true;
+    }
+    int batch_commit()
+    {
+        batching = false;
+        auto up = [](size_t v) { return (v + 255) & ~(size_t)255; };
+        size_t staged = 0, total = 0;
+        for (const Piece& q : batch) {
+            total += up(q.bytes);
+            if (!q.src.empty()) staged += up(q.bytes);
+        }
+        char* base = nullptr;
+        if (total && hipMalloc((void**)&base, total) != hipSuccess) return ICM_ERR_OUT_OF_MEMORY;
+        if (base) allocs.push_back(base);
+        std::vector<char> host(staged);
+        size_t at[2] = {staged, 0};      // without and with a source: those first
+        for (Piece& q : batch) {
+            size_t& o = at[q.src.empty() ? 0 : 1];
+            *q.where = base + o;
+            if (!q.src.empty()) std::memcpy(host.data() + o, q.src.data(), q.src.size());
+            o += up(q.bytes);
+        }
+        batch.clear();
+        if (staged && hipMemcpy(base, host.data(), staged, hipMemcpyHostToDevice) != hipSuccess)
+            return ICM_ERR_HIP;
+        return ICM_OK;
+    }
     template <typename T>
     int alloc(T** p, int64_t n)
     {
         *p = nullptr;
         if (n <= 0) n = 1;
-        void* q = nullptr;
-        if (hipMalloc(&q, (size_t)n * sizeof(T)) != hipSuccess) return ICM_ERR_OUT_OF_MEMORY;
-        allocs.push_back(q);
         bytes += n * (int64_t)sizeof(T);
+        if (batching) {
+            batch.push_back(Piece{(void**)p, (size_t)n * sizeof(T), {}});
+            return ICM_OK;
+        }
+        void* q = nullptr;
+        if (hipMalloc(&q, (size_t)n * sizeof(T)) != hipSuccess) {
+            bytes -= n * (int64_t)sizeof(T);
+            return ICM_ERR_OUT_OF_MEMORY;
+        }
+        allocs.push_back(q);
         *p = (T*)q;
         return ICM_OK;
     }
+    // (in a batch)
     template <typename T>
     int upload(T** p, const std::vector<T>& v)
     {
-        int rc = alloc(p, (int64_t)v.size());
+        const int rc = alloc(p, (int64_t)v.size());
         if (rc) return rc;
-        if (!v.empty() &&
-            hipMemcpy(*p, v.data(), v.size() * sizeof(T), hipMemcpyHostToDevice) != hipSuccess)
-            return ICM_ERR_HIP;
+        if (!v.empty())
+            batch.back().src.assign((const char*)v.data(), (const char*)(v.data() + v.size()));
         return ICM_OK;
     }
     int upload_series(DevSeries& d, const HostSeries& h)
@@ -573,8 +622,7 @@ struct PlanBase {
         for (auto& e : tev) (void)hipEventDestroy(e);
         for (void* p : allocs) (void)hipFree(p);
         allocs.clear();
-        if (h_n_active) (void)hipHostFree(h_n_active);
-        if (h_err) (void)hipHostFree(h_err);
+        if (h_n_active) (void)hipHostFree(h_n_active);   // and h_err
         if (own) (void)hipStreamDestroy(own);
         drop_stage_scratch();
     }
@@ -734,6 +782,7 @@ struct Plan : PlanBase {
     {
         int rc;
         const int M = cfg.num_imfs;
+        batch_begin();
         if ((rc = upload_series(dn, hn))) return rc;
         if ((rc = upload_series(dsig, hsig))) return rc;
         if ((rc = alloc_lane(ln[ICM_PHASE_NOISE], hn))) return rc;
@@ -778,15 +827,24 @@ struct Plan : PlanBase {
             krec.resize(M - 1);
             krec_dev.assign(M - 1, nullptr);
             for (int k = 0; k < M - 1; ++k)
-                if ((rc = alloc_recs(krec[k], &krec_dev[k]))) return rc;
+                if ((rc = alloc_recs(krec[k]))) return rc;
             krec_valid.assign(M - 1, 0);
         }
-        if (hipHostMalloc((void**)&h_n_active, 2 * sizeof(unsigned), hipHostMallocDefault) !=
+        if ((rc = batch_commit())) return rc;
+        for (Lane& L : ln) {
+            L.ovfcount = L.wincount + kEpochs;
+            L.densecnt = L.ovfcount + kEpochs;
+            L.squeue = L.densecnt + kEpochs;
+        }
+        batch_begin();
+        for (size_t k = 0; k < krec.size(); ++k)
+            if ((rc = upload_recs(krec[k], &krec_dev[k]))) return rc;
+        if ((rc = batch_commit())) return rc;
+        // pinned words read by the host: two counts and the error word
+        if (hipHostMalloc((void**)&h_n_active, 3 * sizeof(unsigned), hipHostMallocDefault) !=
             hipSuccess)
             return ICM_ERR_OUT_OF_MEMORY;
-        if (hipHostMalloc((void**)&h_err, sizeof(int), hipHostMallocDefault) != hipSuccess)
-            return ICM_ERR_OUT_OF_MEMORY;
-        if (hipStreamCreateWithFlags(&own, hipStreamNonBlocking) != hipSuccess) return ICM_ERR_HIP;
+        h_err = (int*)(h_n_active + 2);
         for (auto& e : ev)
             if (hipEventCreate(&e) != hipSuccess) return ICM_ERR_HIP;
         for (auto& e : poll_ev)
@@ -860,9 +918,6 @@ struct Plan : PlanBase {
         if ((rc = alloc(&L.kc, 2 * h.kcap))) return rc;
         if ((rc = alloc(&L.winlist, (int64_t)kWinItem * h.maxwin))) return rc;
         if ((rc = alloc(&L.wincount, 4 * (int64_t)kEpochs))) return rc;
-        L.ovfcount = L.wincount + kEpochs;
-        L.densecnt = L.ovfcount + kEpochs;
-        L.squeue = L.densecnt + kEpochs;
         if ((rc = alloc(&L.ovfsegs, nt))) return rc;
         return ICM_OK;
     }
@@ -994,7 +1049,7 @@ struct Plan : PlanBase {
     // h_out: the first pass reads the noise residual itself); null = L.hA.
     int stage_fixed(int phase, int stage, const DevSeries& d, const InitArgs<real>& ia, int S,
                     real* out, hipStream_t st, Rec* record = nullptr, bool full = false,
-                    real* h0 = nullptr, int* nk_out = nullptr)
+                    real* h0 = nullptr)
     {
         Lane& L = ln[phase];
         const SeriesDev sd = d.view(L.kstride, cap);
@@ -1004,7 +1059,6 @@ struct Plan : PlanBase {
             a.passes = S;
             a.out = out ? out : (S & 1 ? L.hB : L.hA);
             a.need_out = !record || full;
-            a.nk_out = nk_out;
             if (record) {
                 a.rec = record == rec.data() ? rec_dev : krec_dev[stage];
                 ICM_TRY(launch_fill_u32((uint32_t*)record[0].wincount, 0u, S, st));
@@ -1366,7 +1420,9 @@ struct Plan : PlanBase {
             // capture on the plan's own stream (and, for both phases, on
             // the second stream that joins it), replay on the caller's
             const uint32_t e0[2] = {ln[0].epoch, ln[1].epoch};
-            const hipError_t be = hipStreamBeginCapture(own, hipStreamCaptureModeThreadLocal);
+            if (!own && hipStreamCreateWithFlags(&own, hipStreamNonBlocking) != hipSuccess) own = nullptr;
+            const hipError_t be = own ? hipStreamBeginCapture(own, hipStreamCaptureModeThreadLocal)
+                                      : hipErrorOutOfMemory;
             if (be != hipSuccess) {
                 graph_failed = true;
                 (void)hip_fail(be, __LINE__);
@@ -1636,13 +1692,13 @@ struct Plan : PlanBase {
         return ICM_OK;
     }
 
-    int alloc_recs(std::vector<Rec>& out, StageRec** table)
+    // records of the passes of one stage (in a batch)
+    int alloc_recs(std::vector<Rec>& rr)
     {
         const int S = cfg.max_sifts;
         int rc;
-        std::vector<Rec> rr(S);
-        unsigned* wc = nullptr;
-        if ((rc = alloc(&wc, S))) return rc;
+        rr.resize(S);
+        if ((rc = alloc(&rr[0].wincount, S))) return rc;
         for (int j = 0; j < S; ++j) {
             if ((rc = alloc(&rr[j].mask, 8 * (int64_t)dsig.ntiles))) return rc;
             if ((rc = alloc(&rr[j].left, 2 * (int64_t)dsig.ntiles))) return rc;
@@ -1652,15 +1708,19 @@ struct Plan : PlanBase {
             if ((rc = alloc(&rr[j].n, 2 * (int64_t)dsig.nseries))) return rc;
             if ((rc = alloc(&rr[j].fixf, 4 * (int64_t)dsig.nseries))) return rc;
             if ((rc = alloc(&rr[j].winlist, (int64_t)kWinItem * dsig.maxwin))) return rc;
-            rr[j].wincount = wc + j;
         }
-        std::vector<StageRec> dev(S);
-        for (int j = 0; j < S; ++j)
-            dev[j] = StageRec{rr[j].mask, rr[j].left, rr[j].right, rr[j].cnt, rr[j].pre,
-                              rr[j].n, rr[j].fixf, rr[j].winlist, rr[j].wincount};
-        if ((rc = upload(table, dev))) return rc;
-        out.swap(rr);
         return ICM_OK;
+    }
+    // their device table, once they are allocated (in a batch)
+    int upload_recs(std::vector<Rec>& rr, StageRec** table)
+    {
+        std::vector<StageRec> dev;
+        for (size_t j = 0; j < rr.size(); ++j) {
+            rr[j].wincount = rr[0].wincount + j;
+            dev.push_back(StageRec{rr[j].mask, rr[j].left, rr[j].right, rr[j].cnt, rr[j].pre,
+                                   rr[j].n, rr[j].fixf, rr[j].winlist, rr[j].wincount});
+        }
+        return upload(table, dev);
     }
 
     int backward_alloc()
@@ -1675,10 +1735,22 @@ struct Plan : PlanBase {
         }
         return rc;
     }
+    int alloc_rec()
+    {
+        int rc;
+        std::vector<Rec> rr;
+        batch_begin();
+        if ((rc = alloc_recs(rr)) || (rc = batch_commit())) return rc;
+        batch_begin();
+        if ((rc = upload_recs(rr, &rec_dev)) || (rc = batch_commit())) return rc;
+        rec.swap(rr);
+        return ICM_OK;
+    }
     int backward_buffers()
     {
         const int M = cfg.num_imfs;
         int rc;
+        batch_begin();
         if (!mu && (rc = alloc(&mu, dsig.samples))) return rc;
         if (!mom && (rc = alloc(&mom, 8 * ln[ICM_PHASE_SIGNAL].kstride))) return rc;
         if (!edge && (rc = alloc(&edge, 16 * (int64_t)dsig.ntiles))) return rc;
@@ -1688,7 +1760,7 @@ struct Plan : PlanBase {
         if (!dots && (rc = alloc(&dots, (int64_t)dsig.nseries))) return rc;
         if (!gcoef && (rc = alloc(&gcoef, cfg.num_channels))) return rc;
         if (!gy && (rc = alloc(&gy, chan_total))) return rc;
-        return ICM_OK;
+        return batch_commit();
     }
 
     // Reverse mode over the signal phase of the last forward.
@@ -1735,7 +1807,7 @@ struct Plan : PlanBase {
             if (!krec.empty() && krec_valid[k]) {
                 R = krec[k].data();   // kept by the forward
             } else {
-                if (rec.empty() && (rc = alloc_recs(rec, &rec_dev))) return rc;
+                if (rec.empty() && (rc = alloc_rec())) return rc;
                 R = rec.data();
                 if ((rc = stage_fixed(ICM_PHASE_SIGNAL, k, dsig, ia, S, nullptr, st, R))) return rc;
             }
@@ -1795,27 +1867,6 @@ struct Plan : PlanBase {
         timing.backward_ms = t03;
         if (*h_err) return ICM_ERR_DEVICE;
         return ICM_OK;
-    }
-
-    // one pass over the noise-phase series (I series of length N, back to back)
-    int sift_once(const real* h, real* hn, int32_t* nk_out, hipStream_t st)
-    {
-        tuning = false;
-        int rc;
-        ICM_TRY(launch_fill_u32((uint32_t*)err, 0u, 1, st));
-        if ((rc = reset_control(ln[ICM_PHASE_NOISE], st))) return rc;
-        InitArgs<real> ia{};
-        ia.mode = INIT_COPY;
-        ia.src = h;
-        const bool whole = whole_stages(ICM_PHASE_NOISE);
-        if ((rc = stage_fixed(ICM_PHASE_NOISE, 0, dn, ia, 1, hn, st, nullptr, false, nullptr, nk_out)))
-            return rc;
-        if (nk_out && !whole)
-            ICM_TRY(launch_copy<float>((float*)nk_out, (const float*)ln[ICM_PHASE_NOISE].nk[0],
-                                       2 * dn.nseries, st));
-        ICM_TRY(hipMemcpyAsync(h_err, err, sizeof(int), hipMemcpyDeviceToHost, st));
-        ICM_TRY(hipStreamSynchronize(st));
-        return *h_err ? ICM_ERR_DEVICE : ICM_OK;
     }
 
     int noise_modes_out(void* d_out, int64_t count, hipStream_t st) override
@@ -2131,17 +2182,13 @@ int icm_sift_pass(int dtype, const void* d_h, int64_t N, int64_t I, void* d_h_ne
     c.noise_max_sifts = 1;
     c.use_graph = 0;
     if (I < 1 || I > (1 << 20)) return ICM_ERR_INVALID_ARG;
-    icm_plan plan = nullptr;
-    int rc = icm_plan_create(&c, &plan);
+    const int rc = validate(&c);
     if (rc) return rc;
-    if (dtype == ICM_DTYPE_F64)
-        rc = static_cast<Plan<double>*>(plan->p)->sift_once((const double*)d_h, (double*)d_h_new,
-                                                            d_nk, (hipStream_t)stream);
-    else
-        rc = static_cast<Plan<float>*>(plan->p)->sift_once((const float*)d_h, (float*)d_h_new,
-                                                           d_nk, (hipStream_t)stream);
-    icm_plan_destroy(plan);
-    return rc;
+    // a set budget refuses what it refused when the pass ran in a plan
+    if (const char* env = std::getenv("ICM_MEMORY_BUDGET"))
+        if (std::atoll(env) >= 0 && plan_bytes_estimate(&c) > std::atoll(env))
+            return ICM_ERR_OUT_OF_MEMORY;
+    return sift_uniform(dtype, d_h, N, I, d_h_new, d_nk, (hipStream_t)stream);
 }
 
 int icm_noise(int dtype, uint64_t seed, int64_t I, int64_t N, void* d_out, void* stream)

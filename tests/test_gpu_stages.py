@@ -82,3 +82,39 @@ def test_stage_records_equal_steps(icm, dev, lens, dt, keep):
         plan.close()
     for a, b in zip(*got):
         assert torch.equal(a, b)
+
+
+@pytest.mark.parametrize("dt", ["f64", "f32"])
+@pytest.mark.parametrize("rows,n", [(3, 4), (2, 256), (700, 257), (5, 4096), (3, 4600), (3, 4700),
+                                    (2, 8600), (2, 9000), (2, 32768), (1, 70001)])
+def test_sift_pass_routes(icm, orc, dev, dt, rows, n):
+    """One pass, through one workgroup per series where its knots fit LDS and
+    through the launch-per-step kernels where not: knot counts and samples of
+    the oracle (FP64 equal, FP32 within 16 rounding errors of the largest
+    sample, on the same float32 input), the same in place, and the same from
+    the allocation-free entry."""
+    import ctypes as C
+
+    import torch
+    dtype = torch.float64 if dt == "f64" else torch.float32
+    print(f"case: sift pass {dt} {rows} x {n}", flush=True)
+    rng = np.random.default_rng(n)
+    h = torch.tensor(rng.standard_normal((rows, n)), dtype=dtype, device="cuda")
+    hn, nk = icm.sift_pass(h)
+    for i in range(0, rows, max(1, rows // 3)):
+        x = h[i].double().cpu().numpy()
+        ref, nmax, nmin, _, _ = orc.sift_pass(x)
+        assert nk[i].tolist() == [nmax, nmin]
+        got = hn[i].double().cpu().numpy()
+        if dt == "f64":
+            assert np.array_equal(got, ref), i
+        else:
+            assert np.max(np.abs(got - ref)) <= 16 * 2.0 ** -24 * max(np.max(np.abs(x)), np.max(np.abs(ref)))
+    st = C.c_void_p(torch.cuda.current_stream(h.device).cuda_stream)
+    inplace, k2 = h.clone(), torch.zeros_like(nk)
+    assert icm.lib().icm_sift_pass(icm._dtype_code(dtype), C.c_void_p(inplace.data_ptr()), n, rows,
+                                   C.c_void_p(inplace.data_ptr()), C.c_void_p(k2.data_ptr()), st) == 0
+    assert torch.equal(inplace, hn) and torch.equal(k2, nk)
+    if rows * n <= 1 << 21:
+        a, b = icm.sift_pass_static(h)
+        assert torch.equal(a, hn) and torch.equal(b, nk)
