@@ -54,31 +54,33 @@ __device__ __forceinline__ int mask_last(const uint64_t (&m)[kWR])
     return last;
 }
 
-// Bitmasks of the strict maxima and minima among one row of 64 samples
-// (v against its neighbours lft, rgt).  Each comparison is balloted on its
-// own and the masks are combined by scalar instructions: the ballot of one
-// comparison is that comparison's lane mask, while the ballot of a
-// combination of flags costs a v_cndmask and a v_cmp (the compiler turns
-// the flag into a 0/1 vector value and compares it again).  The empty asm
-// statement makes the two row masks scalar registers at this point, so the
-// four comparison masks of every row are not all held until the masks are
-// stored (held together they spilled).  `valid` and `end` are the masks of
-// the lanes inside the series and at its two ends (ends are knots of both
-// types); FULL rows have every lane valid and no end, and ignore both.
-template <bool FULL, typename real>
-__device__ __forceinline__ void row_extrema(real v, real lft, real rgt, uint64_t valid, uint64_t end,
+// Strict maxima and minima among one row of 64 samples from the row's
+// comparisons with the sample after each (gt: v[p] > v[p + 1], lt: <) and
+// the same two of the sample before the row (cg, cl: bit 0).  One comparison
+// of neighbours serves both: v[p] > v[p - 1] is lt of p - 1, a scalar shift,
+// so a row takes two compares and one neighbour row instead of four and two.
+// Each comparison is balloted
+// on its own: the ballot of a combination of flags costs a v_cndmask and a
+// v_cmp.  The empty asm statement makes the two row masks scalar registers at
+// this point (held together, the comparison masks of all rows spilled).
+__device__ __forceinline__ void row_extrema(uint64_t gt, uint64_t lt, uint64_t& cg, uint64_t& cl,
                                             uint64_t& mx, uint64_t& mn)
 {
-    const uint64_t gl = wave_ballot(v > lft), gr = wave_ballot(v > rgt);
-    const uint64_t ll = wave_ballot(v < lft), lr = wave_ballot(v < rgt);
-    if (FULL) {
-        mx = gl & gr;
-        mn = ll & lr;
-    } else {
-        mx = valid & (end | (gl & gr));
-        mn = valid & (end | (ll & lr));
-    }
+    mx = gt & ((lt << 1) | cl);
+    mn = lt & ((gt << 1) | cg);
+    cg = gt >> 63;
+    cl = lt >> 63;
     asm volatile("" : "+s"(mx), "+s"(mn));
+}
+
+// masks of the samples of row p0 .. p0 + 63 inside a series of N samples, and
+// of its two ends (ends are knots of both types)
+__device__ __forceinline__ void row_ends(int p0, int N, uint64_t& valid, uint64_t& end)
+{
+    const int left = N - p0;
+    valid = left >= 64 ? ~0ull : left <= 0 ? 0ull : (1ull << left) - 1;
+    end = p0 == 0 ? 1ull : 0ull;
+    if (left >= 1 && left <= 64) end |= 1ull << (left - 1);
 }
 
 // tile offset of the first set bit, -1 if none
@@ -1153,43 +1155,115 @@ __device__ __forceinline__ void store_masks(uint64_t* dst, const uint64_t (&m)[2
 // full tables keep two arrays (records would cost them waves per SIMD:
 // their LDS would grow from 22 to 35 KB per workgroup in FP32, to 52 KB in
 // FP64).
+// Positions are relative to the tile.  The small FP64 table keeps them as
+// doubles, so that t = p - pos is one subtraction; the full one keeps integers
+// (doubles would cost it a wave per SIMD), and so does FP32, where a float
+// holds no position 2^24 samples away (floats were 1 % faster).
 template <typename real, int KC, bool REC>
 struct KnotTableOf {
-    int pos[2][KC];
+    using pos_t = int;
+    pos_t pos[2][KC];
     Coef<real> q[2][KC];
-    __device__ __forceinline__ int& P(int ty, int j) { return pos[ty][j]; }
+    __device__ __forceinline__ pos_t& P(int ty, int j) { return pos[ty][j]; }
     __device__ __forceinline__ Coef<real>& Q(int ty, int j) { return q[ty][j]; }
 };
 template <typename real, int KC>
 struct KnotTableOf<real, KC, true> {
+    using pos_t = typename std::conditional<std::is_same<real, double>::value, double, int>::type;
     struct alignas(sizeof(real) == 4 ? 32 : 16) Rec {
         Coef<real> q;
-        int pos;
+        pos_t pos;
     };
     Rec r[2][KC];
-    __device__ __forceinline__ int& P(int ty, int j) { return r[ty][j].pos; }
+    __device__ __forceinline__ pos_t& P(int ty, int j) { return r[ty][j].pos; }
     __device__ __forceinline__ Coef<real>& Q(int ty, int j) { return r[ty][j].q; }
 };
 template <typename real, int KC>
 using KnotTable = KnotTableOf<real, KC, KC == kWKS>;
 
+// Which samples of a tile a lane of the sift holds: the four from 4 lane in
+// FP32 (one 16-byte load and store, neighbours mostly in the lane itself,
+// ranks and mask bits shared by its four samples), sample 64 q + lane of each
+// row q in FP64, where quads would be 32 bytes apart in every access.  Sift
+// launches of both dtypes in milliseconds (16 ragged FP32 series of 8192 ..
+// 262144 samples x 100; one FP64 series of 244032 x 200): rows 112.8 and
+// 42.4, quads 107.5 and 47.3 to 52.
+template <typename real>
+struct Lay {
+    static constexpr bool kQuad = sizeof(real) == 4;
+    __device__ __forceinline__ static int at(int q, int lane) { return kQuad ? 4 * lane + q : kWave * q + lane; }
+};
+
+// Samples go past the caches in both directions: a pass reads and writes each
+// once, and what is read again (tables, masks) stays cached (sift launches
+// above with rows: 114.3 -> 112.8 ms FP32, 44.5 -> 42.5 FP64).  A whole tile's
+// samples of the lane, a series may start at any sample.
+typedef float Quad __attribute__((ext_vector_type(4), aligned(4)));
+template <typename real>
+__device__ __forceinline__ void load_quad(const real* p, real (&v)[kWR])
+{
+    const Quad q = __builtin_nontemporal_load((const Quad*)p);
+#pragma unroll
+    for (int i = 0; i < kWR; ++i) v[i] = q[i];
+}
+template <typename real>
+__device__ __forceinline__ void store_tile(real* p, int lane, const real (&v)[kWR])
+{
+    if constexpr (Lay<real>::kQuad) {
+        const Quad q = {v[0], v[1], v[2], v[3]};
+        __builtin_nontemporal_store(q, (Quad*)(p + 4 * lane));
+    } else {
+#pragma unroll
+        for (int r = 0; r < kWR; ++r) __builtin_nontemporal_store(v[r], p + r * kWave + lane);
+    }
+}
+
+// 2 v + bit of the lane in m, v + bit of the lane in m
+__device__ __forceinline__ unsigned shift_in(unsigned v, uint64_t m)
+{
+    return v + v + (__builtin_amdgcn_inverse_ballot_w64(m) ? 1u : 0u);
+}
+__device__ __forceinline__ int add_bit(int v, uint64_t m)
+{
+    return v + (__builtin_amdgcn_inverse_ballot_w64(m) ? 1 : 0);
+}
+
+// lanes whose sample q of a tile with nt samples is inside the series, and
+// those where it is one of the series' two ends (left = samples from the
+// tile's start to the series' end)
+template <typename real>
+__device__ __forceinline__ void lay_ends(int q, int nt, bool first, int left, uint64_t& valid, uint64_t& end)
+{
+    const int in = Lay<real>::kQuad ? (nt - q + kWR - 1) / kWR : min(max(nt - q * kWave, 0), kWave);
+    valid = in >= kWave ? ~0ull : (1ull << in) - 1;
+    end = first && q == 0 ? 1ull : 0ull;
+    const int last = left - 1;
+    const int lq = Lay<real>::kQuad ? last % kWR : last / kWave, ll = Lay<real>::kQuad ? last / kWR : last % kWave;
+    if (left <= kWT && lq == q) end |= 1ull << ll;
+}
+
 template <typename real, int KC>
 struct WTile {
     static constexpr int NC = (KC + kWave - 1) / kWave;
     real h[kWR];
-    real hl, hr;          // h[t0 - 1], h[t0 + kWT] (0 outside the series)
     real c[2][NC];        // c of knots pre-2+j, j = lane + 64 k
-    int nbx;              // lanes 0..5: positions of knots pre-1, pre-2, pre+cnt per type
-    real nby;
-    uint64_t mk;          // lanes 0..7: knot bitmasks [type][row] of h (other lanes: copies)
+    int nbx;
+    real nby;             // lanes 0..5: values of knots pre-1, pre-2, pre+cnt per type
+    // knots of h: of the lane's quad, bits 4 (lane & 1) .. of the type's byte;
+    // else lanes 0..7: row masks [type][row] (other lanes: copies)
+    typename std::conditional<Lay<real>::kQuad, unsigned[2], uint64_t>::type mk;
 };
-
 
 // One segment of tiles, sifted by one wavefront with a knot table of KC
 // entries per type.  A tile whose knots do not fit (cnt + 3 > KC) is an error
 // with the full table (KC = kWKC fits every tile); with the small table it is
 // appended to a.ovf_segs for a second launch with the full table, and the
 // tile after it takes h_new of its left neighbour from its own knots.
+//
+//
+// The pass is bound by the number of instructions of all kinds: VALU, scalar
+// and memory pipes were each about 58 % busy, and more than six waves per SIMD
+// changed nothing.
 template <typename real, bool RILL, int KC>
 __device__ __forceinline__ void sift_segment(const SiftArgs<real>& a, const Segment* segs, int sid,
                                              int lane, KnotTable<real, KC>& T)
@@ -1200,43 +1274,43 @@ __device__ __forceinline__ void sift_segment(const SiftArgs<real>& a, const Segm
     if (a.active && !a.active[s]) return;
     const int N = sd.len[s];
     const int tb = sd.tile0[s];
-    const int64_t kb0 = sd.kbase[s], kb1 = sd.kstride + sd.kbase[s];
     const real* h = a.h_in + sd.off[s];
     real* hout = a.h_out + sd.off[s];
-    // FP32: the two sample pointers in vector registers (the empty asm makes
-    // them non-uniform), which frees four scalar registers through the loop;
-    // the small-table instance then spills 8 instead of 21 (FP64 has no
-    // vector registers to spare)
-    if (std::is_same<real, float>::value) asm volatile("" : "+v"(h), "+v"(hout));
     const int nn[2] = {a.kin.n[2 * s], a.kin.n[2 * s + 1]};
-    const real fx[2][2] = {{a.kin.fix[4 * s], a.kin.fix[4 * s + 1]},
-                           {a.kin.fix[4 * s + 2], a.kin.fix[4 * s + 3]}};
+    const real* cp[2] = {a.c + sd.kbase[s], a.c + sd.kstride + sd.kbase[s]};
+    // end-knot values after the endpoint fix, first and last, of the type of
+    // this lane's neighbour knot (lanes 0..2 maxima, 3..5 minima)
+    const real fx0 = a.kin.fix[4 * s + (lane >= 3 ? 2 : 0)], fx1 = a.kin.fix[4 * s + (lane >= 3 ? 3 : 1)];
     const bool use_mean = (nn[0] > 3) && (nn[1] > 3);
+    using pos_t = typename KnotTable<real, KC>::pos_t;
 
-    auto load = [&](int t, const int* pre, const int* cnt, WTile<real, KC>& w) {
+    int mpre[2], mcnt[2];
+    auto meta_ints = [&](int64_t gt, int (&pre)[2], int (&cnt)[2]) {
+        pre[0] = load_scalar(a.kin.pre + 2 * gt);
+        pre[1] = load_scalar(a.kin.pre + 2 * gt + 1);
+        cnt[0] = load_scalar(a.kin.cnt + 2 * gt);
+        cnt[1] = load_scalar(a.kin.cnt + 2 * gt + 1);
+    };
+
+    auto load = [&](int t, const int (&pre)[2], const int (&cnt)[2], WTile<real, KC>& w) {
         const int t0 = t * kWT;
-        if (std::is_same<real, float>::value && t0 + kWT <= N) {
-            // a whole tile (every one but a series' last): no lane tests
-            // (FP32 only: the FP64 instances came out 0.8 % slower with it)
-#pragma unroll
-            for (int r = 0; r < kWR; ++r) w.h[r] = h[t0 + r * kWave + lane];
+        if (Lay<real>::kQuad && t0 + kWT <= N) {
+            load_quad(h + t0 + 4 * lane, w.h);
         } else {
 #pragma unroll
-            for (int r = 0; r < kWR; ++r) {
-                const int p = t0 + r * kWave + lane;
-                w.h[r] = p < N ? h[p] : (real)0;
+            for (int q = 0; q < kWR; ++q) {
+                const int p = t0 + Lay<real>::at(q, lane);
+                w.h[q] = p < N ? __builtin_nontemporal_load(h + p) : (real)0;
             }
         }
-        w.hl = t0 >= 1 ? h[t0 - 1] : (real)0;
-        w.hr = t0 + kWT < N ? h[t0 + kWT] : (real)0;
 #pragma unroll
         for (int ty = 0; ty < 2; ++ty) {
-            const real* cp = a.c + (ty ? kb1 : kb0);
+            // (entries outside the series are never used)
 #pragma unroll
             for (int k = 0; k < WTile<real, KC>::NC; ++k) {
                 const int j = lane + k * kWave;
-                const int g = pre[ty] - 2 + j;
-                w.c[ty][k] = (j < cnt[ty] + 3 && g >= 0 && g < nn[ty]) ? cp[g] : (real)0;
+                w.c[ty][k] = (real)0;
+                if (j < cnt[ty] + 3) w.c[ty][k] = cp[ty][min(max(pre[ty] - 2 + j, 0), nn[ty] - 1)];
             }
         }
         w.nbx = -1;
@@ -1246,27 +1320,43 @@ __device__ __forceinline__ void sift_segment(const SiftArgs<real>& a, const Segm
             w.nbx = a.kin.nbx[o];
             w.nby = a.kin.nby[o];
         }
-        w.mk = a.kin.mask[8 * (int64_t)(tb + t) + (lane & (2 * kWR - 1))];
+        const uint64_t* mw = a.kin.mask + 8 * (int64_t)(tb + t);
+        if constexpr (Lay<real>::kQuad) {
+            const uint8_t* mb = (const uint8_t*)mw + (lane >> 1);
+            w.mk[0] = mb[0];
+            w.mk[1] = mb[32];
+        } else {
+            w.mk = mw[lane & 7];
+        }
     };
 
-    int mpre[2], mcnt[2], npre[2] = {0, 0}, ncnt[2] = {0, 0};
-    {
-        const int gt = tb + seg.t_first;
-        mpre[0] = load_scalar(a.kin.pre + 2 * gt);
-        mpre[1] = load_scalar(a.kin.pre + 2 * gt + 1);
-        mcnt[0] = load_scalar(a.kin.cnt + 2 * gt);
-        mcnt[1] = load_scalar(a.kin.cnt + 2 * gt + 1);
-    }
+    int npre[2] = {0, 0}, ncnt[2] = {0, 0};
+    meta_ints(tb + seg.t_first, mpre, mcnt);
     WTile<real, KC> cur, nxt;
     load(seg.t_first, mpre, mcnt, cur);
+    // the sample just before the tile: h' of it where `carry` (the previous
+    // tile of the segment computed it: same interval, same coefficients, same
+    // bits), else h
+    real edge = seg.t_first > 0 ? h[seg.t_first * kWT - 1] : (real)0;
+    bool carry = false;
     // the first tile is needed at once; waiting here also tells the compiler
     // that nothing loaded before the loop is outstanding inside it, so the
     // loop body never waits on the prefetch of the next tile
     wait_vmem();
-    // h_new of the sample just before the tile: the previous tile of the
-    // segment computed it (same interval, same coefficients, same bits)
-    real hcarry = (real)0;
-    bool carry = false;   // hcarry is valid (the previous tile was sifted here)
+    // The last sample of a tile has its right neighbour in the next one: it is
+    // stored as no knot and added when that tile's h' is known (by lane 0),
+    // instead of evaluating the neighbour with this tile's table as well.
+    // open: bit 0 = such a sample waits, bit 1 (2) = the sample before it is
+    // greater (less).
+    unsigned open = 0;
+    auto close = [&](int gt, unsigned o, unsigned g, unsigned l) {
+        const unsigned bx = (o >> 2) & g, bn = (o >> 1) & l;
+        if (((bx | bn) & 1u) && lane == 0) {
+            const int64_t w = 2 * (int64_t)gt + (bn & 1u);
+            atomicOr((unsigned*)(a.kout.mask + kWR * w + kWR - 1) + 1, 0x80000000u);
+            atomicAdd(a.kout.cnt + w, 1);
+        }
+    };
 
     for (int i = 0; i < seg.count; ++i) {
         const int t = seg.t_first + i;
@@ -1274,33 +1364,36 @@ __device__ __forceinline__ void sift_segment(const SiftArgs<real>& a, const Segm
         const int t0 = t * kWT;
         const int nt = min(kWT, N - t0);
         const int pre[2] = {mpre[0], mpre[1]}, cnt[2] = {mcnt[0], mcnt[1]};
+        // the next tile does not follow here: this one closes its own end
+        bool tail = true;
         if (i + 1 < seg.count) {
-            // the next tile's prefixes and counts, then its prefetch (which
-            // needs them for its coefficient loads); loading them a tile
-            // earlier hid the scalar loads' latency but held four more scalar
-            // registers through the loop, which spilled (through vector
-            // lanes) at 5 % of the pass's time
-            const int g1 = gt + 1;
-            npre[0] = load_scalar(a.kin.pre + 2 * g1);
-            npre[1] = load_scalar(a.kin.pre + 2 * g1 + 1);
-            ncnt[0] = load_scalar(a.kin.cnt + 2 * g1);
-            ncnt[1] = load_scalar(a.kin.cnt + 2 * g1 + 1);
+            meta_ints(gt + 1, npre, ncnt);
+            tail = ncnt[0] + 3 > KC || ncnt[1] + 3 > KC;
             load(t + 1, npre, ncnt, nxt);
         }
 
         // ---- knot flags of h (find_extrema_shfl_*, cudaICEEMDAN.cu:92-148):
         // the previous pass (or the stage start) found them when it wrote h,
-        // from the same neighbour values, and stored them as bitmasks
+        // from the same neighbour values, and stored them as bitmasks; bm[ty][q]
+        // has bit l for sample q of lane l
         uint64_t bm[2][kWR];
-        int tot[2] = {0, 0};
+#pragma unroll
+        for (int ty = 0; ty < 2; ++ty) {
+            if constexpr (Lay<real>::kQuad) {
+                // the lane's bits to the top, then out one by one (bit 3 first)
+                const unsigned n = cur.mk[ty] >> ((lane & 1) * 4);
+#pragma unroll
+                for (int q = 0; q < kWR; ++q) bm[ty][q] = wave_ballot((n & (1u << q)) != 0u);
+            } else {
+#pragma unroll
+                for (int q = 0; q < kWR; ++q) bm[ty][q] = lane_value(cur.mk, ty * kWR + q);
+            }
+        }
+        const bool over = cnt[0] + 3 > KC || cnt[1] + 3 > KC;
+        int tot[2];
 #pragma unroll
         for (int ty = 0; ty < 2; ++ty)
-#pragma unroll
-            for (int r = 0; r < kWR; ++r) {
-                bm[ty][r] = lane_value(cur.mk, ty * kWR + r);
-                tot[ty] += __popcll(bm[ty][r]);
-            }
-        const bool over = cnt[0] + 3 > KC || cnt[1] + 3 > KC;
+            tot[ty] = __popcll(bm[ty][0]) + __popcll(bm[ty][1]) + __popcll(bm[ty][2]) + __popcll(bm[ty][3]);
         if (tot[0] != cnt[0] || tot[1] != cnt[1] || (over && !a.ovf_segs)) {
             if (lane == 0) atomicOr(a.pc.err, ICM_DEVERR_KNOTCAP);
             return;
@@ -1310,25 +1403,58 @@ __device__ __forceinline__ void sift_segment(const SiftArgs<real>& a, const Segm
         // take a copy of the body without the per-lane end tests
         auto tile = [&](auto full_c) {
             constexpr bool FULL = decltype(full_c)::value;
-            // ---- knot table: index j <-> knot pre - 2 + j
-            int rb[2] = {2, 2};   // table index of the row's first knot
+            // interval (table index) of every sample of the lane: knots
+            // strictly before it, less one; a knot's own entry is the next
+            int iv[2][4];
 #pragma unroll
-            for (int r = 0; r < kWR; ++r) {
-                const int p = t0 + r * kWave + lane;
+            for (int ty = 0; ty < 2; ++ty) {
+                int v = 1;
+                if constexpr (Lay<real>::kQuad) {
 #pragma unroll
-                for (int ty = 0; ty < 2; ++ty) {
-                    if (__builtin_amdgcn_inverse_ballot_w64(bm[ty][r])) {
-                        const int j = rank_below(bm[ty][r], rb[ty]);
-                        const int g = pre[ty] - 2 + j;
-                        real y = cur.h[r];
-                        if (!FULL) {   // knots 0 and n-1 lie in the series' end tiles
-                            if (g == 0) y = fx[ty][0];
-                            if (g == nn[ty] - 1) y = fx[ty][1];
-                        }
-                        T.P(ty, j) = p;
-                        T.Q(ty, j).a = y;
+                    for (int q = 0; q < kWR; ++q) v = rank_below(bm[ty][q], v);
+                    iv[ty][0] = v;
+#pragma unroll
+                    for (int q = 0; q < kWR - 1; ++q) iv[ty][q + 1] = add_bit(iv[ty][q], bm[ty][q]);
+                } else {
+#pragma unroll
+                    for (int q = 0; q < kWR; ++q) {
+                        iv[ty][q] = rank_below(bm[ty][q], v);
+                        v += __popcll(bm[ty][q]);
                     }
-                    rb[ty] += __popcll(bm[ty][r]);
+                }
+            }
+            // ---- knot table: index j <-> knot pre - 2 + j
+            if (FULL && Lay<real>::kQuad) {
+                // of two neighbouring samples at most one is a maximum (minimum)
+#pragma unroll
+                for (int q = 0; q < 4; q += 2) {
+#pragma unroll
+                    for (int ty = 0; ty < 2; ++ty) {
+                        if (__builtin_amdgcn_inverse_ballot_w64(bm[ty][q] | bm[ty][q + 1])) {
+                            const bool second = __builtin_amdgcn_inverse_ballot_w64(bm[ty][q + 1]);
+                            const int j = iv[ty][q] + 1;
+                            T.P(ty, j) = (pos_t)(4 * lane + q + (second ? 1 : 0));
+                            T.Q(ty, j).a = second ? cur.h[q + 1] : cur.h[q];
+                        }
+                    }
+                }
+            } else {
+#pragma unroll
+                for (int q = 0; q < 4; ++q) {
+#pragma unroll
+                    for (int ty = 0; ty < 2; ++ty) {
+                        if (__builtin_amdgcn_inverse_ballot_w64(bm[ty][q])) {
+                            const int j = iv[ty][q] + 1;
+                            const int g = pre[ty] - 2 + j;
+                            real y = cur.h[q];
+                            if (!FULL) {   // knots 0 and n-1 lie in the series' end tiles
+                                if (g == 0) y = lane_value(fx0, 3 * ty);
+                                if (g == nn[ty] - 1) y = lane_value(fx1, 3 * ty);
+                            }
+                            T.P(ty, j) = (pos_t)Lay<real>::at(q, lane);
+                            T.Q(ty, j).a = y;
+                        }
+                    }
                 }
             }
             if (lane < 6) {
@@ -1337,9 +1463,9 @@ __device__ __forceinline__ void sift_segment(const SiftArgs<real>& a, const Segm
                 const int g = pre[ty] - 2 + j;
                 if (cur.nbx >= 0 && g >= 0 && g < nn[ty]) {
                     real y = cur.nby;
-                    if (g == 0) y = fx[ty][0];
-                    if (g == nn[ty] - 1) y = fx[ty][1];
-                    T.P(ty, j) = cur.nbx;
+                    if (g == 0) y = fx0;
+                    if (g == nn[ty] - 1) y = fx1;
+                    T.P(ty, j) = (pos_t)(cur.nbx - t0);
                     T.Q(ty, j).a = y;
                 }
             }
@@ -1367,49 +1493,28 @@ __device__ __forceinline__ void sift_segment(const SiftArgs<real>& a, const Segm
 
             // ---- envelopes, mean, h_new = h - m (interpolate :403-439,
             // averageUppperLower :441-454, updateRealizations :527-544)
-            real hn[kWR];
+            // envelope of type ty at tile offset u, interval j of the table
+            auto env = [&](int ty, int j, int u) {
+                return horner(T.Q(ty, j), (real)((pos_t)u - T.P(ty, j)));
+            };
+            real hn[kWR] = {cur.h[0], cur.h[1], cur.h[2], cur.h[3]};
             int sxc = 0;
             bool sxm = false;
-            // MEAN 1: the envelopes' mean is subtracted (both have > 3
-            // knots); 0: h' = h (only the Rilling statistics need U, L);
-            // 2: chosen per sample by use_mean.  FP32 takes 0 or 1 by a
-            // branch per tile (-1.6 % on the FP32 sift); the FP64 instances
-            // came out slower with the two copies and keep 2.
-            auto rows = [&](auto mean_c) {
-                constexpr int MEAN = decltype(mean_c)::value;
-                int eb[2] = {1, 1};   // interval index of the row's first sample, less its rank
+            if (RILL || use_mean) {
 #pragma unroll
-                for (int r = 0; r < kWR; ++r) {
-                    const int u = r * kWave + lane;
-                    const int p = t0 + u;
-                    hn[r] = cur.h[r];
-                    if (MEAN == 0 && !RILL) {
-                        if (FULL || u < nt) hout[p] = hn[r];
-                        continue;
-                    }
-                    const int ru = rank_below(bm[0][r], eb[0]), rl = rank_below(bm[1][r], eb[1]);
-                    eb[0] += __popcll(bm[0][r]);
-                    eb[1] += __popcll(bm[1][r]);
-                    if (FULL || u < nt) {
-                        const bool p0 = !FULL && p == 0;
-                        const int ju = p0 ? 2 : ru;
-                        const int jl = p0 ? 2 : rl;
-                        const real U = horner(T.Q(0, ju), (real)(p - T.P(0, ju)));
-                        const real L = horner(T.Q(1, jl), (real)(p - T.P(1, jl)));
-                        if (MEAN == 1) hn[r] = cur.h[r] - (U + L) / (real)2;
-                        if (MEAN == 2) hn[r] = cur.h[r] - (use_mean ? (U + L) / (real)2 : (real)0);
-                        hout[p] = hn[r];
-                        if (RILL) {
-                            const real sx = fabs((U + L) / (U - L));
-                            sxc += (sx > (real)0.05) ? 1 : 0;
-                            sxm |= sx > (real)0.5;
-                        }
+                for (int q = 0; q < 4; ++q) {
+                    const int u = Lay<real>::at(q, lane);
+                    // sample 0 of the series lies in interval 0
+                    const bool p0 = !FULL && q == 0 && t0 + u == 0;
+                    const real U = env(0, p0 ? 2 : iv[0][q], u), L = env(1, p0 ? 2 : iv[1][q], u);
+                    if (!RILL || use_mean) hn[q] = cur.h[q] - (U + L) / (real)2;
+                    if (RILL && (FULL || u < nt)) {
+                        const real sx = fabs((U + L) / (U - L));
+                        sxc += (sx > (real)0.05) ? 1 : 0;
+                        sxm |= sx > (real)0.5;
                     }
                 }
-            };
-            if (!std::is_same<real, float>::value) rows(std::integral_constant<int, 2>{});
-            else if (use_mean) rows(std::integral_constant<int, 1>{});
-            else rows(std::integral_constant<int, 0>{});
+            }
             if (RILL) {
                 for (int o = 32; o >= 1; o >>= 1) sxc += __shfl_xor(sxc, o, kWave);
                 const uint64_t mk = wave_ballot(sxm);
@@ -1418,49 +1523,125 @@ __device__ __forceinline__ void sift_segment(const SiftArgs<real>& a, const Segm
                     a.sx_mark[gt] = mk != 0ull ? 1 : 0;
                 }
             }
+            // Every store of the tile comes after this wait, which the next
+            // tile's loads (requested at the start of this one) and the
+            // previous tile's stores have passed by now; without it the loop
+            // waits for its own stores at the latch.
+            auto stores = [&]() {
+                wait_vmem();
+                if (FULL) {
+                    store_tile(hout + t0, lane, hn);
+                } else {
+#pragma unroll
+                    for (int q = 0; q < kWR; ++q) {
+                        const int u = Lay<real>::at(q, lane);
+                        if (u < nt) hout[t0 + u] = hn[q];
+                    }
+                }
+            };
 
             if (a.emit) {
-                // h_new just outside the tile, evaluated by every lane (same LDS words)
-                real hnl = hcarry, hnr = (real)0;
+                // h_new of the samples beside the tile where no tile of this
+                // segment has it, by every lane (same LDS words)
+                real hnl = edge, hnr = (real)0;
                 if (!carry && (FULL || t0 >= 1)) {
-                    const int p = t0 - 1;
-                    const int ju = T.P(0, 1) == p ? 0 : 1;
-                    const int jl = T.P(1, 1) == p ? 0 : 1;
-                    const real U = horner(T.Q(0, ju), (real)(p - T.P(0, ju)));
-                    const real L = horner(T.Q(1, jl), (real)(p - T.P(1, jl)));
-                    hnl = cur.hl - (use_mean ? (U + L) / (real)2 : (real)0);
+                    // a knot lies on the interval to its left
+                    const int ju = T.P(0, 1) == (pos_t)-1 ? 0 : 1;
+                    const int jl = T.P(1, 1) == (pos_t)-1 ? 0 : 1;
+                    const real U = env(0, ju, -1), L = env(1, jl, -1);
+                    hnl = edge - (use_mean ? (U + L) / (real)2 : (real)0);
                 }
-                if (FULL || t0 + kWT < N) {
-                    const int p = t0 + kWT;
-                    const int ju = cnt[0] + 1, jl = cnt[1] + 1;
-                    const real U = horner(T.Q(0, ju), (real)(p - T.P(0, ju)));
-                    const real L = horner(T.Q(1, jl), (real)(p - T.P(1, jl)));
-                    hnr = cur.hr - (use_mean ? (U + L) / (real)2 : (real)0);
+                if (tail && (FULL || t0 + kWT < N)) {
+                    const real hr = h[t0 + kWT];
+                    const real U = env(0, cnt[0] + 1, kWT), L = env(1, cnt[1] + 1, kWT);
+                    hnr = hr - (use_mean ? (U + L) / (real)2 : (real)0);
                 }
                 // ---- knots of h_new (select_extrema_*, :150-207): their row
-                // bitmasks and counts (the next pass's knots)
-                int run[2] = {0, 0};
+                // bitmasks and counts (the next pass's knots).  A comparison
+                // of neighbours serves both samples; that of the tile's last
+                // one is known to its tail only.
+                const uint64_t known = tail ? ~0ull : ~0ull >> 1;
+                uint64_t cg = wave_ballot(hnl > hn[0]) & 1ull, cl = wave_ballot(hnl < hn[0]) & 1ull;
+                const unsigned eg = (unsigned)cg, el = (unsigned)cl;
+                const unsigned was = open;
+                unsigned before;   // the last sample but one against the last
                 uint64_t em[2][kWR];
+                int run[2] = {0, 0};
+                if constexpr (Lay<real>::kQuad) {
+                    uint64_t g[kWR], l[kWR];
+                    const real nx = shift_next(hn[0], hnr);
 #pragma unroll
-                for (int r = 0; r < kWR; ++r) {
-                    const int u = r * kWave + lane;
-                    const int p = t0 + u;
-                    const real lft = r == 0 ? shift_prev(hn[0], hnl) : row_prev(hn[r], hn[r > 0 ? r - 1 : 0]);
-                    const real rgt = r == kWR - 1 ? shift_next(hn[r], hnr)
-                                                  : row_next(hn[r], hn[r < kWR - 1 ? r + 1 : r]);
-                    row_extrema<FULL>(hn[r], lft, rgt, FULL ? 0ull : wave_ballot(u < nt),
-                                      FULL ? 0ull : wave_ballot(p == 0) | wave_ballot(p == N - 1),
-                                      em[0][r], em[1][r]);
+                    for (int q = 0; q < kWR; ++q) {
+                        const real rgt = q < kWR - 1 ? hn[q < kWR - 1 ? q + 1 : q] : nx;
+                        g[q] = wave_ballot(hn[q] > rgt);
+                        l[q] = wave_ballot(hn[q] < rgt);
+                    }
+                    g[kWR - 1] &= known;
+                    l[kWR - 1] &= known;
+                    before = (((unsigned)(g[kWR - 2] >> 63) & 1u) << 1) | (((unsigned)(l[kWR - 2] >> 63) & 1u) << 2);
+                    em[0][0] = g[0] & ((l[kWR - 1] << 1) | cl);
+                    em[1][0] = l[0] & ((g[kWR - 1] << 1) | cg);
 #pragma unroll
-                    for (int ty = 0; ty < 2; ++ty) run[ty] += __popcll(em[ty][r]);
+                    for (int q = 1; q < kWR; ++q) {
+                        em[0][q] = g[q] & l[q - 1];
+                        em[1][q] = l[q] & g[q - 1];
+                    }
+                } else {
+#pragma unroll
+                    for (int q = 0; q < kWR; ++q) {
+                        const real rgt = q == kWR - 1 ? shift_next(hn[q], hnr)
+                                                      : row_next(hn[q], hn[q < kWR - 1 ? q + 1 : q]);
+                        uint64_t g = wave_ballot(hn[q] > rgt), l = wave_ballot(hn[q] < rgt);
+                        if (q == kWR - 1) {
+                            g &= known;
+                            l &= known;
+                            before = (((unsigned)(g >> 62) & 1u) << 1) | (((unsigned)(l >> 62) & 1u) << 2);
+                        }
+                        row_extrema(g, l, cg, cl, em[0][q], em[1][q]);
+                    }
                 }
-                store_masks(a.kout.mask + 8 * (int64_t)gt, em, lane);
+                open = tail ? 0u : 1u | before;
+#pragma unroll
+                for (int q = 0; q < kWR; ++q) {
+                    if (!FULL) {
+                        uint64_t valid, end;
+                        lay_ends<real>(q, nt, t0 == 0, N - t0, valid, end);
+#pragma unroll
+                        for (int ty = 0; ty < 2; ++ty) em[ty][q] = valid & (end | em[ty][q]);
+                    }
+#pragma unroll
+                    for (int ty = 0; ty < 2; ++ty) run[ty] += __popcll(em[ty][q]);
+                }
+                unsigned nb[2] = {0, 0};
+                if constexpr (Lay<real>::kQuad) {
+                    // the lane's four bits per type, two lanes to a byte
+#pragma unroll
+                    for (int ty = 0; ty < 2; ++ty) {
+#pragma unroll
+                        for (int q = kWR - 1; q >= 0; --q) nb[ty] = shift_in(nb[ty], em[ty][q]);
+                        nb[ty] |= (unsigned)dpp_next_i((int)nb[ty], 0) << 4;
+                    }
+                }
+                stores();
+                if (was) close(gt - 1, was, eg, el);
+                uint64_t* mw = a.kout.mask + 8 * (int64_t)gt;
+                if constexpr (Lay<real>::kQuad) {
+                    if (!(lane & 1)) {
+                        uint8_t* mb = (uint8_t*)mw + (lane >> 1);
+                        mb[0] = (uint8_t)nb[0];
+                        mb[32] = (uint8_t)nb[1];
+                    }
+                } else {
+                    store_masks(mw, em, lane);
+                }
                 if (lane == 0) {
                     a.kout.cnt[2 * gt] = run[0];
                     a.kout.cnt[2 * gt + 1] = run[1];
                 }
+            } else {
+                stores();
             }
-            hcarry = lane_value(hn[kWR - 1], kWave - 1);
+            edge = lane_value(hn[kWR - 1], kWave - 1);
             carry = true;
         };
         if (over) {
@@ -1474,6 +1655,7 @@ __device__ __forceinline__ void sift_segment(const SiftArgs<real>& a, const Segm
                 o.pad = 0;
                 a.ovf_segs[q] = o;
             }
+            edge = lane_value(cur.h[kWR - 1], kWave - 1);
             carry = false;
         } else if (t0 > 0 && t0 + kWT < N) {
             tile(std::true_type{});
@@ -1500,10 +1682,14 @@ __device__ __forceinline__ void sift_segment(const SiftArgs<real>& a, const Segm
 // used only where the one-wave-per-segment grid would exceed a launch's
 // 2^32 work-items (or when ICM_SIFT_QUEUE=1).  Workgroups of the
 // one-segment grid are dispatched as slots free up, which balances uneven
-// segments as well.  The small-table instances are held to 96 registers, so
-// that five of their waves fit on a SIMD (their tables allow eight).
+// segments as well.  Registers are held to the waves per SIMD that were
+// fastest, small table and full one (sift launches as above, ms: FP32 with 6
+// and 4 waves 108.4, 6 and 5 106.3, 7 and 6, which spills, 113.6; FP64 with 4
+// and 4 43.9, 5 and 4 42.5).
+template <typename real, int KC>
+constexpr int kSiftWaves = sizeof(real) == 4 ? (KC == kWKS ? 6 : 5) : (KC == kWKS ? 5 : 1);
 template <typename real, bool RILL, int KC, bool QUEUE>
-__global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(KC == kWKS ? 5 : 1)))
+__global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(kSiftWaves<real, KC>)))
 void k_sift_w(SiftArgs<real> a, int nsegs)
 {
     constexpr int NW = kThreads / kWave;
@@ -1515,7 +1701,8 @@ void k_sift_w(SiftArgs<real> a, int nsegs)
     if (KC == kWKS && load_scalar(a.dense) > a.dense_max) return;
     if (!QUEUE) {
         const int sid = blockIdx.x * NW + wv;
-        if (sid < nsegs) sift_segment<real, RILL, KC>(a, a.segs, sid, lane, s_tab[wv]);
+        if (sid < nsegs)
+            sift_segment<real, RILL, KC>(a, a.segs, sid, lane, s_tab[wv]);
         return;
     }
     unsigned got = lane == 0 ? atomicAdd(a.queue, 1u) : 0u;
@@ -1644,14 +1831,18 @@ __device__ __forceinline__ void init_store(const InitSeries<real, MODE>& q, cons
     }
     int run[2] = {0, 0};
     uint64_t em[2][kWR];
+    uint64_t cg = wave_ballot(w.xl > w.x[0]) & 1ull, cl = wave_ballot(w.xl < w.x[0]) & 1ull;
+    const bool ends = t0 == 0 || t0 + kWT >= q.N;
 #pragma unroll
     for (int r = 0; r < kWR; ++r) {
-        const int u = r * kWave + lane;
-        const int p = t0 + u;
-        const real lft = r == 0 ? shift_prev(w.x[0], w.xl) : row_prev(w.x[r], w.x[r > 0 ? r - 1 : 0]);
         const real rgt = r == kWR - 1 ? shift_next(w.x[r], w.xr) : row_next(w.x[r], w.x[r < kWR - 1 ? r + 1 : r]);
-        row_extrema<false>(w.x[r], lft, rgt, wave_ballot(u < nt),
-                           wave_ballot(p == 0) | wave_ballot(p == q.N - 1), em[0][r], em[1][r]);
+        row_extrema(wave_ballot(w.x[r] > rgt), wave_ballot(w.x[r] < rgt), cg, cl, em[0][r], em[1][r]);
+        if (ends) {
+            uint64_t valid, end;
+            row_ends(t0 + r * kWave, q.N, valid, end);
+#pragma unroll
+            for (int ty = 0; ty < 2; ++ty) em[ty][r] = valid & (end | em[ty][r]);
+        }
 #pragma unroll
         for (int ty = 0; ty < 2; ++ty) run[ty] += __popcll(em[ty][r]);
     }
