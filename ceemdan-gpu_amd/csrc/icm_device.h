@@ -128,35 +128,6 @@ __device__ __forceinline__ double dpp_row(double v, double fill)
     return __longlong_as_double(((long long)hi << 32) | (unsigned)lo);
 }
 
-template <int CTRL, int ROWS, typename real, int NV>
-__device__ __forceinline__ void seg_scan_step(real (&v)[NV], int key)
-{
-    // a lane that receives nothing sees key + 1, which never matches
-    const bool take = dpp_row_i<CTRL, ROWS>(key, key + 1) == key;
-#pragma unroll
-    for (int z = 0; z < NV; ++z) {
-        const real w = dpp_row<CTRL, ROWS>(v[z], (real)0);
-        v[z] = take ? v[z] + w : v[z];
-    }
-}
-
-// Inclusive scan of NV values per lane over the runs of equal `key`, for
-// keys that do not decrease with the lane number: lane i ends with the sum
-// over the lanes j <= i of its run.  Steps of 1, 2, 4, 8 lanes inside each
-// row, then the last lane of row 0 (2) into row 1 (3), then lane 31 into
-// rows 2 and 3; with non-decreasing keys, "the source lane has my key"
-// means every lane between belongs to my run.  Every lane executes it.
-template <typename real, int NV>
-__device__ __forceinline__ void seg_scan_keys(real (&v)[NV], int key)
-{
-    seg_scan_step<0x111, 0xF>(v, key);
-    seg_scan_step<0x112, 0xF>(v, key);
-    seg_scan_step<0x114, 0xF>(v, key);
-    seg_scan_step<0x118, 0xF>(v, key);
-    seg_scan_step<0x142, 0xA>(v, key);
-    seg_scan_step<0x143, 0xC>(v, key);
-}
-
 // Wave-uniform load through the scalar data cache (constant address space).
 // Only for data that the running kernel does not write.
 template <typename T>

@@ -1218,6 +1218,19 @@ __device__ __forceinline__ void store_tile(real* p, int lane, const real (&v)[kW
     }
 }
 
+// Knots of one type among a lane's four samples of a quad: the mask byte of
+// the lane pair, and from it bit l of bm[q] for sample 4 l + q of the tile.
+__device__ __forceinline__ unsigned quad_byte(const uint64_t* mask, int64_t gt, int ty, int lane)
+{
+    return ((const uint8_t*)(mask + 8 * gt + kWR * ty))[lane >> 1];
+}
+__device__ __forceinline__ void quad_masks(unsigned byte, int lane, uint64_t (&bm)[kWR])
+{
+    const unsigned n = byte >> ((lane & 1) * 4);
+#pragma unroll
+    for (int q = 0; q < kWR; ++q) bm[q] = wave_ballot((n & (1u << q)) != 0u);
+}
+
 // 2 v + bit of the lane in m, v + bit of the lane in m
 __device__ __forceinline__ unsigned shift_in(unsigned v, uint64_t m)
 {
@@ -1320,13 +1333,11 @@ __device__ __forceinline__ void sift_segment(const SiftArgs<real>& a, const Segm
             w.nbx = a.kin.nbx[o];
             w.nby = a.kin.nby[o];
         }
-        const uint64_t* mw = a.kin.mask + 8 * (int64_t)(tb + t);
         if constexpr (Lay<real>::kQuad) {
-            const uint8_t* mb = (const uint8_t*)mw + (lane >> 1);
-            w.mk[0] = mb[0];
-            w.mk[1] = mb[32];
+            w.mk[0] = quad_byte(a.kin.mask, tb + t, 0, lane);
+            w.mk[1] = quad_byte(a.kin.mask, tb + t, 1, lane);
         } else {
-            w.mk = mw[lane & 7];
+            w.mk = a.kin.mask[8 * (int64_t)(tb + t) + (lane & 7)];
         }
     };
 
@@ -1381,9 +1392,7 @@ __device__ __forceinline__ void sift_segment(const SiftArgs<real>& a, const Segm
         for (int ty = 0; ty < 2; ++ty) {
             if constexpr (Lay<real>::kQuad) {
                 // the lane's bits to the top, then out one by one (bit 3 first)
-                const unsigned n = cur.mk[ty] >> ((lane & 1) * 4);
-#pragma unroll
-                for (int q = 0; q < kWR; ++q) bm[ty][q] = wave_ballot((n & (1u << q)) != 0u);
+                quad_masks(cur.mk[ty], lane, bm[ty]);
             } else {
 #pragma unroll
                 for (int q = 0; q < kWR; ++q) bm[ty][q] = lane_value(cur.mk, ty * kWR + q);
@@ -1903,213 +1912,249 @@ __global__ __launch_bounds__(kThreads) void k_init_w(SeriesDev sd, InitArgs<real
 // 1'. Fused per-tile step for 256-sample tiles: one wavefront per tile,
 // lane l owns the four consecutive samples 4l .. 4l+3.  Optionally
 // mu <- broadcast, then mu <- mu - (G_max^T + G_min^T)/2 for the scatter
-// pass, then the moments of mu over the knot intervals of the moment pass:
-// each lane sums its own samples run by run; the run a lane ends with is
-// continued across lanes by a segmented scan keyed by the run number.
-constexpr int kAdjKC = kWT / 2 + 2;
+// pass, then the moments of mu over the knot intervals of the moment pass.
+// Each lane sums its samples run by run, and what follows its last knot is
+// carried to the lane that holds the next one; the runs are put together in
+// LDS and leave as contiguous 16-byte stores (written by the lanes that end
+// them, 32-byte pieces at two to four places, the dense FP64 launch took 703
+// us instead of 404).
+// FP64 is bound by memory (samples in and out, up to 2.7 KB of moments per
+// tile in the first passes: 1.6 GB), FP32 by vector instructions (438 per
+// tile, 135 of the 160 us).  Densest pass of 3200 series of 16384 samples,
+// FP64: 571 us with a scan keyed by run numbers and the knots found through
+// LDS -> 388; 200 of 244032, FP32: 264 -> 160.
+
+// Four consecutive values of a lane, 16 bytes per access; global memory past
+// the caches (mu is read and written once per step).
+template <typename real>
+using Vec16 = real __attribute__((ext_vector_type(16 / sizeof(real)), aligned(sizeof(real))));
+template <bool NT, typename real>
+__device__ __forceinline__ void load_four(const real* p, real (&v)[4])
+{
+    constexpr int E = 16 / sizeof(real);
+#pragma unroll
+    for (int i = 0; i < 4; i += E) {
+        const Vec16<real>* src = (const Vec16<real>*)(p + i);
+        const Vec16<real> q = NT ? __builtin_nontemporal_load(src) : *src;
+#pragma unroll
+        for (int e = 0; e < E; ++e) v[i + e] = q[e];
+    }
+}
+template <bool NT, typename real>
+__device__ __forceinline__ void store_four(real* p, const real (&v)[4])
+{
+    constexpr int E = 16 / sizeof(real);
+#pragma unroll
+    for (int i = 0; i < 4; i += E) {
+        Vec16<real> q;
+#pragma unroll
+        for (int e = 0; e < E; ++e) q[e] = v[i + e];
+        if (NT) __builtin_nontemporal_store(q, (Vec16<real>*)(p + i));
+        else *(Vec16<real>*)(p + i) = q;
+    }
+}
+
+// One step of the segmented scan below: lanes of `take` add the values that
+// the lane move CTRL brings them.
+template <int CTRL, int ROWS, typename real>
+__device__ __forceinline__ void open_scan_step(real (&v)[4], uint64_t take)
+{
+    if (take == 0ull) return;
+    real w[4];
+#pragma unroll
+    for (int z = 0; z < 4; ++z) w[z] = dpp_row<CTRL, ROWS>(v[z], (real)0);
+    if (__builtin_amdgcn_inverse_ballot_w64(take)) {
+#pragma unroll
+        for (int z = 0; z < 4; ++z) v[z] = v[z] + w[z];
+    }
+}
+
+// Inclusive scan of the lanes' open sums: lane l ends with the sum over the
+// lanes from the last one below it with a knot (whose sum is what follows
+// that knot) to itself; `knot` = lanes with a knot.  Which lanes take part in
+// a step is known from the mask by scalar instructions, and a step that no
+// lane takes part in is left out (four lanes without a knot are rare in a
+// dense pass).
+template <typename real>
+__device__ __forceinline__ void open_scan(real (&v)[4], uint64_t knot)
+{
+    // aN: no knot in the N lanes up to this one, or in its row of 16 so far
+    const uint64_t a1 = ~knot;
+    const uint64_t a2 = a1 & ((a1 << 1) | 0x0001000100010001ull);
+    const uint64_t a4 = a2 & ((a2 << 2) | 0x0003000300030003ull);
+    const uint64_t a8 = a4 & ((a4 << 4) | 0x000F000F000F000Full);
+    const uint64_t a16 = a8 & ((a8 << 8) | 0x00FF00FF00FF00FFull);
+    open_scan_step<0x111, 0xF>(v, a1);
+    open_scan_step<0x112, 0xF>(v, a2);
+    open_scan_step<0x114, 0xF>(v, a4);
+    open_scan_step<0x118, 0xF>(v, a8);
+    open_scan_step<0x142, 0xA>(v, a16 & 0xFFFF0000FFFF0000ull);
+    open_scan_step<0x143, 0xC>(v, a16 & (0x0000FFFF00000000ull | ((a16 >> 47) & 1ull ? 0xFFFFull << 48 : 0ull)));
+}
+
+// Inclusive maximum over the lanes.
+__device__ __forceinline__ int max_scan(int v, int least)
+{
+    v = max(v, dpp_row_i<0x111, 0xF>(v, least));
+    v = max(v, dpp_row_i<0x112, 0xF>(v, least));
+    v = max(v, dpp_row_i<0x114, 0xF>(v, least));
+    v = max(v, dpp_row_i<0x118, 0xF>(v, least));
+    v = max(v, dpp_row_i<0x142, 0xA>(v, least));
+    return max(v, dpp_row_i<0x143, 0xC>(v, least));
+}
+
+constexpr int kAdjKC = kWT / 2 + 2;   // knots of one type in a tile, at most
 
 template <typename real>
-__device__ __forceinline__ void adj_tile(const AdjTileArgs<real>& a, int gt, int lane, real* delta,
-                                         int* tp)
+__device__ __forceinline__ void adj_tile(const AdjTileArgs<real>& a, int gt, int lane, real* sm)
 {
-    constexpr int T = kWT;
-    constexpr int NOKEY = 1 << 28;
     const SeriesDev& sd = a.sd;
-    const int s = sd.tile_series[gt];
-    const int t = gt - sd.tile0[s];
-    const int N = sd.len[s];
-    const int t0 = t * T;
-    const int nt = min(T, N - t0);
-    real* mu = a.mu + sd.off[s];
+    const int s = load_scalar(sd.tile_series + gt);
+    const int t0 = (gt - load_scalar(sd.tile0 + s)) * kWT;
+    const int nt = min(kWT, load_scalar(sd.len + s) - t0);
+    const int64_t kb = load_scalar(sd.kbase + s);
+    real* mu = a.mu + load_scalar(sd.off + s) + t0;
     const int ub = 4 * lane;
 
     real v[4];
     bool dirty = false;
-    if (a.bcast) {
-        const real* src = a.bcast + a.chan_off[sd.chan[s]];
+    {
+        const real* src = mu;
+        if (a.bcast) {
+            src = a.bcast + load_scalar(a.chan_off + load_scalar(sd.chan + s)) + t0;
+            dirty = true;
+        }
+        if (nt == kWT) {
+            load_four<true>(src + ub, v);
+        } else {
 #pragma unroll
-        for (int q = 0; q < 4; ++q) v[q] = ub + q < nt ? src[t0 + ub + q] : (real)0;
-        dirty = true;
-    } else {
-#pragma unroll
-        for (int q = 0; q < 4; ++q) v[q] = ub + q < nt ? mu[t0 + ub + q] : (real)0;
+            for (int q = 0; q < 4; ++q) v[q] = ub + q < nt ? src[ub + q] : (real)0;
+        }
     }
-    // ---- scatter of the knot gradients of pass sc: the lane of each knot
-    // bit (sample 64 r + lane of the tile) adds the gradient of its knot
-    if (a.sc.mask && a.sc.n[2 * s] > 3 && a.sc.n[2 * s + 1] > 3) {
+    // ---- scatter of the knot gradients of pass sc: a sample that is a knot
+    // adds the gradient of that knot
+    if (a.sc.mask && load_scalar(a.sc.n + 2 * s) > 3 && load_scalar(a.sc.n + 2 * s + 1) > 3) {
+        real g[2][4];
 #pragma unroll
-        for (int q = 0; q < 4; ++q) delta[ub + q] = (real)0;
-        wave_sync();
         for (int ty = 0; ty < 2; ++ty) {
-            const int64_t kb = sd.kbase[s] + (ty ? sd.kstride : 0);
-            int cb = a.sc.pre[2 * gt + ty];
+            uint64_t bm[4];
+            quad_masks(quad_byte(a.sc.mask, gt, ty, lane), lane, bm);
+            const real* ga = a.ga + kb + (ty ? sd.kstride : 0) + load_scalar(a.sc.pre + 2 * gt + ty);
+            unsigned r = 0;
 #pragma unroll
-            for (int r = 0; r < kWR; ++r) {
-                const uint64_t m = load_scalar(a.sc.mask + 8 * (int64_t)gt + kWR * ty + r);
-                if (__builtin_amdgcn_inverse_ballot_w64(m)) {
-                    const int u = kWave * r + lane;
-                    delta[u] = delta[u] + a.ga[kb + cb + lanes_below(m)];
-                }
-                cb += __popcll(m);
+            for (int q = 0; q < 4; ++q) r = rank_below(bm[q], r);
+#pragma unroll
+            for (int q = 0; q < 4; ++q) {
+                g[ty][q] = (real)0;
+                if (__builtin_amdgcn_inverse_ballot_w64(bm[q])) g[ty][q] = ga[r];
+                r = add_bit(r, bm[q]);
             }
         }
-        wave_sync();
 #pragma unroll
-        for (int q = 0; q < 4; ++q) v[q] = v[q] - delta[ub + q] / (real)2;
+        for (int q = 0; q < 4; ++q) v[q] = v[q] - (g[0][q] + g[1][q]) / (real)2;
         dirty = true;
     }
     if (dirty) {
+        if (nt == kWT) {
+            store_four<true>(mu + ub, v);
+        } else {
 #pragma unroll
-        for (int q = 0; q < 4; ++q)
-            if (ub + q < nt) mu[t0 + ub + q] = v[q];
+            for (int q = 0; q < 4; ++q)
+                if (ub + q < nt) mu[ub + q] = v[q];
+        }
     }
-    // ---- moments of mu over the intervals of pass mo
-    if (!(a.mo.mask && a.mo.n[2 * s] > 3 && a.mo.n[2 * s + 1] > 3)) return;
+    // ---- moments of mu over the intervals of pass mo: run r of the tile are
+    // the samples after its knot r - 1 up to its knot r (sample 0 of the
+    // series joins run 1, the interval (x_0, x_1]), and t is the distance
+    // from the knot before
+    if (!(a.mo.mask && load_scalar(a.mo.n + 2 * s) > 3 && load_scalar(a.mo.n + 2 * s + 1) > 3)) return;
+#pragma unroll
     for (int ty = 0; ty < 2; ++ty) {
-        const int64_t kb = sd.kbase[s] + (ty ? sd.kstride : 0);
-        const int cnt = a.mo.cnt[2 * gt + ty], pre = a.mo.pre[2 * gt + ty];
-        const int left = pre > 0 ? a.mo.left[2 * gt + ty] : 0;
-        // the tile's knot bits (row words) and their positions in rank order
-        uint64_t bits[kWR];
-#pragma unroll
-        for (int r = 0; r < kWR; ++r) bits[r] = load_scalar(a.mo.mask + 8 * (int64_t)gt + kWR * ty + r);
-        wave_sync();
-        {
-            int cb = 0;
-#pragma unroll
-            for (int r = 0; r < kWR; ++r) {
-                if (__builtin_amdgcn_inverse_ballot_w64(bits[r]))
-                    tp[cb + lanes_below(bits[r])] = t0 + kWave * r + lane;
-                cb += __popcll(bits[r]);
-            }
-        }
-        wave_sync();
+        const int cnt = load_scalar(a.mo.cnt + 2 * gt + ty), pre = load_scalar(a.mo.pre + 2 * gt + ty);
+        // the knot before the tile, from its first sample (0 where sample 0
+        // of the series is the first knot)
+        const int left = t0 > 0 ? load_scalar(a.mo.left + 2 * gt + ty) - t0 : 0;
+        uint64_t bm[4];
+        quad_masks(quad_byte(a.mo.mask, gt, ty, lane), lane, bm);
+        if (t0 == 0) bm[0] &= ~1ull;
         real* e = a.edge + 4 * (4 * (int64_t)gt + 2 * ty);
-        if (lane == 0) {
-            // empty edge runs (a knot on the tile's first / last sample)
-            if (cnt > 0 && (t0 == 0 || tp[0] == t0))
-                for (int m = 0; m < 4; ++m) e[m] = (real)0;
-            if (cnt > 0 && tp[cnt - 1] == t0 + nt - 1)
-                for (int m = 0; m < 4; ++m) e[4 + m] = (real)0;
-        }
-        // run number of sample u: knots of the tile strictly before it
-        // (sample 0 of the series joins run 1, the interval (x_0, x_1])
-        // the four samples of a lane lie in knot word ub >> 6: its bits and
-        // the knots of the words before it
-        const int wd = ub >> 6;
-        uint64_t wbits = bits[0];
-        int wbefore = 0;
+        real* mom = a.mom + 4 * (kb + (ty ? sd.kstride : 0) + pre - 1);
+        // distance of the lane's samples from the knot before them
+        int t[4];
+        {
+            int last = left;
 #pragma unroll
-        for (int w = 1; w < kWR; ++w) {
-            wbefore += wd >= w ? __popcll(bits[w - 1]) : 0;
-            wbits = wd == w ? bits[w] : wbits;
+            for (int q = 0; q < 4; ++q) last = __builtin_amdgcn_inverse_ballot_w64(bm[q]) ? ub + q : last;
+            t[0] = ub - dpp_prev_i(max_scan(last, left), left);
+#pragma unroll
+            for (int q = 0; q < 3; ++q) t[q + 1] = __builtin_amdgcn_inverse_ballot_w64(bm[q]) ? 1 : t[q] + 1;
         }
-        auto key_of = [&](int u) -> int {
-            if (u >= nt) return NOKEY;
-            if (t0 == 0 && u == 0) return 1;
-            const int b = u & 63;
-            return wbefore + (b ? __popcll(wbits << (64 - b)) : 0);
-        };
-        auto dst_of = [&](int r) -> real* {
-            if (r >= 1 && r < cnt) return a.mom + 4 * (kb + pre + r - 1);
-            return e + (r == 0 ? 0 : 4);
-        };
-        int key[4];
-        real m[4][4];
+        real p[4][3];
 #pragma unroll
         for (int q = 0; q < 4; ++q) {
-            const int u = ub + q;
-            key[q] = key_of(u);
-            real tt = (real)0;
-            if (key[q] != NOKEY) {
-                const int lp = (t0 == 0 && u == 0) ? 0 : (key[q] >= 1 ? tp[key[q] - 1] : left);
-                tt = (real)(t0 + u - lp);
-            }
-            const real g = key[q] != NOKEY ? v[q] : (real)0;
-            m[q][0] = g;
-            m[q][1] = g * tt;
-            m[q][2] = m[q][1] * tt;
-            m[q][3] = m[q][2] * tt;
+            p[q][0] = (real)t[q];
+            p[q][1] = p[q][0] * p[q][0];
+            p[q][2] = p[q][1] * p[q][0];
         }
-        // runs inside the lane: the first (maybe continued from the left),
-        // complete middle runs, the last (maybe continued to the right)
-        const int kfirst = key[0];
-        real first[4] = {m[0][0], m[0][1], m[0][2], m[0][3]};
-        bool closed = false;
-        int kcur = kfirst;
-        real cur[4] = {m[0][0], m[0][1], m[0][2], m[0][3]};
+        auto add = [&](real (&m)[4], int q, real g) {
+            m[0] = m[0] + g;
 #pragma unroll
-        for (int q = 1; q < 4; ++q) {
-            if (key[q] == kcur) {
+            for (int z = 0; z < 3; ++z) m[z + 1] = fma(g, p[q][z], m[z + 1]);
+        };
+        // runs that end in the lane, their part before it still missing, and
+        // what follows the lane's last knot
+        real run[4] = {(real)0, (real)0, (real)0, (real)0};
+        int r = t0 == 0 ? 1 : 0;
 #pragma unroll
-                for (int z = 0; z < 4; ++z) cur[z] = cur[z] + m[q][z];
-            } else {
-                if (!closed) {
+        for (int q = 0; q < 4; ++q) r = rank_below(bm[q], r);
+        real* mine = &sm[4 * r];
+        real* d = mine;
 #pragma unroll
-                    for (int z = 0; z < 4; ++z) first[z] = cur[z];
-                    closed = true;
-                } else if (kcur != NOKEY) {
-                    real* d = dst_of(kcur);
+        for (int q = 0; q < 4; ++q) {
+            add(run, q, v[q]);
+            if (__builtin_amdgcn_inverse_ballot_w64(bm[q])) {
+                store_four<false>(d, run);
+                d += 4;
 #pragma unroll
-                    for (int z = 0; z < 4; ++z) d[z] = cur[z];
-                }
-                kcur = key[q];
-#pragma unroll
-                for (int z = 0; z < 4; ++z) cur[z] = m[q][z];
+                for (int z = 0; z < 4; ++z) run[z] = (real)0;
             }
         }
-        // segmented inclusive scan of the last runs over the lanes (the
-        // last-run keys do not decrease with the lane)
-        real sc[4] = {cur[0], cur[1], cur[2], cur[3]};
-        seg_scan_keys(sc, kcur);
-        // lane moves run on every lane
-        const int kprev = dpp_prev_i(kcur, NOKEY + 1);
-        real prevs[4];
+        const uint64_t knot = bm[0] | bm[1] | bm[2] | bm[3];
+        open_scan(run, knot);
+        if (lane == kWave - 1) store_four<false>(e + (cnt > 0 ? 4 : 0), run);
 #pragma unroll
-        for (int z = 0; z < 4; ++z) prevs[z] = shift_prev(sc[z], (real)0);
-        const int knext_first = dpp_next_i(kfirst, NOKEY + 1);
-        if (closed && kfirst != NOKEY) {
-            // the first run ends inside this lane
-            real tot[4];
+        for (int z = 0; z < 4; ++z) run[z] = shift_prev(run[z], (real)0);
+        if (__builtin_amdgcn_inverse_ballot_w64(knot)) {
+            real m[4];
+            load_four<false>(mine, m);
 #pragma unroll
-            for (int z = 0; z < 4; ++z)
-                tot[z] = (kprev == kfirst) ? prevs[z] + first[z] : first[z];
-            real* d = dst_of(kfirst);
-#pragma unroll
-            for (int z = 0; z < 4; ++z) d[z] = tot[z];
+            for (int z = 0; z < 4; ++z) m[z] = run[z] + m[z];
+            store_four<false>(mine, m);
         }
-        // the last run ends at this lane's end unless the next lane continues it
-        const bool ends = (lane == kWave - 1) || (knext_first != kcur);
-        if (ends && kcur != NOKEY) {
-            real* d = dst_of(kcur);
-#pragma unroll
-            for (int z = 0; z < 4; ++z) d[z] = sc[z];
-        }
+        wave_sync();
+        // runs 1 .. cnt - 1 lie side by side in mom, run 0 goes to the edge
+        constexpr int E = 16 / sizeof(real);
+        for (int i = E * lane; i < 4 * cnt; i += E * kWave)
+            *(Vec16<real>*)(i < 4 ? e + i : mom + i) = *(const Vec16<real>*)&sm[i];
+        wave_sync();
     }
 }
 
 // One wavefront per tile (LOOP = false), or a grid-stride loop over the
-// tiles where one wave per tile would exceed a launch's 2^32 work-items
-// (the wave's LDS slice is reused by its next tile only after a wave
-// barrier).  The loop keeps the arguments live across its iterations, which
-// spilled scalar registers (20, restored through v_readlane every tile) and
-// made the adjoint tile step 44 % slower, so it is used only where it must.
+// tiles where one wave per tile would exceed a launch's 2^32 work-items.
 template <typename real, bool LOOP>
 __global__ __launch_bounds__(kThreads) void k_adj_tile(AdjTileArgs<real> a)
 {
     constexpr int NW = kThreads / kWave;
-    __shared__ real s_delta[NW][kWT];
-    __shared__ int s_tp[NW][kAdjKC];
+    __shared__ alignas(16) real s_mom[NW][4 * kAdjKC];
     const int lane = threadIdx.x & 63, wv = wave_index();
     if (!LOOP) {
         const int gt = blockIdx.x * NW + wv;
-        if (gt < a.sd.ntiles) adj_tile<real>(a, gt, lane, s_delta[wv], s_tp[wv]);
+        if (gt < a.sd.ntiles) adj_tile<real>(a, gt, lane, s_mom[wv]);
         return;
     }
-    for (int gt = blockIdx.x * NW + wv; gt < a.sd.ntiles; gt += gridDim.x * NW) {
-        adj_tile<real>(a, gt, lane, s_delta[wv], s_tp[wv]);
-        wave_sync();
-    }
+    for (int gt = blockIdx.x * NW + wv; gt < a.sd.ntiles; gt += gridDim.x * NW)
+        adj_tile<real>(a, gt, lane, s_mom[wv]);
 }
 
 // 2. intervals that leave their tile: the last run of the tile holding the
