@@ -160,6 +160,20 @@ __device__ __forceinline__ double lane_value(double v, int l)
     return __longlong_as_double(((long long)hi << 32) | (unsigned)lo);
 }
 
+// v's value in lane `l` becomes x (both wave-uniform).  One instruction per
+// 32 bits; a select on the lane number takes a compare, a move and a select
+// each.  (The lane number goes through m0: an instruction reads one scalar
+// register besides it.)
+__device__ __forceinline__ void set_lane(uint64_t& v, uint64_t x, int l)
+{
+    uint32_t lo = (uint32_t)v, hi = (uint32_t)(v >> 32);
+    asm("s_mov_b32 m0, %4\n\tv_writelane_b32 %0, %2, m0\n\tv_writelane_b32 %1, %3, m0"
+        : "+v"(lo), "+v"(hi)
+        : "s"((uint32_t)x), "s"((uint32_t)(x >> 32)), "s"(l)
+        : "m0");
+    v = ((uint64_t)hi << 32) | lo;
+}
+
 // ------------------------------------------------------------------ Philox
 struct u64x4 {
     uint64_t v[4];

@@ -29,10 +29,12 @@ namespace {
 
 // Entries before knot 0 and after the last knot of a type.  A window's lanes
 // read the B + 2 knots around their rows without a bound test: from H + 1
-// entries before knot 0 (never used by an inner row) to B + 2 after the last.
+// entries before knot 0 (never used by an inner row) to 17 after the last.  A
+// type's entries begin at a multiple of 8 and so do the B + 2 of every lane
+// (one per row and one on each side, B = 8), which are read 16 bytes at a time.
 template <typename real> struct Pad {
     static constexpr int front = Geom<real>::H + 1;
-    static constexpr int total = Geom<real>::H + 1 + 14;
+    static constexpr int total = Geom<real>::H + 1 + 18;
 };
 
 // Knots and intervals of one pass: `e1` entries for the maxima, then the
@@ -48,16 +50,47 @@ struct KnotRows {
 template <typename real>
 __device__ __forceinline__ KnotRows<real> knot_rows(char* base, int entries)
 {
+    // (c one entry short of the others' alignment: a lane stores it from its
+    // first row, one entry after the first that it reads)
     KnotRows<real> k;
     k.bd = (Coef2<real>*)base;
     k.y = (real*)(k.bd + entries);
-    k.c = k.y + entries;
-    k.p = (uint16_t*)(k.c + entries);
+    k.c = k.y + entries + 7;
+    k.p = (uint16_t*)(k.c + entries + 1);
     return k;
 }
 
 template <typename real>
-constexpr int kEntryBytes = 4 * (int)sizeof(real) + 2;
+constexpr int64_t rows_bytes(int64_t entries)
+{
+    return entries * (4 * (int64_t)sizeof(real) + 2) + 8 * (int64_t)sizeof(real);
+}
+
+// entries of the maxima (a multiple of 8) and of both types
+template <typename real>
+__host__ __device__ constexpr int64_t type_entries(int64_t n) { return (n + Pad<real>::total + 7) & ~(int64_t)7; }
+
+// N consecutive values from a 16-byte boundary (bytes a multiple of 16, or
+// the rest after those)
+template <int N, typename T>
+__device__ __forceinline__ void load_wide(const T* p, T (&v)[N])
+{
+    typedef T Vec __attribute__((ext_vector_type(16 / sizeof(T)), aligned(16)));
+    constexpr int E = 16 / sizeof(T);
+#pragma unroll
+    for (int i = 0; i + E <= N; i += E) {
+        const Vec q = *(const Vec*)(p + i);
+#pragma unroll
+        for (int e = 0; e < E; ++e) v[i + e] = q[e];
+    }
+#pragma unroll
+    for (int i = N / E * E; i < N; i += 2) {
+        typedef T Two __attribute__((ext_vector_type(2), aligned(2 * sizeof(T))));
+        const Two q = *(const Two*)(p + i);
+        v[i] = q[0];
+        v[i + 1] = q[1];
+    }
+}
 
 // x[q] of the lane and row that hold window row r (wave-uniform result)
 template <typename real, int B>
@@ -74,94 +107,78 @@ __device__ __forceinline__ real window_row(const real (&x)[B], int r)
     return v;
 }
 
-// Endpoint fix of an end knot (position p0, value y0) from the line through
-// the two knots next to it (setBoundaryMax/Min, cudaICEEMDAN.cu:209-291).
-template <typename real, bool LAST>
-__device__ __forceinline__ real end_value(int ty, int n, int p0, int p1, int p2, real y0, real y1,
-                                          real y2, int& replaced)
-{
-    real t;
-    if (!LAST) {
-        const real slope = (y2 - y1) / (real)(p2 - p1);
-        t = y1 - slope * (real)(p1 - p0);
-    } else {
-        const real slope = (y1 - y2) / (real)(p1 - p2);
-        t = y1 + slope * (real)(p0 - p1);
-    }
-    const bool take = n >= 6 && (ty == 0 ? (t > y0) : (t < y0));
-    replaced = take ? 1 : 0;
-    return take ? t : y0;
-}
-
 // Solves window w of the n knots of type ty (entries from e0 = knot 0) and
 // writes c of the rows it keeps; the window that keeps an end knot stores the
 // end values after the endpoint fix in fix[0..1].  Not-a-knot ends change
 // rows 1 and n - 2 only: their entries are wave-uniform, selected per row.
-template <typename real>
+// A short series has one window per type, so a pass waits for the serial
+// chain and the issue slots of one wave here (half of it): 7.7 -> 5.2 thousand
+// cycles in FP64, 5.3 -> 3.1 in FP32, with the entries in 16-byte reads
+// (eight lanes met in a bank before), both ends at once in even and odd lanes,
+// no branch among the rows, pivots without operand scaling and the levels of
+// partition_pcr that change nothing left out.
+template <typename real, bool NAK>
 __device__ __forceinline__ void solve_window(const KnotRows<real>& k, int e0, int ty, int n, int w,
-                                             int lane, bool nak, real* fix, int* fixf)
+                                             int lane, real* fix, int* fixf)
 {
     constexpr int B = Geom<real>::B, H = Geom<real>::H, W = kWave * B, K = W - 2 * H;
     const int g0 = w * K - H, lo = g0 - 1;
     const int rb = lane * B;
-    // the three knots at each end, and the lane's own (lanes past the last
-    // knot read its tail padding)
-    const int m0 = min(2, n - 1), m1 = max(n - 3, 0);
-    const int pa0 = k.p[e0], pa1 = k.p[e0 + 1], pa2 = k.p[e0 + m0];
-    const int pz0 = k.p[e0 + n - 1], pz1 = k.p[e0 + n - 2], pz2 = k.p[e0 + m1];
-    const real ya0 = k.y[e0], ya1 = k.y[e0 + 1], ya2 = k.y[e0 + m0];
-    const real yz0 = k.y[e0 + n - 1], yz1 = k.y[e0 + n - 2], yz2 = k.y[e0 + m1];
-    int px[B + 2];
+    // knots 0, 1, 2 (even lanes) or n-1, n-2, n-3 (odd lanes): the two ends
+    // are mirror images with the same arithmetic, bit for bit
+    const bool odd = lane & 1;
+    const int i0 = e0 + (odd ? n - 1 : 0), i1 = e0 + (odd ? n - 2 : 1), i2 = e0 + (odd ? max(n - 3, 0) : min(2, n - 1));
+    const int he = (int)k.p[i1] - (int)k.p[i0], hn = (int)k.p[i2] - (int)k.p[i1];
+    const real y0 = k.y[i0], y1 = k.y[i1], y2 = k.y[i2];
+    uint16_t px[B + 2];
     real py[B + 2];
     {
-        const int at = e0 + min(lo + rb, n + 1);
-#pragma unroll
-        for (int j = 0; j < B + 2; ++j) {
-            px[j] = (int)k.p[at + j];
-            py[j] = k.y[at + j];
-        }
-    }
-    // rows of not-a-knot ends: (dl, d, du) of row 1 and of row n - 2
-    int gn1 = -1, gn2 = -1;
-    real d1 = (real)1, u1 = (real)0, l2 = (real)0, d2 = (real)1;
-    if (lo <= 0) {
-        int replaced;
-        const real v = end_value<real, false>(ty, n, pa0, pa1, pa2, ya0, ya1, ya2, replaced);
-#pragma unroll
-        for (int j = 0; j < B + 2; ++j) py[j] = lo + rb + j == 0 ? v : py[j];
-        if (w == 0 && lane == 0) {
-            fix[0] = v;
-            if (fixf) fixf[0] = replaced;
-        }
-        if (nak) {
-            const int hl = pa1 - pa0, hr = pa2 - pa1;
-            gn1 = 1;
-            d1 = (real)(3 * hl + 2 * hr) + (real)hl * (real)hl / (real)hr;
-            u1 = (real)hr - (real)hl * (real)hl / (real)hr;
-        }
-    }
-    if (n - 1 - lo < W + 2) {
-        int replaced;
-        const real v = end_value<real, true>(ty, n, pz0, pz1, pz2, yz0, yz1, yz2, replaced);
-#pragma unroll
-        for (int j = 0; j < B + 2; ++j) py[j] = lo + rb + j == n - 1 ? v : py[j];
-        if (n - 1 >= w * K && n - 1 < w * K + K && lane == 0) {
-            fix[1] = v;
-            if (fixf) fixf[1] = replaced;
-        }
-        if (nak) {
-            const int hl = pz1 - pz2, hr = pz0 - pz1;
-            gn2 = n - 2;
-            l2 = (real)hl - (real)hr * (real)hr / (real)hl;
-            d2 = (real)(2 * hl + 3 * hr) + (real)hr * (real)hr / (real)hl;
-        }
+        const int at = e0 + lo + min(rb, (n - lo + 7) & ~7);
+        load_wide(k.p + at, px);
+        load_wide(k.y + at, py);
     }
     int hx[B + 1];
     real sl[B + 1];
 #pragma unroll
     for (int j = 0; j <= B; ++j) {
-        hx[j] = px[j + 1] - px[j];
+        hx[j] = (int)px[j + 1] - (int)px[j];
         sl[j] = sdiv<real>(py[j + 1] - py[j], (real)hx[j]);
+    }
+    // endpoint fix from the line through the two knots next to the end
+    // (setBoundaryMax/Min, cudaICEEMDAN.cu:209-291), and the slopes of the
+    // first and last interval with it
+    {
+        const real t = y1 - (y2 - y1) / (real)hn * (real)he;
+        const bool above = t > y0, below = t < y0;
+        const bool take = n >= 6 && (ty == 0 ? above : below);
+        const real v = take ? t : y0;
+        const real se = sdiv<real>(y1 - v, (real)he);
+        const real sa = lane_value(se, 0), sz = lane_value(se, 1);
+        constexpr int j0 = (H + 1) % B;
+        sl[j0] = lo + rb + j0 == 0 ? sa : sl[j0];
+        const int jz = n - 2 - lo - rb;
+#pragma unroll
+        for (int j = 0; j <= B; ++j) sl[j] = j == jz ? sz : sl[j];
+        // stored by the window that keeps the end
+        const int ge = odd ? n - 1 : 0;
+        if (lane < 2 && ge >= w * K && ge < w * K + K) {
+            fix[lane] = v;
+            if (fixf) fixf[lane] = take ? 1 : 0;
+        }
+    }
+    // rows of not-a-knot ends: (dl, d, du) of row 1 and of row n - 2
+    int gn1 = -1, gn2 = -1;
+    real d1 = (real)1, u1 = (real)0, l2 = (real)0, d2 = (real)1;
+    if (NAK) {
+        const int ae = abs(he), an = abs(hn);
+        const real dd = (real)(3 * ae + 2 * an) + (real)ae * (real)ae / (real)an;
+        const real oo = (real)an - (real)ae * (real)ae / (real)an;
+        gn1 = 1;
+        gn2 = n - 2;
+        d1 = lane_value(dd, 0);
+        u1 = lane_value(oo, 0);
+        d2 = lane_value(dd, 1);
+        l2 = lane_value(oo, 1);
     }
     real xs[B];
     partition_pcr<real, B>(
@@ -169,7 +186,7 @@ __device__ __forceinline__ void solve_window(const KnotRows<real>& k, int e0, in
         [&](int q, real& dl, real& d, real& du, real& f) {
             const int g = g0 + rb + q;
             spline_row<real, false>(n, g, hx[q], hx[q + 1], sl[q], sl[q + 1], dl, d, du, f);
-            if (nak) {
+            if (NAK) {
                 // n >= 4, so rows 1 and n - 2 are different rows
                 d = g == gn1 ? d1 : g == gn2 ? d2 : d;
                 du = g == gn1 ? u1 : g == gn2 ? (real)0 : du;
@@ -180,19 +197,26 @@ __device__ __forceinline__ void solve_window(const KnotRows<real>& k, int e0, in
     // whole lanes keep their rows; a lane's rows past the last knot land in
     // its tail padding
     if (lane >= H / B && lane < kWave - H / B && g0 + rb < n) {
+        typedef real Vec __attribute__((ext_vector_type(16 / sizeof(real)), aligned(16)));
+        constexpr int E = 16 / sizeof(real);
 #pragma unroll
-        for (int q = 0; q < B; ++q) k.c[e0 + g0 + rb + q] = xs[q];
+        for (int q = 0; q < B; q += E) {
+            Vec v;
+#pragma unroll
+            for (int e = 0; e < E; ++e) v[e] = xs[q + e];
+            *(Vec*)(k.c + e0 + g0 + rb + q) = v;
+        }
     }
-    if (nak) {
+    if (NAK) {
         // the window that keeps an end knot recovers it from its own rows
         const int r0 = -g0, r1 = n - 1 - g0;
         if (r0 >= H && r0 < H + K) {
             const real c1 = window_row<real, B>(xs, r0 + 1), c2 = window_row<real, B>(xs, r0 + 2);
-            if (lane == 0) k.c[e0] = nak_end<real>(c1, c2, pa1 - pa0, pa2 - pa1);
+            if (lane == 0) k.c[e0] = nak_end<real>(c1, c2, he, hn);
         }
         if (r1 >= H && r1 < H + K) {
             const real c1 = window_row<real, B>(xs, r1 - 1), c2 = window_row<real, B>(xs, r1 - 2);
-            if (lane == 0) k.c[e0 + n - 1] = nak_end<real>(c1, c2, pz0 - pz1, pz1 - pz2);
+            if (lane == 1) k.c[e0 + n - 1] = nak_end<real>(c1, c2, -he, -hn);
         }
     }
 }
@@ -351,8 +375,8 @@ void k_stage(StageArgs<real> a)
                 }
                 tot[0] += __popcll(mx);
                 tot[1] += __popcll(mn);
-                mk = lane == tl * kWR + r ? mx : mk;
-                mk = lane == 32 + tl * kWR + r ? mn : mk;
+                set_lane(mk, mx, tl * kWR + r);
+                set_lane(mk, mn, 32 + tl * kWR + r);
             }
         };
         auto first_row = [&](real el, real v0) {
@@ -467,9 +491,9 @@ void k_stage(StageArgs<real> a)
                 break;
             }
             const bool use_mean = n[0] > 3 && n[1] > 3;
-            e1 = n[0] + Pad<real>::total;
-            entries = (e1 + n[1] + Pad<real>::total + 3) & ~3;
-            in_lds = HOLD || entries * kEntryBytes<real> <= a.lds_bytes;
+            e1 = (int)type_entries<real>(n[0]);
+            entries = e1 + (int)type_entries<real>(n[1]);
+            in_lds = HOLD || rows_bytes<real>(entries) <= a.lds_bytes;
             const bool last = !RILL && j == a.passes - 1;
             const real* const hin = j & 1 ? buf1 : buf0;                        // input of pass j
             real* const hout = last ? a.out + off : j & 1 ? buf0 : buf1;
@@ -480,9 +504,18 @@ void k_stage(StageArgs<real> a)
                 // ---- knots by index
                 {
                     int rb[2] = {base[0] + F, base[1] + F + e1};
+                    real nx[kWR];
+                    if constexpr (!HOLD) {
+                        if (nt > 0) fetch(hin, 0, nx);
+                    }
                     for (int tl = 0; tl < nt; ++tl) {
                         const int t0 = start + tl * kWT;
-                        if constexpr (!HOLD) fetch(hin, tl, hv);
+                        if constexpr (!HOLD) {
+                            // the next tile is requested before this one is used
+#pragma unroll
+                            for (int r = 0; r < kWR; ++r) hv[r] = nx[r];
+                            if (tl + 1 < nt) fetch(hin, tl + 1, nx);
+                        }
                         const int before[2] = {rb[0], rb[1]};
 #pragma unroll
                         for (int r = 0; r < kWR; ++r) {
@@ -543,8 +576,11 @@ void k_stage(StageArgs<real> a)
                 for (int w = wv; w < wmx + wmn; w += NWV) {
                     const int ty = w >= wmx, wi = ty ? w - wmx : w;
                     const int nty = ty ? n[1] : n[0];
-                    solve_window<real>(kr, (ty ? e1 : 0) + F, ty, nty, wi, lane, a.nak && nty >= 4,
-                                       s_fix[ty], REC ? a.rec[j].fixf + 4 * s + 2 * ty : nullptr);
+                    int* const fixf = REC ? a.rec[j].fixf + 4 * s + 2 * ty : nullptr;
+                    if (a.nak && nty >= 4)
+                        solve_window<real, true>(kr, (ty ? e1 : 0) + F, ty, nty, wi, lane, s_fix[ty], fixf);
+                    else
+                        solve_window<real, false>(kr, (ty ? e1 : 0) + F, ty, nty, wi, lane, s_fix[ty], fixf);
                 }
                 __syncthreads();
                 if (done) return;
@@ -685,8 +721,8 @@ StageGeom stage_geometry(int real_size, int64_t max_len, int64_t nseries)
     g.nwv = ntl <= 4 ? 4 : ntl <= 8 || (!f64 && ntl <= 16 && nseries > 256) ? 8 : 16;
     g.hold = ntl <= g.nwv;
     // knot rows of the densest pass (at most N + 4 knots of both types)
-    const int64_t entries = max_len + 4 + 2 * (f64 ? Pad<double>::total : Pad<float>::total) + 4;
-    const size_t worst = (size_t)entries * (f64 ? kEntryBytes<double> : kEntryBytes<float>);
+    const int64_t entries = max_len + 4 + 2 * (f64 ? type_entries<double>(0) : type_entries<float>(0)) + 16;
+    const size_t worst = (size_t)(f64 ? rows_bytes<double>(entries) : rows_bytes<float>(entries));
     const size_t most = 160 * 1024 - 2048;     // static arrays aside
     g.lds = std::min(worst, most);
     g.slot = worst <= most ? 0 : (worst + 255) / 256 * 256;
