@@ -1913,8 +1913,8 @@ __global__ __launch_bounds__(kThreads) void k_init_w(SeriesDev sd, InitArgs<real
 // lane l owns the four consecutive samples 4l .. 4l+3.  Optionally
 // mu <- broadcast, then mu <- mu - (G_max^T + G_min^T)/2 for the scatter
 // pass, then the moments of mu over the knot intervals of the moment pass.
-// Each lane sums its samples run by run, and what follows its last knot is
-// carried to the lane that holds the next one; the runs are put together in
+// Each lane sums its samples run by run, and the run that a lane leaves open
+// is carried to the lane that ends it; the runs are put together in
 // LDS and leave as contiguous 16-byte stores (written by the lanes that end
 // them, 32-byte pieces at two to four places, the dense FP64 launch took 703
 // us instead of 404).
@@ -1970,16 +1970,15 @@ __device__ __forceinline__ void open_scan_step(real (&v)[4], uint64_t take)
 }
 
 // Inclusive scan of the lanes' open sums: lane l ends with the sum over the
-// lanes from the last one below it with a knot (whose sum is what follows
-// that knot) to itself; `knot` = lanes with a knot.  Which lanes take part in
-// a step is known from the mask by scalar instructions, and a step that no
-// lane takes part in is left out (four lanes without a knot are rare in a
-// dense pass).
+// lanes down to the nearest one that is not linked to the lane before it.
+// Which lanes take part in a step is known from the mask of links by scalar
+// instructions, and a step that no lane takes part in is left out (four lanes
+// without a knot are rare in a dense pass).
 template <typename real>
-__device__ __forceinline__ void open_scan(real (&v)[4], uint64_t knot)
+__device__ __forceinline__ void open_scan(real (&v)[4], uint64_t link)
 {
-    // aN: no knot in the N lanes up to this one, or in its row of 16 so far
-    const uint64_t a1 = ~knot;
+    // aN: the N lanes up to this one are linked, or those of its row of 16
+    const uint64_t a1 = link;
     const uint64_t a2 = a1 & ((a1 << 1) | 0x0001000100010001ull);
     const uint64_t a4 = a2 & ((a2 << 2) | 0x0003000300030003ull);
     const uint64_t a8 = a4 & ((a4 << 4) | 0x000F000F000F000Full);
@@ -2089,20 +2088,8 @@ __device__ __forceinline__ void adj_tile(const AdjTileArgs<real>& a, int gt, int
 #pragma unroll
             for (int q = 0; q < 3; ++q) t[q + 1] = __builtin_amdgcn_inverse_ballot_w64(bm[q]) ? 1 : t[q] + 1;
         }
-        real p[4][3];
-#pragma unroll
-        for (int q = 0; q < 4; ++q) {
-            p[q][0] = (real)t[q];
-            p[q][1] = p[q][0] * p[q][0];
-            p[q][2] = p[q][1] * p[q][0];
-        }
-        auto add = [&](real (&m)[4], int q, real g) {
-            m[0] = m[0] + g;
-#pragma unroll
-            for (int z = 0; z < 3; ++z) m[z + 1] = fma(g, p[q][z], m[z + 1]);
-        };
-        // runs that end in the lane, their part before it still missing, and
-        // what follows the lane's last knot
+        // moments of the runs within the lane; one that ends on its last
+        // sample (or goes on) is open
         real run[4] = {(real)0, (real)0, (real)0, (real)0};
         int r = t0 == 0 ? 1 : 0;
 #pragma unroll
@@ -2111,20 +2098,33 @@ __device__ __forceinline__ void adj_tile(const AdjTileArgs<real>& a, int gt, int
         real* d = mine;
 #pragma unroll
         for (int q = 0; q < 4; ++q) {
-            add(run, q, v[q]);
-            if (__builtin_amdgcn_inverse_ballot_w64(bm[q])) {
+            real m = v[q];
+            run[0] = run[0] + m;
+#pragma unroll
+            for (int z = 1; z < 4; ++z) {
+                m = m * (real)t[q];
+                run[z] = run[z] + m;
+            }
+            if (q < 3 && __builtin_amdgcn_inverse_ballot_w64(bm[q])) {
                 store_four<false>(d, run);
                 d += 4;
 #pragma unroll
                 for (int z = 0; z < 4; ++z) run[z] = (real)0;
             }
         }
-        const uint64_t knot = bm[0] | bm[1] | bm[2] | bm[3];
-        open_scan(run, knot);
-        if (lane == kWave - 1) store_four<false>(e + (cnt > 0 ? 4 : 0), run);
+        const uint64_t inside = bm[0] | bm[1] | bm[2], after = bm[3] << 1;
+        open_scan(run, ~(inside | after));
+        if (__builtin_amdgcn_inverse_ballot_w64(bm[3])) store_four<false>(d, run);
+        if (lane == kWave - 1) {
+            real rest[4];
+#pragma unroll
+            for (int z = 0; z < 4; ++z) rest[z] = bm[3] >> 63 ? (real)0 : run[z];
+            store_four<false>(e + (cnt > 0 ? 4 : 0), rest);
+        }
+        // the first run that ends inside the lane goes on from the lane before
 #pragma unroll
         for (int z = 0; z < 4; ++z) run[z] = shift_prev(run[z], (real)0);
-        if (__builtin_amdgcn_inverse_ballot_w64(knot)) {
+        if (__builtin_amdgcn_inverse_ballot_w64(inside & ~after)) {
             real m[4];
             load_four<false>(mine, m);
 #pragma unroll
