@@ -727,25 +727,25 @@ __global__ __launch_bounds__(kThreads) void k_knot_prefix_w(SeriesDev sd, KnotsD
 // g - lo), from the tile bitmasks (mask [tile][type][row]), knot prefixes and
 // counts.  One wavefront; tpre (64 ints) and tmask (64 x 4 words) are LDS
 // scratch.  Tiles are taken 64 at a time (their prefixes and masks in LDS).
-// When the knots of a chunk lie in few tiles (dense knots), every lane tests
-// its own bit of each tile row and the set bits' ranks give the knot
-// indices; otherwise each lane finds the tile of its knots g + lane + 64 j by
-// binary search and the knot's bit by selection.  hint = the tile holding
-// knot glo, or -1 (64-ary search).  NIT >= the knots of one window / 64.
+// When the knots of a chunk lie in up to 40 tiles, each lane walks the set
+// bits of 32 samples at a time; otherwise of its own tile (solve launches, 16
+// ragged FP32 series x 100, with the line at 16 / 40 / 64 tiles: 36.2 / 35.9 /
+// 36.4 ms, 36.9 when every lane of a few-tile chunk tested its own bit of each
+// row; one FP64 series of 244032 x 200: 16.32 / 16.30 / 17.4, before 16.4).
+// hint = the tile holding knot glo, or -1 (64-ary search).
 // (inlined: as a called function it cost the solve 8 % and the adjoint
 // window solve 1 %)
 // row masks of one staged tile in LDS (TW words per tile).  The adjoint
 // pads them from 4 to 5 words: the 64 lanes store their tiles' rows at a
 // 40-byte stride instead of 32, which spreads the stores over the banks.
-// The solve keeps 4: 2 KB less LDS per workgroup gives its FP32 instance a
-// sixth wave per SIMD, which is worth more than the conflicts (-2.5 %).
+// The solve keeps 4: 2 KB less LDS per workgroup.
 constexpr int kTMaskW = kWR + 1;
 
 template <int TW>
 __device__ __forceinline__ void gather_positions(const SeriesDev& sd, const uint64_t* kmask,
                                                  const int* kpre, const int* kcnt, int s, int type,
                                                  long lo, int glo, int ghi, int* sp, int* tpre,
-                                                 uint64_t (*tmask)[TW], int hint)
+                                                 uint64_t (*tmask)[TW], int hint, int n)
 {
     const int lane = threadIdx.x & 63;
     const int tb = load_scalar(sd.tile0 + s), ntl = load_scalar(sd.ntl + s);
@@ -761,14 +761,34 @@ __device__ __forceinline__ void gather_positions(const SeriesDev& sd, const uint
     }
     int g = glo;
     int tile = a;
+    // the lane's tile of a chunk: prefix, count, row masks
+    struct Chunk {
+        int p, c;
+        uint64_t mk[kWR];
+    };
+    auto request = [&](int first, Chunk& q) {
+        const int tl = first + lane;
+        const bool valid = tl < ntl;
+        q.p = valid ? kpre[2 * (tb + tl) + type] : 0x7FFFFFFF;
+        q.c = valid ? kcnt[2 * (tb + tl) + type] : 0;
+#pragma unroll
+        for (int r = 0; r < kWR; ++r) q.mk[r] = valid ? kmask[8 * (int64_t)(tb + tl) + kWR * type + r] : 0ull;
+    };
+    Chunk cur, nxt;
+    request(tile, cur);
+    const bool sparse = (int64_t)(ghi - glo) * ntl > (int64_t)n * kWave;
     while (g < ghi) {
+        // where a window spans more than one chunk, the next is requested
+        // before this one is waited for (FP32 solve launches 35.9 -> 35.8 ms,
+        // FP64 16.30 -> 16.20)
         const int tl = tile + lane;
         const bool valid = tl < ntl;
-        const int p = valid ? kpre[2 * (tb + tl) + type] : 0x7FFFFFFF;
-        const int c = valid ? kcnt[2 * (tb + tl) + type] : 0;
+        const bool ahead = sparse && tile + kWave < ntl;
+        if (ahead) request(tile + kWave, nxt);
+        const int p = cur.p, c = cur.c;
         uint64_t mk[kWR];
 #pragma unroll
-        for (int r = 0; r < kWR; ++r) mk[r] = valid ? kmask[8 * (int64_t)(tb + tl) + kWR * type + r] : 0ull;
+        for (int r = 0; r < kWR; ++r) mk[r] = cur.mk[r];
         tpre[lane] = p;
 #pragma unroll
         for (int r = 0; r < kWR; ++r) tmask[lane][r] = mk[r];
@@ -782,29 +802,28 @@ __device__ __forceinline__ void gather_positions(const SeriesDev& sd, const uint
         const int xa = ua ? 63 - __builtin_clzll(ua) : 0;
         const int xb = ub ? 63 - __builtin_clzll(ub) : 0;
         wave_sync();
-        if (xb - xa < 16) {
-            // few tiles with many knots each: the wave goes through the
-            // tiles, one lane per sample of a row
-            for (int x = xa; x <= xb; ++x) {
-                // the tile's prefix and four row masks in one round of LDS
-                // reads, moved to scalar registers (the same in every lane):
-                // the lane test is then the exec mask, the counts scalar
-                int cb = __builtin_amdgcn_readfirstlane(tpre[x]);
-                uint64_t mr[kWR];
-#pragma unroll
-                for (int r = 0; r < kWR; ++r) {
-                    const uint64_t m = tmask[x][r];
-                    mr[r] = ((uint64_t)(uint32_t)__builtin_amdgcn_readfirstlane((int)(m >> 32)) << 32) |
-                            (uint32_t)__builtin_amdgcn_readfirstlane((int)(uint32_t)m);
-                }
-#pragma unroll
-                for (int r = 0; r < kWR; ++r) {
-                    if (__builtin_amdgcn_inverse_ballot_w64(mr[r])) {
-                        const int gi = __builtin_amdgcn_mbcnt_hi(
-                            (uint32_t)(mr[r] >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)mr[r], (uint32_t)cb));
-                        if (gi >= g && gi < gend) sp[gi - lo] = (tile + x) * kWT + kWave * r + lane;
-                    }
-                    cb += __popcll(mr[r]);
+        if (xb - xa < 40) {
+            // a lane per 32 samples: it walks the set bits of its word, from
+            // the rank that its tile's prefix and the words before it give
+            for (int q0 = 8 * xa; q0 <= 8 * xb; q0 += kWave) {
+                const int x = (q0 + lane) >> 3, sub = lane & 7;
+                const bool in = x <= xb;
+                uint32_t m = in ? ((const uint32_t*)tmask[in ? x : 0])[sub] : 0u;
+                int before = __popc(m);
+                int gi = (in ? tpre[in ? x : 0] : 0) - before;
+                const int s1 = dpp_row_i<0x111, 0xF>(before, 0);
+                before += sub >= 1 ? s1 : 0;
+                const int s2 = dpp_row_i<0x112, 0xF>(before, 0);
+                before += sub >= 2 ? s2 : 0;
+                const int s4 = dpp_row_i<0x114, 0xF>(before, 0);
+                before += sub >= 4 ? s4 : 0;
+                gi += before;
+                const int pos = (tile + x) * kWT + 32 * sub;
+                while (m != 0u) {
+                    const int bit = __builtin_ctz(m);
+                    m &= m - 1u;
+                    if ((unsigned)(gi - g) < (unsigned)(gend - g)) sp[gi - lo] = pos + bit;
+                    ++gi;
                 }
             }
         } else if (lane >= xa && lane <= xb) {
@@ -825,6 +844,8 @@ __device__ __forceinline__ void gather_positions(const SeriesDev& sd, const uint
         g = gend;
         tile += kWave;
         wave_sync();
+        if (ahead) cur = nxt;
+        else if (g < ghi) request(tile, cur);
     }
 }
 
@@ -890,7 +911,7 @@ __global__ __launch_bounds__(kThreads) void k_solve(SolveArgs<real> a)
         const int ghi = (int)min(lo + W + 2, (long)n);
         constexpr int NIT = (W + 2 + kWave - 1) / kWave;
         gather_positions<kWR>(a.sd, a.k.mask, a.k.pre, a.k.cnt, s, type, lo, glo, ghi, sp,
-                              s_tpre[wv], s_tmask[wv], hint);
+                              s_tpre[wv], s_tmask[wv], hint, n);
         wave_sync();
         gather_values<real, NIT>(a.h + load_scalar(a.sd.off + s), load_scalar(a.sd.len + s), lo, glo,
                                  ghi, sp, sy);
@@ -2249,7 +2270,7 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(3))) v
         const int glo = (int)max(lo, 0L);
         const int ghi = (int)min(lo + W + 2, (long)n);
         gather_positions<kTMaskW>(a.sd, a.ps.mask, a.ps.pre, a.ps.cnt, s, type, lo, glo, ghi, sp,
-                                  s_tpre[wv], s_tmask[wv], hint);
+                                  s_tpre[wv], s_tmask[wv], hint, n);
         wave_sync();
         // lane l owns window rows r = l*B + q (knot gb + q); everything a row
         // needs comes from its own lane's registers or a neighbour lane's
