@@ -100,29 +100,64 @@ __device__ __forceinline__ void load_masks(const KnotsDev<real>& k, int64_t gt, 
     for (int r = 0; r < kWR; ++r) m[r] = k.mask[8 * gt + kWR * type + r];
 }
 
+// The last knot and the one before it among some tiles (positions, -1 =
+// none).  Positions are distinct, so combining two sets needs no order.
 struct LastTwo {
-    int c;
-    int64_t l1, l2;
+    int a, b;
 };
 
 __device__ __forceinline__ LastTwo lt_combine(const LastTwo& A, const LastTwo& B)
 {
-    // written as selects (no early returns) so the result stays in registers
-    LastTwo r;
-    r.c = B.c >= 2 ? 2 : (B.c == 1 ? min(A.c + 1, 2) : A.c);
-    r.l1 = B.c >= 1 ? B.l1 : A.l1;
-    r.l2 = B.c >= 2 ? B.l2 : (B.c == 1 ? A.l1 : A.l2);
-    return r;
+    return LastTwo{max(A.a, B.a), max(max(A.b, B.b), min(A.a, B.a))};
 }
 
-__device__ __forceinline__ LastTwo lt_shfl_up(const LastTwo& v, int o)
+__device__ __forceinline__ LastTwo lt_none() { return LastTwo{-1, -1}; }
+
+// Inclusive scans over the lanes by lane moves inside the vector unit (two to
+// five instructions a step; by ds_bpermute each took a round trip to LDS, and
+// a decomposition of 16 ragged FP32 series x 100 took 177.2 ms instead of
+// 174.7): sums, last two knots, and (downwards) the least value of the lanes
+// from this one.
+__device__ __forceinline__ int sum_scan(int v)
 {
-    LastTwo r;
-    r.c = shfl_up(v.c, o);
-    r.l1 = shfl_up(v.l1, o);
-    r.l2 = shfl_up(v.l2, o);
-    return r;
+    v += dpp_row_i<0x111, 0xF>(v, 0);
+    v += dpp_row_i<0x112, 0xF>(v, 0);
+    v += dpp_row_i<0x114, 0xF>(v, 0);
+    v += dpp_row_i<0x118, 0xF>(v, 0);
+    v += dpp_row_i<0x142, 0xA>(v, 0);
+    v += dpp_row_i<0x143, 0xC>(v, 0);
+    return v;
 }
+template <int CTRL, int ROWS>
+__device__ __forceinline__ void lt_step(LastTwo& v)
+{
+    v = lt_combine(LastTwo{dpp_row_i<CTRL, ROWS>(v.a, -1), dpp_row_i<CTRL, ROWS>(v.b, -1)}, v);
+}
+__device__ __forceinline__ LastTwo lt_scan(LastTwo v)
+{
+    lt_step<0x111, 0xF>(v);
+    lt_step<0x112, 0xF>(v);
+    lt_step<0x114, 0xF>(v);
+    lt_step<0x118, 0xF>(v);
+    lt_step<0x142, 0xA>(v);
+    lt_step<0x143, 0xC>(v);
+    return v;
+}
+__device__ __forceinline__ int suffix_min(int v)
+{
+    constexpr int INF = 0x7FFFFFFF;
+    v = min(v, dpp_row_i<0x101, 0xF>(v, INF));
+    v = min(v, dpp_row_i<0x102, 0xF>(v, INF));
+    v = min(v, dpp_row_i<0x104, 0xF>(v, INF));
+    v = min(v, dpp_row_i<0x108, 0xF>(v, INF));
+    // rows 1, 2, 3 begin at lanes 16, 32, 48
+    const int r3 = __builtin_amdgcn_readlane(v, 48), r2 = min(__builtin_amdgcn_readlane(v, 32), r3);
+    const int r1 = min(__builtin_amdgcn_readlane(v, 16), r2);
+    const int row = (threadIdx.x & 63) >> 4;
+    return min(v, row == 0 ? r1 : row == 1 ? r2 : row == 2 ? r3 : INF);
+}
+// what the lanes before this one hold together (after a scan)
+__device__ __forceinline__ LastTwo lt_before(const LastTwo& v) { return LastTwo{dpp_prev_i(v.a, -1), dpp_prev_i(v.b, -1)}; }
 
 // Knot prefix: per-series exclusive scan of the tile knot counts (the CUB
 // ExclusiveSum of cudaICEEMDAN.cu:859-883, over tiles instead of samples),
@@ -134,15 +169,6 @@ __device__ __forceinline__ LastTwo lt_shfl_up(const LastTwo& v, int o)
 // thread (chunks of 1024 tiles): workgroup scans forward (counts, last two
 // knots) and backward (next knot), carried from chunk to chunk.
 constexpr int kPT = 1024;
-
-__device__ __forceinline__ LastTwo lt_none()
-{
-    LastTwo r;
-    r.c = 0;
-    r.l1 = -1;
-    r.l2 = -1;
-    return r;
-}
 
 // Window item w of a series with wmx windows of maxima and wmn of minima:
 // the two types alternate (maxima window i, then minima window i), so the
@@ -200,22 +226,13 @@ __global__ __launch_bounds__(kPT) void k_knot_prefix_b(SeriesDev sd, KnotsDev<re
                 load_masks(k, tb + t, ty, m);
                 const int b1 = mask_last(m);
                 m[b1 / kWave] ^= 1ull << (b1 % kWave);
-                own.c = min(c, 2);
-                own.l1 = (int64_t)t * kWT + b1;
-                own.l2 = c >= 2 ? (int64_t)t * kWT + mask_last(m) : -1;
+                own.a = t * kWT + b1;
+                own.b = c >= 2 ? t * kWT + mask_last(m) : -1;
             }
-            int inc = c;
-            LastTwo sc = own;
-            for (int o = 1; o < kWave; o <<= 1) {
-                const int v = shfl_up(inc, o);
-                const LastTwo w = lt_shfl_up(sc, o);
-                if (lane >= o) {
-                    inc += v;
-                    sc = lt_combine(w, sc);
-                }
-            }
-            const int xi = shfl_up(inc, 1);
-            const LastTwo xl = lt_shfl_up(sc, 1);
+            const int inc = sum_scan(c);
+            const LastTwo sc = lt_scan(own);
+            const int xi = dpp_prev_i(inc, 0);
+            const LastTwo xl = lt_before(sc);
             __syncthreads();   // earlier readers of s_* are done
             if (lane == kWave - 1) {
                 s_tot[wv] = inc;
@@ -224,22 +241,13 @@ __global__ __launch_bounds__(kPT) void k_knot_prefix_b(SeriesDev sd, KnotsDev<re
             __syncthreads();
             if (wv == 0) {
                 // exclusive scan of the wave totals by the first NWV lanes
-                int v = lane < NWV ? s_tot[lane] : 0;
-                LastTwo l = lane < NWV ? s_lt[lane] : lt_none();
-                int vi = v;
-                LastTwo li = l;
-                for (int o = 1; o < NWV; o <<= 1) {
-                    const int a1 = shfl_up(vi, o);
-                    const LastTwo b1 = lt_shfl_up(li, o);
-                    if (lane >= o) {
-                        vi += a1;
-                        li = lt_combine(b1, li);
-                    }
-                }
-                const LastTwo le = lt_shfl_up(li, 1);
+                const int v = lane < NWV ? s_tot[lane] : 0;
+                const int vi = sum_scan(v);
+                const LastTwo li = lt_scan(lane < NWV ? s_lt[lane] : lt_none());
+                const LastTwo le = lt_before(li);
                 if (lane < NWV) {
                     s_ex_tot[lane] = vi - v;
-                    s_ex_lt[lane] = lane > 0 ? le : lt_none();
+                    s_ex_lt[lane] = le;
                 }
                 if (lane == NWV - 1) {
                     s_all = vi;
@@ -247,17 +255,16 @@ __global__ __launch_bounds__(kPT) void k_knot_prefix_b(SeriesDev sd, KnotsDev<re
                 }
             }
             __syncthreads();
-            const int ex = carry + s_ex_tot[wv] + (lane > 0 ? xi : 0);
-            const LastTwo before =
-                lt_combine(carry_lt, lt_combine(s_ex_lt[wv], lane > 0 ? xl : lt_none()));
+            const int ex = carry + s_ex_tot[wv] + xi;
+            const LastTwo before = lt_combine(carry_lt, lt_combine(s_ex_lt[wv], xl));
             if (t < nt) {
                 k.pre[2 * (tb + t) + ty] = ex;
                 const int64_t o = 6 * (int64_t)(tb + t) + 3 * ty;
-                k.nbx[o] = before.l1 >= 0 ? (int)before.l1 : -1;
-                k.nby[o] = before.l1 >= 0 ? hs[before.l1] : (real)0;
-                k.nbx[o + 1] = before.l2 >= 0 ? (int)before.l2 : -1;
-                k.nby[o + 1] = before.l2 >= 0 ? hs[before.l2] : (real)0;
-                if (k.left) k.left[2 * (tb + t) + ty] = (int)before.l1;
+                k.nbx[o] = before.a;
+                k.nby[o] = before.a >= 0 ? hs[before.a] : (real)0;
+                k.nbx[o + 1] = before.b;
+                k.nby[o + 1] = before.b >= 0 ? hs[before.b] : (real)0;
+                if (k.left) k.left[2 * (tb + t) + ty] = before.a;
             }
             carry += s_all;
             carry_lt = lt_combine(carry_lt, s_all_lt);
@@ -268,16 +275,12 @@ __global__ __launch_bounds__(kPT) void k_knot_prefix_b(SeriesDev sd, KnotsDev<re
         for (int base = ((nt - 1) / kPT) * kPT; base >= 0; base -= kPT) {
             const int t = base + tid;
             const int c = t < nt ? k.cnt[2 * (tb + t) + ty] : 0;
-            int mn = c > 0 ? t : INF;
-            for (int o = 1; o < kWave; o <<= 1) {
-                const int m = shfl_down(mn, o);
-                if (lane + o < kWave) mn = min(mn, m);
-            }
-            const int xm = shfl_down(mn, 1);
+            const int mn = suffix_min(c > 0 ? t : INF);
+            const int xm = dpp_next_i(mn, INF);
             __syncthreads();
             if (lane == 0) s_min[wv] = mn;
             __syncthreads();
-            int after = min(carry_min, lane < kWave - 1 ? xm : INF);
+            int after = min(carry_min, xm);
             int all = carry_min;
             for (int w = 0; w < NWV; ++w) {
                 if (w > wv) after = min(after, s_min[w]);
@@ -363,9 +366,8 @@ __global__ __launch_bounds__(kPT) void k_knot_prefix_1(SeriesDev sd, KnotsDev<re
             first[ty] = mask_first(m);
             const int b1 = mask_last(m);
             m[b1 / kWave] ^= 1ull << (b1 % kWave);
-            sc[ty].c = min(c[ty], 2);
-            sc[ty].l1 = (int64_t)t * kWT + b1;
-            sc[ty].l2 = c[ty] >= 2 ? (int64_t)t * kWT + mask_last(m) : -1;
+            sc[ty].a = t * kWT + b1;
+            sc[ty].b = c[ty] >= 2 ? t * kWT + mask_last(m) : -1;
         }
         inc[ty] = c[ty];
         mn[ty] = c[ty] > 0 ? t : INF;
@@ -375,26 +377,16 @@ __global__ __launch_bounds__(kPT) void k_knot_prefix_1(SeriesDev sd, KnotsDev<re
         const unsigned d = (unsigned)__popcll(wave_ballot(c[0] + 3 > kWKS || c[1] + 3 > kWKS));
         if (lane == 0) s_dense[wv] = d;
     }
-    for (int o = 1; o < kWave; o <<= 1) {
-#pragma unroll
-        for (int ty = 0; ty < 2; ++ty) {
-            const int v = shfl_up(inc[ty], o);
-            const LastTwo w = lt_shfl_up(sc[ty], o);
-            const int m = shfl_down(mn[ty], o);
-            if (lane >= o) {
-                inc[ty] += v;
-                sc[ty] = lt_combine(w, sc[ty]);
-            }
-            if (lane + o < kWave) mn[ty] = min(mn[ty], m);
-        }
-    }
     int xi[2], xm[2];
     LastTwo xl[2];
 #pragma unroll
     for (int ty = 0; ty < 2; ++ty) {
-        xi[ty] = shfl_up(inc[ty], 1);
-        xl[ty] = lt_shfl_up(sc[ty], 1);
-        xm[ty] = shfl_down(mn[ty], 1);
+        inc[ty] = sum_scan(inc[ty]);
+        sc[ty] = lt_scan(sc[ty]);
+        mn[ty] = suffix_min(mn[ty]);
+        xi[ty] = dpp_prev_i(inc[ty], 0);
+        xl[ty] = lt_before(sc[ty]);
+        xm[ty] = dpp_next_i(mn[ty], INF);
         if (lane == kWave - 1) {
             s_tot[ty][wv] = inc[ty];
             s_lt[ty][wv] = sc[ty];
@@ -408,26 +400,14 @@ __global__ __launch_bounds__(kPT) void k_knot_prefix_1(SeriesDev sd, KnotsDev<re
 #pragma unroll
         for (int ty = 0; ty < 2; ++ty) {
             const int v = lane < NWV ? s_tot[ty][lane] : 0;
-            const LastTwo l = lane < NWV ? s_lt[ty][lane] : lt_none();
-            const int m0 = lane < NWV ? s_min[ty][lane] : INF;
-            int vi = v, mi = m0;
-            LastTwo li = l;
-            for (int o = 1; o < NWV; o <<= 1) {
-                const int a1 = shfl_up(vi, o);
-                const LastTwo b1 = lt_shfl_up(li, o);
-                const int c1 = shfl_down(mi, o);
-                if (lane >= o) {
-                    vi += a1;
-                    li = lt_combine(b1, li);
-                }
-                if (lane + o < NWV) mi = min(mi, c1);
-            }
-            const LastTwo le = lt_shfl_up(li, 1);
-            const int me = shfl_down(mi, 1);
+            const int vi = sum_scan(v), mi = suffix_min(lane < NWV ? s_min[ty][lane] : INF);
+            const LastTwo li = lt_scan(lane < NWV ? s_lt[ty][lane] : lt_none());
+            const LastTwo le = lt_before(li);
+            const int me = dpp_next_i(mi, INF);
             if (lane < NWV) {
                 s_ex_tot[ty][lane] = vi - v;
-                s_ex_lt[ty][lane] = lane > 0 ? le : lt_none();
-                s_ex_min[ty][lane] = lane < NWV - 1 ? me : INF;
+                s_ex_lt[ty][lane] = le;
+                s_ex_min[ty][lane] = me;
             }
             if (lane == NWV - 1) s_all[ty] = vi;
         }
@@ -440,11 +420,11 @@ __global__ __launch_bounds__(kPT) void k_knot_prefix_1(SeriesDev sd, KnotsDev<re
         int ex[2], xs[2][3];
 #pragma unroll
         for (int ty = 0; ty < 2; ++ty) {
-            ex[ty] = s_ex_tot[ty][wv] + (lane > 0 ? xi[ty] : 0);
-            const LastTwo before = lt_combine(s_ex_lt[ty][wv], lane > 0 ? xl[ty] : lt_none());
-            const int after = min(s_ex_min[ty][wv], lane < kWave - 1 ? xm[ty] : INF);
-            xs[ty][0] = before.l1 >= 0 ? (int)before.l1 : -1;
-            xs[ty][1] = before.l2 >= 0 ? (int)before.l2 : -1;
+            ex[ty] = s_ex_tot[ty][wv] + xi[ty];
+            const LastTwo before = lt_combine(s_ex_lt[ty][wv], xl[ty]);
+            const int after = min(s_ex_min[ty][wv], xm[ty]);
+            xs[ty][0] = before.a;
+            xs[ty][1] = before.b;
             xs[ty][2] = after == INF ? -1 : after * kWT + s_first[ty][after];
         }
         real ys[2][3];
@@ -522,36 +502,13 @@ __global__ __launch_bounds__(kPT) void k_knot_prefix_1(SeriesDev sd, KnotsDev<re
 // free (a 1024-thread workgroup needs 16 free slots on one CU at once, and
 // then waited for the other stream's sift to drain: 3.5 ms per pass beside
 // it against 0.5 ms alone).
-struct Two {
-    int c, l1, l2;   // number of knots seen (at most 2), the last, the one before
-};
-
-__device__ __forceinline__ Two two_none() { return Two{0, -1, -1}; }
-
-__device__ __forceinline__ Two two_combine(const Two& A, const Two& B)
-{
-    Two r;
-    r.c = B.c >= 2 ? 2 : (B.c == 1 ? min(A.c + 1, 2) : A.c);
-    r.l1 = B.c >= 1 ? B.l1 : A.l1;
-    r.l2 = B.c >= 2 ? B.l2 : (B.c == 1 ? A.l1 : A.l2);
-    return r;
-}
-
-__device__ __forceinline__ Two two_shfl_up(const Two& v, int o)
-{
-    return Two{shfl_up(v.c, o), shfl_up(v.l1, o), shfl_up(v.l2, o)};
-}
-
-__device__ __forceinline__ Two two_lane(const Two& v, int l)
-{
-    return Two{__builtin_amdgcn_readlane(v.c, l), __builtin_amdgcn_readlane(v.l1, l),
-                __builtin_amdgcn_readlane(v.l2, l)};
-}
-
 // windows per type of a series of at most kPT tiles: <= 129 knots per tile
 // and type, K >= 448 rows kept per window
 constexpr int kPWin = (kPT * 129 + 447) / 448 + 1;
-// series length (tiles) up to which the one-wave kernel is used
+// series length (tiles) up to which the one-wave kernel is used (a wave takes
+// 64 tiles at a time, one after the other: on 200 series of 954 tiles it more
+// than doubled what a decomposition spends outside init, solve and sift, 10.0
+// -> 21.9 ms; where a 1024-thread workgroup would be mostly idle it is ahead)
 constexpr int kPWTiles = 128;
 
 template <typename real>
@@ -583,7 +540,7 @@ __global__ __launch_bounds__(kThreads) void k_knot_prefix_w(SeriesDev sd, KnotsD
     };
 
     int carry[2] = {0, 0};
-    Two carry_lt[2] = {two_none(), two_none()};
+    LastTwo carry_lt[2] = {lt_none(), lt_none()};
     unsigned dense = 0;   // tiles the small sift table cannot hold
     int c[2], cn[2] = {0, 0};
     uint64_t m[2 * kWR], mn[2 * kWR] = {};
@@ -600,32 +557,21 @@ __global__ __launch_bounds__(kThreads) void k_knot_prefix_w(SeriesDev sd, KnotsD
             uint64_t mm[kWR];
 #pragma unroll
             for (int r = 0; r < kWR; ++r) mm[r] = m[ty * kWR + r];
-            Two own = two_none();
+            LastTwo own = lt_none();
             fp[ty] = -1;
             if (c[ty] > 0) {
                 fp[ty] = t * kWT + mask_first(mm);
                 const int b1 = mask_last(mm);
                 mm[b1 / kWave] ^= 1ull << (b1 % kWave);
-                own.c = min(c[ty], 2);
-                own.l1 = t * kWT + b1;
-                own.l2 = c[ty] >= 2 ? t * kWT + mask_last(mm) : -1;
+                own.a = t * kWT + b1;
+                own.b = c[ty] >= 2 ? t * kWT + mask_last(mm) : -1;
             }
-            int inc = c[ty];
-            Two sc = own;
-#pragma unroll
-            for (int o = 1; o < kWave; o <<= 1) {
-                const int v = shfl_up(inc, o);
-                const Two w = two_shfl_up(sc, o);
-                if (lane >= o) {
-                    inc += v;
-                    sc = two_combine(w, sc);
-                }
-            }
+            const int inc = sum_scan(c[ty]);
+            const LastTwo sc = lt_scan(own);
             ex[ty] = carry[ty] + inc - c[ty];
-            const Two xl = two_shfl_up(sc, 1);
-            const Two before = two_combine(carry_lt[ty], lane > 0 ? xl : two_none());
-            xb[ty][0] = before.l1;
-            xb[ty][1] = before.l2;
+            const LastTwo before = lt_combine(carry_lt[ty], lt_before(sc));
+            xb[ty][0] = before.a;
+            xb[ty][1] = before.b;
             // the window whose first gathered knot (max(w K - H - 1, 0)) lies
             // in this tile: at most one, as K exceeds a tile's knots
             if (c[ty] > 0) {
@@ -634,7 +580,8 @@ __global__ __launch_bounds__(kThreads) void k_knot_prefix_w(SeriesDev sd, KnotsD
                 if (w >= 1 && w < kPWin && w * K - H - 1 >= ex[ty]) s_hint[wv][ty][w] = t;
             }
             carry[ty] += __builtin_amdgcn_readlane(inc, kWave - 1);
-            carry_lt[ty] = two_combine(carry_lt[ty], two_lane(sc, kWave - 1));
+            carry_lt[ty] = lt_combine(carry_lt[ty], LastTwo{__builtin_amdgcn_readlane(sc.a, kWave - 1),
+                                                            __builtin_amdgcn_readlane(sc.b, kWave - 1)});
         }
         // values of the knots before the tile (positions of knots that exist,
         // or 0), all loads before the stores
@@ -673,14 +620,8 @@ __global__ __launch_bounds__(kThreads) void k_knot_prefix_w(SeriesDev sd, KnotsD
 #pragma unroll
         for (int ty = 0; ty < 2; ++ty) {
             const int f = in ? k.nbx[6 * gt + 3 * ty + 2] : -1;
-            int mnv = f >= 0 ? f : INF;
-#pragma unroll
-            for (int o = 1; o < kWave; o <<= 1) {
-                const int v = shfl_down(mnv, o);
-                if (lane + o < kWave) mnv = min(mnv, v);
-            }
-            const int nx = shfl_down(mnv, 1);
-            after[ty] = min(cmin[ty], lane < kWave - 1 ? nx : INF);
+            const int mnv = suffix_min(f >= 0 ? f : INF);
+            after[ty] = min(cmin[ty], dpp_next_i(mnv, INF));
             cmin[ty] = min(cmin[ty], __builtin_amdgcn_readlane(mnv, 0));
         }
         real ya[2];
