@@ -9,7 +9,7 @@
 // launch-per-step kernels (icm_spline.h), on the same windows, so the two
 // paths give the same bits.
 //
-// Layout of a series in the workgroup: wave w owns `tpw` consecutive tiles of
+// Layout of a series in the workgroup: a wave owns consecutive tiles of
 // 256 samples, lane l the samples 64 r + l of each.  A pass is
 //   samples     the stage start, or both envelopes of the previous pass at
 //               the wave's own samples (and at the two samples beside them)
@@ -329,9 +329,13 @@ void k_stage(StageArgs<real> a)
         const int N = uni ? a.uniform_len : a.sd.len[s];
         const int64_t off = uni ? (int64_t)s * N : a.sd.off[s];
         const int ntl = (N + kWT - 1) / kWT;
-        const int tpw = HOLD ? 1 : (ntl + NWV - 1) / NWV;
-        const int t_first = wv * tpw;
-        const int nt = max(0, min(tpw, ntl - t_first));     // tiles of this wave
+        // tiles of this wave: the first waves have one more where they do not
+        // divide evenly (waves go to the SIMDs in turn, so these share alike;
+        // with ceil(tiles / waves) for all but the last, a sparse pass of 10007
+        // FP32 samples took 25.4 thousand cycles instead of 22.1, of 30504 60.1
+        // instead of 56.9)
+        const int rest = ntl % NWV, t_first = wv * (ntl / NWV) + min(wv, rest);
+        const int nt = ntl / NWV + (wv < rest ? 1 : 0);
         const int start = t_first * kWT, end = min(start + nt * kWT, N);
         // sample buffers: RILLING alternates hA and hB (a series that stops
         // at pass j exports the input of pass j); FIXED keeps one
