@@ -706,21 +706,25 @@ void launch_one(const StageArgs<real>& a, unsigned grid, size_t lds, hipStream_t
 }  // namespace
 
 // Which phases take the stage kernel, and its workgroup.  Measured per pass
-// (us) against the launch-per-step path on EEG-like noise-mode stages:
+// (us) against the tuned launch-per-step path on EEG-like noise-mode stages
+// (the first four rows: an earlier state of both):
 //   series x samples    FP32 steps / stage     FP64 steps / stage
 //     50 x   1000           30.9 /  5.7            35.2 /  7.4
 //   4000 x   1000           94.8 / 25.9           118.2 / 44.3
 //     50 x   4000           33.3 /  7.0            37.3 /  9.1
 //   4000 x   4000          147.7 / 84.8           211.6 / 142.6
-//    500 x   8000           46.7 / 21.9            61.6 / 44.7
-//   4000 x   8000          218.4 / 172.7          332.4 / 352.3
-//    500 x  16000           65.9 / 42.7            91.7 / 79.0
-//   1500 x  16000          147.0 / 126.0          231.2 / 235.2
-//    500 x  32000          104.2 / 88.9           158.8 / 167.8
+//   4000 x   8000          246.3 / 182.4          347.8 / 288.8
+//   3000 x  16000          295.9 / 242.4          434.4 / 363.6
+//    500 x  24000           88.9 / 56.1           126.3 / 87.4
+//   3000 x  24000          410.8 / 334.1          606.2 / 509.0
+//    250 x  32000           70.4 / 39.3            95.6 / 68.6
+//    500 x  32000          108.7 / 76.6           155.0 / 133.5
+//    800 x  32000          153.5 / 144.5          232.0 / 253.1
+//   3000 x  32000          528.6 / 457.4          783.6 / 806.8
 // A workgroup sifts one series at a time and one fits a CU from about 2000
 // samples on, so its time grows with series / 256 while the launch-per-step
-// path spreads any one pass over the chip: the line falls where the series
-// are both long and many, earlier in FP64 (half as many knots fit LDS).
+// path spreads any one pass over the chip: only FP64 series of more than 96
+// tiles lose here, beyond three workgroups per CU.
 // Waves per workgroup: one tile each as far as 16 waves go (the shortest
 // pass); FP32 series of up to 16 tiles in plans of more series than CUs take
 // 8 waves, so that two workgroups share a CU (500 x 4000: 11.8 against 13.4).
@@ -729,8 +733,7 @@ StageGeom stage_geometry(int real_size, int64_t max_len, int64_t nseries)
     StageGeom g{};
     const bool f64 = real_size == 8;
     const int64_t ntl = (max_len + kWT - 1) / kWT;
-    const int64_t most_series = f64 ? (ntl <= 16 ? INT64_MAX : ntl <= 32 ? 1536 : ntl <= 64 ? 1024 : 0)
-                                    : (ntl <= 64 ? INT64_MAX : ntl <= 128 ? 768 : 0);
+    const int64_t most_series = ntl > 128 ? 0 : f64 && ntl > 96 ? 768 : INT64_MAX;
     if (nseries > most_series) return g;
     g.nwv = ntl <= 4 ? 4 : ntl <= 8 || (!f64 && ntl <= 16 && nseries > 256) ? 8 : 16;
     g.hold = ntl <= g.nwv;
