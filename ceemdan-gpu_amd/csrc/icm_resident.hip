@@ -112,6 +112,23 @@ __device__ __forceinline__ real window_row(const real (&x)[B], int r)
     return v;
 }
 
+// Record of pass j with its pointers as ones to global memory (pointers read
+// from memory are generic, and generic accesses wait for LDS as well).
+template <typename T>
+using Global = __attribute__((address_space(1))) T*;
+struct PassRecord {
+    Global<uint64_t> mask;
+    Global<int> left, right, cnt, pre, n, fixf, winlist;
+    unsigned* wincount;
+};
+__device__ __forceinline__ PassRecord record(const StageRec* rec, int j)
+{
+    const StageRec& r = rec[j];
+    return PassRecord{(Global<uint64_t>)r.mask, (Global<int>)r.left, (Global<int>)r.right,
+                      (Global<int>)r.cnt, (Global<int>)r.pre, (Global<int>)r.n, (Global<int>)r.fixf,
+                      (Global<int>)r.winlist, r.wincount};
+}
+
 // Solves window w of the n knots of type ty (entries from e0 = knot 0) and
 // writes c of the rows it keeps; the window that keeps an end knot stores the
 // end values after the endpoint fix in fix[0..1].  Not-a-knot ends change
@@ -124,7 +141,7 @@ __device__ __forceinline__ real window_row(const real (&x)[B], int r)
 // partition_pcr that change nothing left out.
 template <typename real, bool NAK>
 __device__ __forceinline__ void solve_window(const KnotRows<real>& k, int e0, int ty, int n, int w,
-                                             int lane, real* fix, int* fixf)
+                                             int lane, real* fix, Global<int> fixf)
 {
     constexpr int B = Geom<real>::B, H = Geom<real>::H, W = kWave * B, K = W - 2 * H;
     const int g0 = w * K - H, lo = g0 - 1;
@@ -541,7 +558,7 @@ void k_stage(StageArgs<real> a)
                         }
                         if (REC && lane < 2) {
                             const int gt = (uni ? s * ntl : a.sd.tile0[s]) + t_first + tl;
-                            const StageRec& R = a.rec[j];
+                            const PassRecord R = record(a.rec, j);
                             R.pre[2 * gt + lane] = (lane ? before[1] - e1 : before[0]) - F;
                             R.cnt[2 * gt + lane] = lane ? rb[1] - before[1] : rb[0] - before[0];
                         }
@@ -551,31 +568,34 @@ void k_stage(StageArgs<real> a)
                         const int row = lane & 31;
                         const int gt = (uni ? s * ntl : a.sd.tile0[s]) + t_first + row / kWR;
                         if (row < nt * kWR)
-                            a.rec[j].mask[8 * (int64_t)gt + kWR * (lane >> 5) + row % kWR] = mk;
+                            record(a.rec, j).mask[8 * (int64_t)gt + kWR * (lane >> 5) + row % kWR] = mk;
                     }
                 }
                 __syncthreads();
                 // ---- windows of the spline system
                 const int wmx = (n[0] + K - 1) / K, wmn = (n[1] + K - 1) / K;
                 if (REC) {
-                    const StageRec R = a.rec[j];
+                    // by the last waves: the first ones have the windows (11 stages
+                    // of 3200 series of 16384 FP64 samples: 32.6 ms unrecorded,
+                    // recorded by the first waves 39.8, by the last 38.0)
+                    const PassRecord R = record(a.rec, j);
                     const int gt0 = uni ? s * ntl : a.sd.tile0[s];
                     if (threadIdx.x < 2) R.n[2 * s + threadIdx.x] = threadIdx.x ? n[1] : n[0];
-                    for (int q = threadIdx.x; q < 2 * ntl; q += NT) {
+                    for (int q = NT - 1 - threadIdx.x; q < 2 * ntl; q += NT) {
                         const int t = q >> 1, ty = q & 1, at = 2 * (gt0 + t) + ty;
                         const int pre = R.pre[at], nx = pre + R.cnt[at];
                         const int e0 = (ty ? e1 : 0) + F;
                         R.left[at] = pre > 0 ? (int)kr.p[e0 + pre - 1] : -1;
                         R.right[at] = nx < (ty ? n[1] : n[0]) ? (int)kr.p[e0 + nx] : -1;
                     }
-                    if (wv == 0) {
+                    if (wv == NWV - 1) {
                         unsigned wb = 0;
                         if (lane == 0) wb = atomicAdd(R.wincount, (unsigned)(wmx + wmn));
                         wb = (unsigned)__builtin_amdgcn_readfirstlane((int)wb);
                         for (int w = lane; w < wmx + wmn; w += kWave) {
                             const int ty = w >= wmx, wi = ty ? w - wmx : w;
                             const int g = max(wi * K - H - 1, 0);
-                            int* item = R.winlist + kWinItem * (int64_t)(wb + w);
+                            const Global<int> item = R.winlist + kWinItem * (int64_t)(wb + w);
                             item[0] = s;
                             item[1] = (wi << 1) | ty;
                             item[2] = (int)kr.p[(ty ? e1 : 0) + F + g] / kWT;   // tile of its first knot
@@ -585,7 +605,7 @@ void k_stage(StageArgs<real> a)
                 for (int w = wv; w < wmx + wmn; w += NWV) {
                     const int ty = w >= wmx, wi = ty ? w - wmx : w;
                     const int nty = ty ? n[1] : n[0];
-                    int* const fixf = REC ? a.rec[j].fixf + 4 * s + 2 * ty : nullptr;
+                    const Global<int> fixf = REC ? record(a.rec, j).fixf + 4 * s + 2 * ty : nullptr;
                     if (a.nak && nty >= 4)
                         solve_window<real, true>(kr, (ty ? e1 : 0) + F, ty, nty, wi, lane, s_fix[ty], fixf);
                     else
