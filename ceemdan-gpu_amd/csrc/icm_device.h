@@ -13,8 +13,6 @@ namespace icm {
 
 constexpr int kWave = 64;
 
-__device__ __forceinline__ int lane_id() { return __lane_id(); }
-
 // Index of this wavefront in its workgroup as a scalar value.  The compiler
 // cannot prove threadIdx.x >> 6 uniform over the wave; without this, every
 // per-wave quantity derived from it (work item, series, base pointers,
@@ -24,21 +22,12 @@ __device__ __forceinline__ int wave_index()
     return __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
 }
 
-// number of set bits of `mask` below this lane
-__device__ __forceinline__ int lanes_below(uint64_t mask)
-{
-    return __builtin_amdgcn_mbcnt_hi((uint32_t)(mask >> 32),
-                                     __builtin_amdgcn_mbcnt_lo((uint32_t)mask, 0u));
-}
-
 __device__ __forceinline__ uint64_t wave_ballot(bool p) { return __ballot(p); }
 
 template <typename T>
 __device__ __forceinline__ T shfl_up(T v, int d) { return __shfl_up(v, (unsigned)d, kWave); }
 template <typename T>
 __device__ __forceinline__ T shfl_down(T v, int d) { return __shfl_down(v, (unsigned)d, kWave); }
-template <typename T>
-__device__ __forceinline__ T shfl(T v, int src) { return __shfl(v, src, kWave); }
 
 // Whole-wave shifts by one lane (DPP wave_shr:1 / wave_shl:1): lane i gets
 // lane i-1 (shift_prev) or lane i+1 (shift_next); the lane with no source
@@ -74,28 +63,15 @@ __device__ __forceinline__ double shift_next(double v, double fill)
     return __longlong_as_double(((long long)hi << 32) | (unsigned)lo);
 }
 
-// Left and right neighbours of the samples of row v of a tile, where row p
-// (q) is the row before (after) it: lane i gets lane i-1 (i+1) of v, and
-// lane 0 (63) gets lane 63 (0) of p (q).  The other row's lane comes from a
-// whole-wave rotation by one lane (DPP wave_ror:1 / wave_rol:1), which is
-// then the fill of the shift: two moves, where a shift with a wave-uniform
-// fill takes a lane read, a move and the shift.
-__device__ __forceinline__ int dpp_rot_prev_i(int v) { return __builtin_amdgcn_mov_dpp(v, 0x13C, 0xF, 0xF, false); }
+// Right neighbours of the samples of row v of a tile, where row q is the row
+// after it: lane i gets lane i+1 of v, and lane 63 gets lane 0 of q.  The other
+// row's lane comes from a whole-wave rotation by one lane (DPP wave_rol:1),
+// which is then the fill of the shift: two moves, where a shift with a
+// wave-uniform fill takes a lane read, a move and the shift.
 __device__ __forceinline__ int dpp_rot_next_i(int v) { return __builtin_amdgcn_mov_dpp(v, 0x134, 0xF, 0xF, false); }
-__device__ __forceinline__ float row_prev(float v, float p)
-{
-    return __int_as_float(dpp_prev_i(__float_as_int(v), dpp_rot_prev_i(__float_as_int(p))));
-}
 __device__ __forceinline__ float row_next(float v, float q)
 {
     return __int_as_float(dpp_next_i(__float_as_int(v), dpp_rot_next_i(__float_as_int(q))));
-}
-__device__ __forceinline__ double row_prev(double v, double p)
-{
-    const long long b = __double_as_longlong(v), f = __double_as_longlong(p);
-    const int lo = dpp_prev_i((int)b, dpp_rot_prev_i((int)f));
-    const int hi = dpp_prev_i((int)(b >> 32), dpp_rot_prev_i((int)(f >> 32)));
-    return __longlong_as_double(((long long)hi << 32) | (unsigned)lo);
 }
 __device__ __forceinline__ double row_next(double v, double q)
 {
