@@ -974,11 +974,15 @@ struct Plan : PlanBase {
         L.epoch = 0;
         return ICM_OK;
     }
-    int reset_controls(hipStream_t st)
+    // A forward in one call knows its path (the stage kernel has no control
+    // words).  Between the calls of a staged forward the caller may set
+    // profiling, tuning or traces, which moves its later stages to the
+    // launches per step: both lanes start clear.
+    int reset_controls(hipStream_t st, bool staged)
     {
         int rc;
-        for (int ph = 0; ph < 2; ++ph)   // the stage kernel has no control words
-            if (!whole_stages(ph) && (rc = reset_control(ln[ph], st))) return rc;
+        for (int ph = 0; ph < 2; ++ph)
+            if ((staged || !whole_stages(ph)) && (rc = reset_control(ln[ph], st))) return rc;
         return ICM_OK;
     }
     static uint32_t next_epoch(Lane& L) { return ++L.epoch; }
@@ -1493,7 +1497,7 @@ struct Plan : PlanBase {
         ICM_TRY(launch_fill_u32((uint32_t*)err, 0u, 1, st));
         int rc;
         if ((rc = inputs_and_noise(sig, noise, st))) return rc;
-        if ((rc = reset_controls(st))) return rc;
+        if ((rc = reset_controls(st, false))) return rc;
         const bool both = overlap();
         const bool split = !(both && graph_on());   // phase times measured
         if (both) {
@@ -1570,7 +1574,7 @@ struct Plan : PlanBase {
         ICM_TRY(launch_fill_u32((uint32_t*)err, 0u, 1, st));
         int rc;
         if ((rc = inputs_and_noise(sig, noise, st))) return rc;
-        if ((rc = reset_controls(st))) return rc;
+        if ((rc = reset_controls(st, true))) return rc;
         if ((rc = noise_phase(st))) return rc;
         if ((rc = signal_begin(st))) return rc;
         if ((rc = sync_err(st))) return rc;
@@ -1694,7 +1698,7 @@ struct Plan : PlanBase {
         std::fill(krec_valid.begin(), krec_valid.end(), (char)0);
         ICM_TRY(launch_fill_u32((uint32_t*)err, 0u, 1, st));
         if ((rc = inputs_and_noise(nullptr, noise, st))) return rc;
-        if ((rc = reset_controls(st))) return rc;
+        if ((rc = reset_controls(st, true))) return rc;
         if ((rc = noise_phase(st))) return rc;
         if ((rc = signal_begin(st))) return rc;
         if ((rc = sync_err(st))) return rc;

@@ -1,0 +1,120 @@
+// Host code of the plan without a GPU (see fake_hip.cpp): one check per name
+// on the command line; prints "ok" for each that holds.
+#include "fake_hip.h"
+
+#include <cstdio>
+#include <cstdlib>
+#include <cstring>
+#include <string>
+#include <vector>
+
+#include "../../ceemdan-gpu_amd/csrc/icm_kernels.h"
+#include "../../include/iceemdan_mi355x.h"
+
+using namespace icm;
+
+#define CHECK(x)                                                    \
+    do {                                                            \
+        if (!(x)) {                                                 \
+            std::printf("line %d: %s\n", __LINE__, #x);             \
+            return false;                                           \
+        }                                                           \
+    } while (0)
+
+namespace {
+
+struct Call {
+    std::vector<int64_t> lens;
+    std::vector<std::vector<double>> in, out;   // large enough for either dtype
+    std::vector<void*> inp, outp;
+    icm_config c;
+    Call(std::vector<int64_t> l, int I, int M, int dtype, int stop = ICM_STOP_FIXED) : lens(std::move(l))
+    {
+        icm_config_default(&c);
+        c.dtype = dtype;
+        c.num_channels = (int)lens.size();
+        c.lengths = lens.data();
+        c.num_noise = I;
+        c.num_imfs = M;
+        c.stop_mode = stop;
+        c.use_graph = 0;
+        if (stop == ICM_STOP_RILLING) c.max_sifts = c.noise_max_sifts = 100;
+        for (int64_t n : lens) {
+            in.emplace_back(n, 1.0);
+            out.emplace_back(n * M, 0.0);
+        }
+        for (auto& v : in) inp.push_back(v.data());
+        for (auto& v : out) outp.push_back(v.data());
+    }
+};
+
+int g_prefixes, g_stages, g_dirty;
+
+bool is(const FakeLaunch& l, const char* kernel) { return std::strstr(l.name, kernel) != nullptr; }
+
+// counts the launches of either path; a knot prefix whose control words are
+// not clear is one that would write past the window list
+void watch(const FakeLaunch& l)
+{
+    if (is(l, "k_stage")) ++g_stages;
+    if (!is(l, "k_knot_prefix")) return;
+    ++g_prefixes;
+    const PassCtl pc = *(const PassCtl*)l.args[3];
+    if (*pc.wincount != 0u || pc.dense[pc.epoch] != 0u) ++g_dirty;
+}
+
+void reset_watch()
+{
+    g_prefixes = g_stages = g_dirty = 0;
+    fake_on_launch = watch;
+}
+
+// A staged forward that leaves the stage kernel between its calls.
+bool staged_switch()
+{
+    for (int dtype : {ICM_DTYPE_F32, ICM_DTYPE_F64})
+        for (int stop : {ICM_STOP_FIXED, ICM_STOP_RILLING})
+            for (int how = 0; how < 3; ++how)
+                for (int load = 0; load < 2; ++load) {
+                    Call k({1000, 300}, 3, 4, dtype, stop);
+                    icm_plan p = nullptr, q = nullptr;
+                    reset_watch();
+                    CHECK(icm_plan_create(&k.c, &p) == ICM_OK);
+                    CHECK(icm_forward_begin(p, k.inp.data(), nullptr, nullptr) == ICM_OK);
+                    if (load) {
+                        int64_t n = 0;
+                        CHECK(icm_state_bytes(p, &n) == ICM_OK);
+                        std::vector<char> state(n);
+                        CHECK(icm_state_save(p, state.data(), n, nullptr) == ICM_OK);
+                        CHECK(icm_plan_create(&k.c, &q) == ICM_OK);
+                        CHECK(icm_state_load(q, state.data(), n, nullptr, nullptr) == ICM_OK);
+                        std::swap(p, q);
+                    }
+                    CHECK(g_stages > 0 && g_prefixes == 0);
+                    const int32_t cand[3] = {0, 0, 0};
+                    if (how == 0) CHECK(icm_set_profiling(p, 1) == ICM_OK);
+                    if (how == 1) CHECK(icm_set_tuning(p, ICM_PHASE_SIGNAL, cand, 3) == ICM_OK);
+                    if (how == 2) CHECK(icm_set_trace(p, 2) == ICM_OK);
+                    CHECK(icm_forward_stages(p, 3, nullptr, nullptr) == ICM_OK);
+                    CHECK(g_prefixes > 0);
+                    CHECK(g_dirty == 0);
+                    CHECK(icm_forward_finish(p, k.outp.data(), nullptr) == ICM_OK);
+                    CHECK(icm_plan_destroy(p) == ICM_OK);
+                    if (q) CHECK(icm_plan_destroy(q) == ICM_OK);
+                    CHECK(fake_used_bytes == 0);
+                }
+    return true;
+}
+
+}  // namespace
+
+int main(int argc, char** argv)
+{
+    const struct { const char* name; bool (*run)(); } all[] = {
+        {"staged_switch", staged_switch},
+    };
+    for (int i = 1; i < argc; ++i)
+        for (const auto& t : all)
+            if (!std::strcmp(argv[i], t.name) && t.run()) std::printf("%s ok\n", t.name);
+    return 0;
+}

@@ -1,0 +1,45 @@
+"""Host code of the plans on the CPU: the library's entry points over a HIP
+runtime that allocates host memory and runs no kernel (tests/host), so that
+what is launched, cleared and allocated can be looked at where running it
+could fault a GPU."""
+import os
+import shutil
+import subprocess
+
+import pytest
+
+ROOT = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
+HOST = os.path.join(ROOT, "tests", "host")
+PKG = os.path.join(ROOT, "ceemdan-gpu_amd")
+ROCM = os.environ.get("ROCM_PATH", "/opt/rocm")
+
+
+@pytest.fixture(scope="module")
+def driver(icm, tmp_path_factory):
+    if not shutil.which("g++") or not os.path.isdir(os.path.join(ROCM, "include", "hip")):
+        pytest.skip("no host compiler or HIP headers")
+    icm.lib()   # says so if the library is not built
+    d = tmp_path_factory.mktemp("host")
+    flags = ["-O1", "-std=c++17", "-D__HIP_PLATFORM_AMD__", "-I", os.path.join(ROCM, "include"), "-w"]
+    fake, exe = d / "libfake_hip.so", d / "plan_driver"
+    subprocess.run(["g++", *flags, "-shared", "-fPIC", os.path.join(HOST, "fake_hip.cpp"), "-o",
+                    str(fake)], check=True)
+    # the fake runtime first: its definitions are the ones found
+    subprocess.run(["g++", *flags, os.path.join(HOST, "plan_driver.cpp"), "-o", str(exe),
+                    "-Wl,--no-as-needed", str(fake), f"-L{PKG}", "-liceemdan_mi355x",
+                    f"-Wl,-rpath,{d}:{PKG}:{ROCM}/lib", f"-Wl,-rpath-link,{ROCM}/lib"], check=True)
+
+    def run(name, **env):
+        base = {k: v for k, v in os.environ.items() if not k.startswith("ICM_")}
+        p = subprocess.run([str(exe), name], capture_output=True, text=True, timeout=300,
+                           env=dict(base, **env))
+        assert p.returncode == 0 and p.stdout == f"{name} ok\n", (p.returncode, p.stdout, p.stderr[-2000:])
+    return run
+
+
+def test_staged_forward_that_changes_path_has_clear_control_words(driver):
+    """icm_set_profiling, icm_set_tuning or icm_set_trace between
+    icm_forward_begin (or icm_state_load) and icm_forward_stages moves the
+    remaining stages from the stage kernel to the launches per step, whose
+    window lists are indexed by counters that must start at zero."""
+    driver("staged_switch")
