@@ -763,7 +763,9 @@ StageGeom stage_geometry(int real_size, int64_t max_len, int64_t nseries)
     const size_t most = 160 * 1024 - 2048;     // static arrays aside
     g.lds = std::min(worst, most);
     g.slot = worst <= most ? 0 : (worst + 255) / 256 * 256;
-    g.grid = g.slot ? std::min<int64_t>(nseries, 256) : nseries;   // one per CU
+    // with scratch one workgroup per CU; else one per series, up to a grid of
+    // at most 2^30 work-items (a workgroup goes on to the next series)
+    g.grid = std::min<int64_t>(nseries, g.slot ? 256 : 1 << 20);
     g.ok = true;
     return g;
 }

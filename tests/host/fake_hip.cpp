@@ -67,9 +67,11 @@ hipError_t __hipPopCallConfiguration(dim3* grid, dim3* block, size_t* lds, hipSt
 hipError_t hipLaunchKernel(const void* f, dim3 grid, dim3 block, void** args, size_t lds, hipStream_t)
 {
     const FakeLaunch l{kernels()[f].c_str(), grid, block, lds, args};
-    // limits of a launch: 2^32 - 1 work-items, 1024 per workgroup
-    const unsigned long long threads = (unsigned long long)block.x * block.y * block.z;
-    if (threads > 1024 || threads * grid.x * grid.y * grid.z > 0xFFFFFFFFull)
+    // limits of a launch: 1024 work-items per workgroup, 2^32 - 1 per dimension
+    const unsigned long long most = 0xFFFFFFFFull;
+    if ((unsigned long long)block.x * block.y * block.z > 1024 ||
+        (unsigned long long)grid.x * block.x > most || (unsigned long long)grid.y * block.y > most ||
+        (unsigned long long)grid.z * block.z > most)
         return hipErrorInvalidConfiguration;
     if (fake_on_launch) fake_on_launch(l);
     if (std::strstr(l.name, "k_fill_u32")) {

@@ -106,12 +106,29 @@ bool staged_switch()
     return true;
 }
 
+// Launch shapes of the stage kernel at the most series a phase may have (2^28
+// tiles): below 2^32 work-items, no scratch slot without a workgroup.
+bool stage_grid()
+{
+    for (int size : {4, 8})
+        for (int64_t ntl = 1; ntl <= 130; ++ntl)
+            for (int64_t nser : {(int64_t)1, (int64_t)257, ((int64_t)1 << 28) / ntl}) {
+                const StageGeom g = stage_geometry(size, 256 * ntl, nser);
+                if (!g.ok) continue;
+                CHECK(g.grid >= 1 && g.grid <= nser);
+                CHECK((uint64_t)g.grid * g.nwv * 64 <= 0xFFFFFFFFull);
+                CHECK(g.slot == 0 || g.slot * (uint64_t)g.grid <= (uint64_t)300 << 20);
+            }
+    return true;
+}
+
 }  // namespace
 
 int main(int argc, char** argv)
 {
     const struct { const char* name; bool (*run)(); } all[] = {
         {"staged_switch", staged_switch},
+        {"stage_grid", stage_grid},
     };
     for (int i = 1; i < argc; ++i)
         for (const auto& t : all)

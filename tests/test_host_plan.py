@@ -43,3 +43,8 @@ def test_staged_forward_that_changes_path_has_clear_control_words(driver):
     remaining stages from the stage kernel to the launches per step, whose
     window lists are indexed by counters that must start at zero."""
     driver("staged_switch")
+
+
+def test_stage_kernel_grid_fits_a_launch(driver):
+    """Plans of up to 2^28 tiles, of any length that the stage kernel takes."""
+    driver("stage_grid")
