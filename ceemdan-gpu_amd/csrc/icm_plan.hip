@@ -690,10 +690,32 @@ void layout(PlanBase& P)
     P.cap = T / 2 + 2;   // strict extrema are never adjacent, plus the two ends
 }
 
-int64_t plan_bytes_estimate(const icm_config* c)
+// Launch shape of the stage kernel for one phase (ok = false: launches per
+// step).  ICM_WHOLE_STAGES=0 turns it off.
+StageGeom stage_choice(const icm_config& c, int phase, const HostSeries& h)
 {
-    PlanBase* dummy = nullptr;
-    (void)dummy;
+    const char* env = std::getenv("ICM_WHOLE_STAGES");
+    if (env && std::atoi(env) == 0) return StageGeom{};
+    StageGeom g = stage_geometry(c.dtype == ICM_DTYPE_F64 ? 8 : 4, h.max_len, (int64_t)h.len.size());
+    // a stage of a few passes does not repay the allocation
+    const int passes = phase == ICM_PHASE_NOISE ? c.noise_max_sifts : c.max_sifts;
+    if (g.slot && passes < 4) g.ok = false;
+    return g;
+}
+
+// its scratch: an extra that a plan goes without where memory is short
+int64_t stage_scratch(const StageGeom& g) { return g.ok ? (int64_t)g.slot * g.grid : 0; }
+
+// ICM_MEMORY_BUDGET in bytes, -1 if there is none
+int64_t memory_budget()
+{
+    const char* env = std::getenv("ICM_MEMORY_BUDGET");
+    return env ? std::max<int64_t>(-1, std::atoll(env)) : -1;
+}
+
+// bytes that a plan cannot do without, and in *extra the stage kernel's scratch
+int64_t plan_bytes_estimate(const icm_config* c, int64_t* extra = nullptr)
+{
     struct Tmp : PlanBase {
         int forward(const void* const*, void* const*, const void*, hipStream_t) override { return 0; }
         int noise_modes_out(void*, int64_t, hipStream_t) override { return 0; }
@@ -730,6 +752,9 @@ int64_t plan_bytes_estimate(const icm_config* c)
         b += (int64_t)(M - 1) * c->max_sifts *
              ((int64_t)P.hsig.ntiles * (64 + 16 + 16) + 6 * (int64_t)P.hsig.len.size() * 4 +
               (int64_t)kWinItem * P.hsig.maxwin * 4);
+    if (extra)
+        *extra = stage_scratch(stage_choice(*c, ICM_PHASE_NOISE, P.hn)) +
+                 stage_scratch(stage_choice(*c, ICM_PHASE_SIGNAL, P.hsig));
     return b;
 }
 
@@ -880,23 +905,17 @@ struct Plan : PlanBase {
 
     // Launch shapes of the stage kernel, and its scratch where the knot rows
     // do not fit LDS.  The scratch is an extra: a plan that leaves little
-    // memory goes without (and keeps the launch-per-step path).
-    // ICM_WHOLE_STAGES=0 turns the stage kernel off.
+    // memory, or that it would take past ICM_MEMORY_BUDGET, goes without (and
+    // keeps the launch-per-step path).
     void setup_whole_stages()
     {
-        if (const char* env = std::getenv("ICM_WHOLE_STAGES"))
-            if (std::atoi(env) == 0) return;
+        const int64_t budget = memory_budget();
         for (int ph = 0; ph < 2; ++ph) {
-            const DevSeries& d = ph == ICM_PHASE_NOISE ? dn : dsig;
-            StageGeom g = stage_geometry((int)sizeof(real), d.max_len, d.nseries);
-            // a stage of a few passes does not repay the allocation
-            const int passes = ph == ICM_PHASE_NOISE ? cfg.noise_max_sifts : cfg.max_sifts;
-            if (g.slot && passes < 4) g.ok = false;
-            if (g.ok && g.slot) {
-                const int64_t need = (int64_t)g.slot * g.grid;
+            StageGeom g = stage_choice(cfg, ph, ph == ICM_PHASE_NOISE ? hn : hsig);
+            if (const int64_t need = stage_scratch(g)) {
                 size_t fr = 0, tot = 0;
-                if (hipMemGetInfo(&fr, &tot) != hipSuccess || need > (int64_t)fr / 16 ||
-                    hipMalloc((void**)&sscratch[ph], (size_t)need) != hipSuccess) {
+                if ((budget >= 0 && bytes + need > budget) || hipMemGetInfo(&fr, &tot) != hipSuccess ||
+                    need > (int64_t)fr / 16 || hipMalloc((void**)&sscratch[ph], (size_t)need) != hipSuccess) {
                     (void)hipGetLastError();
                     sscratch[ph] = nullptr;
                     g.ok = false;
@@ -1947,7 +1966,9 @@ int icm_plan_bytes(const icm_config* c, int64_t* bytes)
     int rc = validate(c);
     if (rc) return rc;
     if (!bytes) return ICM_ERR_INVALID_ARG;
-    *bytes = plan_bytes_estimate(c);
+    int64_t extra = 0;
+    *bytes = plan_bytes_estimate(c, &extra);
+    *bytes += extra;
     return ICM_OK;
 }
 
@@ -1960,11 +1981,9 @@ int icm_plan_create(const icm_config* c, icm_plan* out)
     // refuse a plan that cannot fit before allocating any of it: against
     // ICM_MEMORY_BUDGET (bytes) when set, else the device's free memory
     const int64_t need = plan_bytes_estimate(c);
-    int64_t budget = -1;
+    int64_t budget = memory_budget();
     const char* what = "budget";
-    if (const char* env = std::getenv("ICM_MEMORY_BUDGET")) {
-        budget = std::atoll(env);
-    } else {
+    if (!std::getenv("ICM_MEMORY_BUDGET")) {
         size_t fr = 0, tot = 0;
         if (hipMemGetInfo(&fr, &tot) == hipSuccess) {
             budget = (int64_t)fr;
@@ -2202,9 +2221,8 @@ int icm_sift_pass(int dtype, const void* d_h, int64_t N, int64_t I, void* d_h_ne
     const int rc = validate(&c);
     if (rc) return rc;
     // a set budget refuses what it refused when the pass ran in a plan
-    if (const char* env = std::getenv("ICM_MEMORY_BUDGET"))
-        if (std::atoll(env) >= 0 && plan_bytes_estimate(&c) > std::atoll(env))
-            return ICM_ERR_OUT_OF_MEMORY;
+    const int64_t budget = memory_budget();
+    if (budget >= 0 && plan_bytes_estimate(&c) > budget) return ICM_ERR_OUT_OF_MEMORY;
     return sift_uniform(dtype, d_h, N, I, d_h_new, d_nk, (hipStream_t)stream);
 }
 

@@ -100,6 +100,9 @@ const char* icm_last_error(void);
 /* Host-only checks (no device calls). */
 int icm_config_default(icm_config* cfg);
 int icm_validate_config(const icm_config* cfg);
+/* Device memory of a plan of this configuration, with the scratch of the
+ * whole-stage kernel (at most 256 x 1.1 MB per phase), which a plan goes
+ * without where it would not fit free memory or ICM_MEMORY_BUDGET. */
 int icm_plan_bytes(const icm_config* cfg, int64_t* bytes);
 
 /* Plan lifecycle.  A plan owns all scratch; it is reentrant across plans but

@@ -122,6 +122,44 @@ bool stage_grid()
     return true;
 }
 
+// A plan stays within what icm_plan_bytes says and within ICM_MEMORY_BUDGET
+// (but for its small tables, which the estimate leaves out), is refused where
+// it was, and has the stage kernel's scratch where that fits.
+bool budget()
+{
+    for (int dtype : {ICM_DTYPE_F32, ICM_DTYPE_F64})
+        for (int n : {3000, 20000, 32768})
+            for (int I : {20, 300}) {
+                Call k({n, n - 7}, I, 3, dtype);
+                setenv("ICM_WHOLE_STAGES", "0", 1);
+                int64_t least = 0, most = 0;
+                CHECK(icm_plan_bytes(&k.c, &least) == ICM_OK);
+                unsetenv("ICM_WHOLE_STAGES");
+                CHECK(icm_plan_bytes(&k.c, &most) == ICM_OK);
+                const int64_t tables = (128 << 10) + least / 500;
+                CHECK(n == 3000 ? most == least : most > least);
+                for (int64_t room : {least - 1, least, (least + most) / 2, most + tables}) {
+                    setenv("ICM_MEMORY_BUDGET", std::to_string(room).c_str(), 1);
+                    icm_plan p = nullptr;
+                    const int rc = icm_plan_create(&k.c, &p);
+                    unsetenv("ICM_MEMORY_BUDGET");
+                    CHECK(rc == (room < least ? ICM_ERR_OUT_OF_MEMORY : ICM_OK));
+                    if (rc) continue;
+                    CHECK(fake_used_bytes <= room + tables);
+                    icm_plan_info info;
+                    CHECK(icm_plan_get_info(p, &info) == ICM_OK);
+                    CHECK(info.device_bytes <= fake_used_bytes && info.device_bytes >= fake_used_bytes - tables);
+                    reset_watch();
+                    CHECK(icm_set_autotune(p, 0) == ICM_OK);
+                    CHECK(icm_forward(p, k.inp.data(), k.outp.data(), nullptr, nullptr) == ICM_OK);
+                    if (room > most) CHECK(g_stages > 0 && g_prefixes == 0);
+                    CHECK(icm_plan_destroy(p) == ICM_OK);
+                    CHECK(fake_used_bytes == 0);
+                }
+            }
+    return true;
+}
+
 }  // namespace
 
 int main(int argc, char** argv)
@@ -129,6 +167,7 @@ int main(int argc, char** argv)
     const struct { const char* name; bool (*run)(); } all[] = {
         {"staged_switch", staged_switch},
         {"stage_grid", stage_grid},
+        {"budget", budget},
     };
     for (int i = 1; i < argc; ++i)
         for (const auto& t : all)

@@ -48,3 +48,9 @@ def test_staged_forward_that_changes_path_has_clear_control_words(driver):
 def test_stage_kernel_grid_fits_a_launch(driver):
     """Plans of up to 2^28 tiles, of any length that the stage kernel takes."""
     driver("stage_grid")
+
+
+def test_plan_keeps_to_its_estimate_and_budget(driver):
+    """The stage kernel's scratch is in icm_plan_bytes and within
+    ICM_MEMORY_BUDGET; a budget that holds the rest of the plan is enough."""
+    driver("budget")
