@@ -534,7 +534,11 @@ struct PlanBase {
             if (!q.src.empty()) staged += up(q.bytes);
         }
         char* base = nullptr;
-        if (total && hipMalloc((void**)&base, total) != hipSuccess) return ICM_ERR_OUT_OF_MEMORY;
+        if (total && hipMalloc((void**)&base, total) != hipSuccess) {
+            for (const Piece& q : batch) bytes -= (int64_t)q.bytes;   // counted when noted
+            batch.clear();
+            return ICM_ERR_OUT_OF_MEMORY;
+        }
         if (base) allocs.push_back(base);
         std::vector<char> host(staged);
         size_t at[2] = {staged, 0};      // without and with a source: those first

@@ -160,6 +160,33 @@ bool budget()
     return true;
 }
 
+int64_t device_bytes(icm_plan p)
+{
+    icm_plan_info info;
+    return icm_plan_get_info(p, &info) == ICM_OK ? info.device_bytes : -1;
+}
+
+// A backward whose buffers fit only in place of the stage kernel's scratch
+// takes them there and counts them once.
+bool backward_room()
+{
+    Call k({32768}, 40, 3, ICM_DTYPE_F64);
+    for (int round = 0; round < 2; ++round) {
+        icm_plan p = nullptr;
+        CHECK(icm_plan_create(&k.c, &p) == ICM_OK);
+        CHECK(icm_forward(p, k.inp.data(), k.outp.data(), nullptr, nullptr) == ICM_OK);
+        if (round) fake_free_bytes = fake_used_bytes + (30 << 20);
+        const int rc = icm_backward(p, k.outp.data(), k.inp.data(), nullptr);
+        fake_free_bytes = (long long)1 << 40;
+        CHECK(rc == ICM_OK);
+        // (pieces of an allocation begin at multiples of 256 bytes)
+        CHECK(device_bytes(p) <= fake_used_bytes && device_bytes(p) >= fake_used_bytes - (64 << 10));
+        CHECK(icm_plan_destroy(p) == ICM_OK);
+        CHECK(fake_used_bytes == 0);
+    }
+    return true;
+}
+
 }  // namespace
 
 int main(int argc, char** argv)
@@ -168,6 +195,7 @@ int main(int argc, char** argv)
         {"staged_switch", staged_switch},
         {"stage_grid", stage_grid},
         {"budget", budget},
+        {"backward_room", backward_room},
     };
     for (int i = 1; i < argc; ++i)
         for (const auto& t : all)

@@ -54,3 +54,7 @@ def test_plan_keeps_to_its_estimate_and_budget(driver):
     """The stage kernel's scratch is in icm_plan_bytes and within
     ICM_MEMORY_BUDGET; a budget that holds the rest of the plan is enough."""
     driver("budget")
+
+
+def test_backward_buffers_in_place_of_scratch_are_counted_once(driver):
+    driver("backward_room")
