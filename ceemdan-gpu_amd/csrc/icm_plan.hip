@@ -507,6 +507,18 @@ struct PlanBase {
     virtual int state_save(void* host, int64_t bytes, hipStream_t st) = 0;
     virtual int state_load(const void* host, int64_t bytes, const void* noise, hipStream_t st) = 0;
 
+    // Device memory; where it is short the stage kernel's scratch makes room.
+    bool take(void** p, size_t n)
+    {
+        if (hipMalloc(p, n) == hipSuccess) return true;
+        (void)hipGetLastError();
+        if (!sscratch[0] && !sscratch[1]) return false;
+        drop_stage_scratch();
+        drop_graphs();
+        if (hipMalloc(p, n) == hipSuccess) return true;
+        (void)hipGetLastError();
+        return false;
+    }
     // Device memory is taken in batches: alloc and upload between
     // batch_begin and batch_commit only note what is wanted; the commit makes
     // one allocation, sets the pointers (which must live until then) and
@@ -534,7 +546,7 @@ struct PlanBase {
             if (!q.src.empty()) staged += up(q.bytes);
         }
         char* base = nullptr;
-        if (total && hipMalloc((void**)&base, total) != hipSuccess) {
+        if (total && !take((void**)&base, total)) {
             for (const Piece& q : batch) bytes -= (int64_t)q.bytes;   // counted when noted
             batch.clear();
             return ICM_ERR_OUT_OF_MEMORY;
@@ -564,7 +576,7 @@ struct PlanBase {
             return ICM_OK;
         }
         void* q = nullptr;
-        if (hipMalloc(&q, (size_t)n * sizeof(T)) != hipSuccess) {
+        if (!take(&q, (size_t)n * sizeof(T))) {
             bytes -= n * (int64_t)sizeof(T);
             return ICM_ERR_OUT_OF_MEMORY;
         }
@@ -876,7 +888,7 @@ struct Plan : PlanBase {
         }
         batch_begin();
         for (size_t k = 0; k < krec.size(); ++k)
-            if ((rc = upload_recs(krec[k], &krec_dev[k]))) return rc;
+            if ((rc = upload(&krec_dev[k], record_table(krec[k])))) return rc;
         if ((rc = batch_commit())) return rc;
         // pinned words read by the host: two counts and the error word
         if (hipHostMalloc((void**)&h_n_active, 3 * sizeof(unsigned), hipHostMallocDefault) !=
@@ -1751,8 +1763,8 @@ struct Plan : PlanBase {
         }
         return ICM_OK;
     }
-    // their device table, once they are allocated (in a batch)
-    int upload_recs(std::vector<Rec>& rr, StageRec** table)
+    // their device table, once they are allocated
+    std::vector<StageRec> record_table(std::vector<Rec>& rr)
     {
         std::vector<StageRec> dev;
         for (size_t j = 0; j < rr.size(); ++j) {
@@ -1760,29 +1772,21 @@ struct Plan : PlanBase {
             dev.push_back(StageRec{rr[j].mask, rr[j].left, rr[j].right, rr[j].cnt, rr[j].pre,
                                    rr[j].n, rr[j].fixf, rr[j].winlist, rr[j].wincount});
         }
-        return upload(table, dev);
+        return dev;
     }
 
-    int backward_alloc()
-    {
-        int rc = backward_buffers();
-        if (rc == ICM_ERR_OUT_OF_MEMORY && (sscratch[0] || sscratch[1])) {
-            // the stage kernel's scratch makes room
-            (void)hipGetLastError();
-            drop_stage_scratch();
-            drop_graphs();
-            rc = backward_buffers();
-        }
-        return rc;
-    }
     int alloc_rec()
     {
-        int rc;
         std::vector<Rec> rr;
+        StageRec* table = nullptr;
+        int rc;
         batch_begin();
-        if ((rc = alloc_recs(rr)) || (rc = batch_commit())) return rc;
-        batch_begin();
-        if ((rc = upload_recs(rr, &rec_dev)) || (rc = batch_commit())) return rc;
+        if ((rc = alloc_recs(rr)) || (rc = alloc(&table, cfg.max_sifts)) || (rc = batch_commit()))
+            return rc;
+        const std::vector<StageRec> dev = record_table(rr);
+        if (hipMemcpy(table, dev.data(), dev.size() * sizeof(StageRec), hipMemcpyHostToDevice) != hipSuccess)
+            return ICM_ERR_HIP;
+        rec_dev = table;
         rec.swap(rr);
         return ICM_OK;
     }
@@ -1813,7 +1817,7 @@ struct Plan : PlanBase {
         const int C = cfg.num_channels, M = cfg.num_imfs, I = cfg.num_noise, S = cfg.max_sifts;
         const real eps0 = (real)cfg.noise_strength;
         int rc;
-        if ((rc = backward_alloc())) return rc;
+        if ((rc = backward_buffers())) return rc;
         *h_err = 0;
         ICM_TRY(hipEventRecord(ev[0], st));
         ICM_TRY(launch_fill_u32((uint32_t*)err, 0u, 1, st));

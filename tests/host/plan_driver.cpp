@@ -187,6 +187,60 @@ bool backward_room()
     return true;
 }
 
+// The same for traces.
+bool trace_room()
+{
+    Call k({32768}, 40, 3, ICM_DTYPE_F64);
+    icm_plan p = nullptr;
+    CHECK(icm_plan_create(&k.c, &p) == ICM_OK);
+    fake_free_bytes = fake_used_bytes + 1000;
+    const int rc = icm_set_trace(p, 10);
+    fake_free_bytes = (long long)1 << 40;
+    CHECK(rc == ICM_OK);
+    CHECK(device_bytes(p) <= fake_used_bytes && device_bytes(p) >= fake_used_bytes - (64 << 10));
+    CHECK(icm_plan_destroy(p) == ICM_OK);
+    CHECK(fake_used_bytes == 0);
+    return true;
+}
+
+// The same for the records of a backward that sifts again: with room for the
+// backward's buffers and not for the records, and for the records and not for
+// their device table; then once more, with what it has.
+bool record_room()
+{
+    Call k({32768}, 40, 3, ICM_DTYPE_F64);
+    int64_t buffers = 0, records = 0;
+    for (int keep = 1; keep >= 0; --keep) {
+        icm_plan p = nullptr;
+        k.c.keep_records = keep;   // with kept records the backward takes its buffers only
+        CHECK(icm_plan_create(&k.c, &p) == ICM_OK);
+        CHECK(icm_forward(p, k.inp.data(), k.outp.data(), nullptr, nullptr) == ICM_OK);
+        const long long before = fake_used_bytes;
+        CHECK(icm_backward(p, k.outp.data(), k.inp.data(), nullptr) == ICM_OK);
+        (keep ? buffers : records) = fake_used_bytes - before - (keep ? 0 : buffers);
+        CHECK(icm_plan_destroy(p) == ICM_OK);
+    }
+    CHECK(buffers > 0 && records > 1 << 20);
+    for (int64_t room : {buffers + 4096, buffers + records - 256}) {
+        icm_plan p = nullptr;
+        CHECK(icm_plan_create(&k.c, &p) == ICM_OK);
+        CHECK(icm_forward(p, k.inp.data(), k.outp.data(), nullptr, nullptr) == ICM_OK);
+        fake_free_bytes = fake_used_bytes + room;
+        reset_watch();
+        for (int n = 0; n < 2; ++n) {
+            const int rc = icm_backward(p, k.outp.data(), k.inp.data(), nullptr);
+            if (rc != ICM_OK) fake_free_bytes = (long long)1 << 40;
+            CHECK(rc == ICM_OK);
+        }
+        CHECK(g_prefixes > 0 && g_dirty == 0);   // without scratch: launches per step
+        fake_free_bytes = (long long)1 << 40;
+        CHECK(device_bytes(p) <= fake_used_bytes && device_bytes(p) >= fake_used_bytes - (64 << 10));
+        CHECK(icm_plan_destroy(p) == ICM_OK);
+        CHECK(fake_used_bytes == 0);
+    }
+    return true;
+}
+
 }  // namespace
 
 int main(int argc, char** argv)
@@ -196,6 +250,8 @@ int main(int argc, char** argv)
         {"stage_grid", stage_grid},
         {"budget", budget},
         {"backward_room", backward_room},
+        {"record_room", record_room},
+        {"trace_room", trace_room},
     };
     for (int i = 1; i < argc; ++i)
         for (const auto& t : all)

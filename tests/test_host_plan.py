@@ -58,3 +58,10 @@ def test_plan_keeps_to_its_estimate_and_budget(driver):
 
 def test_backward_buffers_in_place_of_scratch_are_counted_once(driver):
     driver("backward_room")
+
+
+@pytest.mark.parametrize("what", ["record_room", "trace_room"])
+def test_records_and_traces_in_place_of_scratch(driver, what):
+    """The records of a backward that sifts again, and traces, where memory
+    holds them only without the stage kernel's scratch."""
+    driver(what)
