@@ -265,13 +265,13 @@ struct PlanBase {
     // whole stages of short series, one workgroup per series
     StageGeom sgeom[2] = {};
     char* sscratch[2] = {nullptr, nullptr};
-    bool geometry_set = false;        // icm_set_tuning chose the sift geometry
+    bool geometry_set[2] = {};        // icm_set_tuning chose a phase's sift geometry
     // The stage kernel runs unless a caller asks for what only the
     // launch-per-step path has: sift geometries being timed or set, traces,
     // per-kernel times.
     bool whole_stages(int phase) const
     {
-        return sgeom[phase].ok && !tuning && !geometry_set && !trace_passes && !prof;
+        return sgeom[phase].ok && !tuning && !geometry_set[phase] && !trace_passes && !prof;
     }
     int* h_err = nullptr;             // pinned
     // rilling
@@ -437,7 +437,7 @@ struct PlanBase {
         }
         tune_left = forwards;
         tune_round = 0;
-        geometry_set = false;
+        geometry_set[0] = geometry_set[1] = false;
         drop_graphs();
         return ICM_OK;
     }
@@ -454,8 +454,12 @@ struct PlanBase {
             return ICM_ERR_INVALID_ARG;
         for (int64_t k = 0; k < count; ++k)
             if (in[k] < -1 || in[k] >= kNCand) return ICM_ERR_INVALID_ARG;
-        for (int64_t k = 0; k < count; ++k) choice[phase][k] = in[k];
-        geometry_set = true;
+        // (all -1 is the default, which is no choice)
+        geometry_set[phase] = false;
+        for (int64_t k = 0; k < count; ++k) {
+            choice[phase][k] = in[k];
+            geometry_set[phase] |= in[k] >= 0;
+        }
         tune_left = 0;
         drop_graphs();
         return ICM_OK;

@@ -141,9 +141,10 @@ int icm_set_overlap(icm_plan plan, int on);
 int icm_get_graph_status(icm_plan plan, int* status);
 
 /* Per-kernel timing with HIP events on the forward's stream (disables the
- * hipGraph replay while on).  kind: 0 = stage init (extrema of the stage
- * input), 1 = spline solve, 2 = sift pass.  Totals of the last forward;
- * alg_bytes = algorithmic bytes (2 * sizeof(real) per sample per launch). */
+ * hipGraph replay while on, and moves stages of short series that run whole
+ * in one kernel to the launches that are timed here).  kind: 0 = stage init
+ * (extrema of the stage input), 1 = spline solve, 2 = sift pass.  Totals of
+ * the last forward; alg_bytes = algorithmic bytes (2 * sizeof(real) per sample per launch). */
 #define ICM_KERNEL_INIT 0
 #define ICM_KERNEL_SOLVE 1
 #define ICM_KERNEL_SIFT 2
@@ -170,14 +171,19 @@ int icm_set_autotune(icm_plan plan, int forwards);
 int icm_get_tuning_left(icm_plan plan, int* forwards);
 /* Candidate per stage of a phase (host_out[k], k < M-1; -1 = default). */
 int icm_get_tuning(icm_plan plan, int phase, int32_t* host_out, int64_t count);
-/* Sets every stage's candidate (-1 .. 7; count = M-1) and ends tuning. */
+/* Sets every stage's candidate (-1 .. 7; count = M-1) and ends tuning.  A
+ * phase of short series whose stages run whole in one kernel (no sift
+ * launches, and nothing to tune: such a plan reports -1) takes launches per
+ * step while any of its candidates is >= 0, and while candidates are timed;
+ * all -1 (or icm_set_autotune(plan, 0)) is the default again. */
 int icm_set_tuning(icm_plan plan, int phase, const int32_t* host_in, int64_t count);
 /* Meaning of candidate `cand`: tiles per segment (0 = default) and small
  * knot tables (1), full tables (0) or the default rule (-1). */
 int icm_tuning_candidate(int cand, int* segment_tiles, int* small_tables);
 
 /* Per-pass knot counts (debug/parity): enable before a forward with the
- * number of passes to keep per stage; read back [M-1][passes][series][2]
+ * number of passes to keep per stage (traced forwards launch step by step,
+ * those of short series too); read back [M-1][passes][series][2]
  * (n_max, n_min of each pass input) of a phase. */
 int icm_set_trace(icm_plan plan, int passes);
 int icm_get_trace(icm_plan plan, int phase, int32_t* host_out, int64_t count);

@@ -65,3 +65,7 @@ def test_records_and_traces_in_place_of_scratch(driver, what):
     """The records of a backward that sifts again, and traces, where memory
     holds them only without the stage kernel's scratch."""
     driver(what)
+
+
+def test_default_tuning_given_back_keeps_the_stage_kernel(driver):
+    driver("tuning_round_trip")
