@@ -239,9 +239,10 @@ struct StageArgs {
 
 // Launch shape of a phase: waves per workgroup, one tile per wave or more,
 // workgroups, their LDS, and the scratch of each for passes whose knot rows
-// do not fit it.  ok = false: the series are too long.
+// do not fit it.  ok = false: the series are too long, or too few for their
+// length (few).
 struct StageGeom {
-    bool ok, hold;
+    bool ok, few, hold;
     int nwv;
     size_t lds, slot;
     int64_t grid;

@@ -422,8 +422,8 @@ struct PlanBase {
         tune_left = n;
         if (n > 0 && tune_table_get(tkey[0], choice[0]) && tune_table_get(tkey[1], choice[1]))
             tune_left = 0;
-        else if (sgeom[0].ok && sgeom[1].ok)
-            tune_left = 0;   // nothing to choose: no sift launches
+        else if ((sgeom[0].ok || sgeom[0].few) && (sgeom[1].ok || sgeom[1].few))
+            tune_left = 0;   // no sift launches, or ones too small to tell candidates apart
         else if (tune_left > 0)
             for (int ph = 0; ph < 2; ++ph) choice[ph].assign(M - 1, -1);
     }
@@ -710,8 +710,33 @@ void layout(PlanBase& P)
     P.cap = T / 2 + 2;   // strict extrema are never adjacent, plus the two ends
 }
 
+// Series that a workgroup each takes longer for than launches per step that
+// spread one pass over the chip: long FP64 ones, while they are few.  A
+// decomposition of one channel, M = 6, in ms, launches (default geometry) /
+// stage kernel, both phases side by side where FIXED:
+//   FIXED, 10 sifts    series  16          32          48          64          80
+//     26000 samples        2.42/2.70   2.68/2.84   3.05/2.94   3.35/2.97   3.54/3.01
+//     28000                2.61/2.91   2.86/3.05   3.12/3.10   3.39/3.14   3.73/3.20
+//     30000                2.60/3.08   2.89/3.25   3.22/3.37   3.47/3.40   3.89/3.46
+//     32768                2.65/3.41   2.95/3.61   3.30/3.68   3.62/3.72   4.01/3.77
+//   RILLING, caps 100 and 2000, 16, 40 and 80 series
+//     26000                39.6/36.6   44.1/40.8   51.7/44.8
+//     28000                37.3/38.2   44.1/42.9   51.5/47.6
+//     30000                44.0/45.9   52.5/52.9   59.8/57.1
+//     32768                48.1/54.6   59.8/66.9   70.2/73.4
+// (another run had the launches at 16 series up to 0.3 ms slower: the line
+// keeps to the stage kernel where the two runs disagree.)  Up to 98 tiles the
+// stage kernel is not behind at any number, nor in FP32 at any length it takes
+// (4 series of 32768: 2.43 / 2.02).
+bool few_long_series(const icm_config& c, const HostSeries& h)
+{
+    if (c.dtype != ICM_DTYPE_F64) return false;
+    const int64_t ntl = (h.max_len + tile_of(c.dtype) - 1) / tile_of(c.dtype), n = (int64_t)h.len.size();
+    return c.stop_mode == ICM_STOP_FIXED ? n < std::min<int64_t>(3 * (ntl - 98), 72) : n < 4 * (ntl - 103);
+}
+
 // Launch shape of the stage kernel for one phase (ok = false: launches per
-// step).  ICM_WHOLE_STAGES=0 turns it off.
+// step).  ICM_WHOLE_STAGES=0 turns it off, 1 takes it for few long series too.
 StageGeom stage_choice(const icm_config& c, int phase, const HostSeries& h)
 {
     const char* env = std::getenv("ICM_WHOLE_STAGES");
@@ -720,6 +745,10 @@ StageGeom stage_choice(const icm_config& c, int phase, const HostSeries& h)
     // a stage of a few passes does not repay the allocation
     const int passes = phase == ICM_PHASE_NOISE ? c.noise_max_sifts : c.max_sifts;
     if (g.slot && passes < 4) g.ok = false;
+    if (g.ok && !env && few_long_series(c, h)) {
+        g.ok = false;
+        g.few = true;
+    }
     return g;
 }
 

@@ -134,7 +134,7 @@ bool budget()
                 setenv("ICM_WHOLE_STAGES", "0", 1);
                 int64_t least = 0, most = 0;
                 CHECK(icm_plan_bytes(&k.c, &least) == ICM_OK);
-                unsetenv("ICM_WHOLE_STAGES");
+                setenv("ICM_WHOLE_STAGES", "1", 1);
                 CHECK(icm_plan_bytes(&k.c, &most) == ICM_OK);
                 const int64_t tables = (128 << 10) + least / 500;
                 CHECK(n == 3000 ? most == least : most > least);
@@ -268,6 +268,33 @@ bool tuning_round_trip()
     return true;
 }
 
+// Which path a plan takes by its series' length and number.
+bool few_series()
+{
+    const struct { int dtype, stop, n, I; bool whole; } t[] = {
+        {ICM_DTYPE_F64, ICM_STOP_FIXED, 32768, 4, false},  {ICM_DTYPE_F64, ICM_STOP_FIXED, 32768, 71, false},
+        {ICM_DTYPE_F64, ICM_STOP_FIXED, 32768, 72, true},  {ICM_DTYPE_F64, ICM_STOP_FIXED, 28160, 35, false},
+        {ICM_DTYPE_F64, ICM_STOP_FIXED, 28160, 36, true},  {ICM_DTYPE_F64, ICM_STOP_FIXED, 25088, 1, true},
+        {ICM_DTYPE_F64, ICM_STOP_RILLING, 32768, 99, false}, {ICM_DTYPE_F64, ICM_STOP_RILLING, 32768, 100, true},
+        {ICM_DTYPE_F64, ICM_STOP_RILLING, 26368, 1, true}, {ICM_DTYPE_F32, ICM_STOP_FIXED, 32768, 1, true},
+        {ICM_DTYPE_F32, ICM_STOP_RILLING, 32768, 1, true}, {ICM_DTYPE_F64, ICM_STOP_FIXED, 1000, 1, true},
+    };
+    for (const auto& q : t) {
+        Call k({q.n}, q.I, 2, q.dtype, q.stop);
+        icm_plan p = nullptr;
+        CHECK(icm_plan_create(&k.c, &p) == ICM_OK);
+        int left = -1;
+        CHECK(icm_get_tuning_left(p, &left) == ICM_OK && left == 0);
+        reset_watch();
+        CHECK(icm_forward(p, k.inp.data(), k.outp.data(), nullptr, nullptr) == ICM_OK);
+        if ((g_stages > 0) != q.whole || (g_prefixes > 0) == q.whole)
+            std::printf("dtype %d stop %d %d x %d\n", q.dtype, q.stop, q.I, q.n);
+        CHECK((g_stages > 0) == q.whole && (g_prefixes > 0) != q.whole);
+        CHECK(icm_plan_destroy(p) == ICM_OK);
+    }
+    return true;
+}
+
 }  // namespace
 
 int main(int argc, char** argv)
@@ -280,6 +307,7 @@ int main(int argc, char** argv)
         {"record_room", record_room},
         {"trace_room", trace_room},
         {"tuning_round_trip", tuning_round_trip},
+        {"few_series", few_series},
     };
     for (int i = 1; i < argc; ++i)
         for (const auto& t : all)

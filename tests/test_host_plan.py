@@ -57,15 +57,21 @@ def test_plan_keeps_to_its_estimate_and_budget(driver):
 
 
 def test_backward_buffers_in_place_of_scratch_are_counted_once(driver):
-    driver("backward_room")
+    driver("backward_room", ICM_WHOLE_STAGES="1")
 
 
 @pytest.mark.parametrize("what", ["record_room", "trace_room"])
 def test_records_and_traces_in_place_of_scratch(driver, what):
     """The records of a backward that sifts again, and traces, where memory
     holds them only without the stage kernel's scratch."""
-    driver(what)
+    driver(what, ICM_WHOLE_STAGES="1")
 
 
 def test_default_tuning_given_back_keeps_the_stage_kernel(driver):
     driver("tuning_round_trip")
+
+
+def test_few_long_series_launch_step_by_step(driver):
+    """FP64 series of about 100 to 128 tiles, too few to fill the chip with a
+    workgroup each; nothing is tuned on either path."""
+    driver("few_series")
