@@ -284,7 +284,7 @@ hipError_t launch_series_var(const real* base, const int64_t* off, int64_t strid
 template <typename real>
 hipError_t launch_noise(uint64_t seed, int I, int64_t N, real* out, hipStream_t st);
 template <typename real>
-hipError_t launch_noise_groups(uint64_t seed, int I, int ngroups, int64_t max_len, const int* len,
+hipError_t launch_noise_groups(uint64_t seed, int I, int ngroups, const int64_t* host_len, const int* len,
                                const int64_t* row_off, real* out, hipStream_t st);
 
 // r_{k+1} and IMF_k of every channel from the stage's realizations

