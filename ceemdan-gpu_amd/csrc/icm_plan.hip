@@ -727,11 +727,13 @@ void layout(PlanBase& P)
 // (another run had the launches at 16 series up to 0.3 ms slower: the line
 // keeps to the stage kernel where the two runs disagree.)  Up to 98 tiles the
 // stage kernel is not behind at any number, nor in FP32 at any length it takes
-// (4 series of 32768: 2.43 / 2.02).
+// (4 series of 32768: 2.43 / 2.02).  Series of other lengths in the plan count
+// by their tiles: 20 of 32768 and 400 of 300 samples 2.75 / 3.22, 400 of 3000
+// 3.04 / 3.30.
 bool few_long_series(const icm_config& c, const HostSeries& h)
 {
     if (c.dtype != ICM_DTYPE_F64) return false;
-    const int64_t ntl = (h.max_len + tile_of(c.dtype) - 1) / tile_of(c.dtype), n = (int64_t)h.len.size();
+    const int64_t ntl = (h.max_len + tile_of(c.dtype) - 1) / tile_of(c.dtype), n = (h.ntiles + ntl - 1) / ntl;
     return c.stop_mode == ICM_STOP_FIXED ? n < std::min<int64_t>(3 * (ntl - 98), 72) : n < 4 * (ntl - 103);
 }
 

@@ -271,16 +271,21 @@ bool tuning_round_trip()
 // Which path a plan takes by its series' length and number.
 bool few_series()
 {
-    const struct { int dtype, stop, n, I; bool whole; } t[] = {
+    // (`more` channels of 300 samples beside the one)
+    const struct { int dtype, stop, n, I; bool whole; int more; } t[] = {
         {ICM_DTYPE_F64, ICM_STOP_FIXED, 32768, 4, false},  {ICM_DTYPE_F64, ICM_STOP_FIXED, 32768, 71, false},
         {ICM_DTYPE_F64, ICM_STOP_FIXED, 32768, 72, true},  {ICM_DTYPE_F64, ICM_STOP_FIXED, 28160, 35, false},
         {ICM_DTYPE_F64, ICM_STOP_FIXED, 28160, 36, true},  {ICM_DTYPE_F64, ICM_STOP_FIXED, 25088, 1, true},
         {ICM_DTYPE_F64, ICM_STOP_RILLING, 32768, 99, false}, {ICM_DTYPE_F64, ICM_STOP_RILLING, 32768, 100, true},
         {ICM_DTYPE_F64, ICM_STOP_RILLING, 26368, 1, true}, {ICM_DTYPE_F32, ICM_STOP_FIXED, 32768, 1, true},
         {ICM_DTYPE_F32, ICM_STOP_RILLING, 32768, 1, true}, {ICM_DTYPE_F64, ICM_STOP_FIXED, 1000, 1, true},
+        {ICM_DTYPE_F64, ICM_STOP_FIXED, 32768, 20, false, 20}, {ICM_DTYPE_F64, ICM_STOP_FIXED, 32768, 70, true, 9},
+        {ICM_DTYPE_F32, ICM_STOP_FIXED, 32768, 20, true, 20},
     };
     for (const auto& q : t) {
-        Call k({q.n}, q.I, 2, q.dtype, q.stop);
+        std::vector<int64_t> lens(1 + q.more, 300);
+        lens[0] = q.n;
+        Call k(lens, q.I, 2, q.dtype, q.stop);
         icm_plan p = nullptr;
         CHECK(icm_plan_create(&k.c, &p) == ICM_OK);
         int left = -1;
