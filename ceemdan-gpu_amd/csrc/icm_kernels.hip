@@ -920,7 +920,7 @@ __global__ __launch_bounds__(kThreads) void k_solve(SolveArgs<real> a)
             }
         }
         real xs[B];
-        partition_pcr<real, B>(
+        partition_pcr<real, B, !NAK>(
             lane,
             [&](int q, real& dl, real& d, real& du, real& f) {
                 spline_row<real, NAK>(n, g0 + rb + q, hx[q], hx[q + 1], sl[q], sl[q + 1], dl, d, du,
@@ -2255,7 +2255,7 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(3))) v
             vr_prev = vr;
         }
         real xs[B];
-        partition_pcr<real, B>(
+        partition_pcr<real, B, true>(
             lane,
             [&](int q, real& dl, real& d, real& du, real& f) {
                 const long g = gb + q;

@@ -203,7 +203,7 @@ __device__ __forceinline__ void solve_window(const KnotRows<real>& k, int e0, in
         l2 = lane_value(oo, 1);
     }
     real xs[B];
-    partition_pcr<real, B>(
+    partition_pcr<real, B, !NAK>(
         lane,
         [&](int q, real& dl, real& d, real& du, real& f) {
             const int g = g0 + rb + q;

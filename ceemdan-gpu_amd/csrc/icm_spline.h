@@ -183,7 +183,9 @@ __device__ __forceinline__ real pivot_inv(real x)
     }
 }
 
-template <typename real, int B, class RowFn>
+// SYM: row g couples to row g + 1 as that to row g, or one of them not at all
+// (true but for not-a-knot ends)
+template <typename real, int B, bool SYM, class RowFn>
 __device__ __forceinline__ void partition_pcr(int lane, RowFn row, real (&x)[B])
 {
     real cp[B], al[B], be[B], ga[B];
@@ -225,11 +227,14 @@ __device__ __forceinline__ void partition_pcr(int lane, RowFn row, real (&x)[B])
     real D = (d + dl * ga[B - 2]) + du * nb0;
     real C = du * ng0;
     real R = (f - dl * al[B - 2]) - du * na0;
-    // one reduction by st lanes; false if it changed no D and no R.  Then no
-    // later one does: with k1(l) = A(l) / D(l - st), unchanged means
-    // |R(l - st) k1(l)| <= ulp / 2 of R(l) for every l, and the next level's
-    // factor is k1(l - st) k1(l), so its products are smaller by another
+    // one reduction by st lanes; false if neither of its two terms changed any
+    // D or R.  Then no later one does: with k1(l) = A(l) / D(l - st), unchanged
+    // means |R(l - st) k1(l)| <= ulp / 2 of R(l) for every l, and the next
+    // level's factor is k1(l - st) k1(l), so its products are smaller by another
     // factor of the unit roundoff (the same for D; a NaN counts as changed).
+    // They are compared after each term, as two terms that cancel each other
+    // need not be small; D only where that can happen: in a symmetric system
+    // A(l) C(l - st) is a square or zero, and both terms reduce D.
     // Interfaces eight rows apart are coupled by about 0.27^8, so two or three
     // of the six levels do anything and one more shows it (a whole-stage pass
     // of 1000 FP64 samples 15.7 -> 14.6 thousand cycles, of 2800 FP32 ones 13.2
@@ -247,13 +252,15 @@ __device__ __forceinline__ void partition_pcr(int lane, RowFn row, real (&x)[B])
             d2 = d2 - Cm * k1;
             r2 = r2 - Rm * k1;
         }
+        const real d1 = d2, r1 = r2;
         if (lane + st < kWave) {
             const real k2 = sdiv<real>(C, Dp);
             c2 = -(Cp * k2);
             d2 = d2 - Ap * k2;
             r2 = r2 - Rp * k2;
         }
-        const bool changed = wave_ballot(!(d2 == D) | !(r2 == R)) != 0ull;
+        const bool changed =
+            wave_ballot(!(SYM || d1 == D) | !(d2 == D) | !(r1 == R) | !(r2 == R)) != 0ull;
         A = a2;
         C = c2;
         D = d2;
