@@ -682,6 +682,9 @@ __global__ __launch_bounds__(kThreads) void k_knot_prefix_w(SeriesDev sd, KnotsD
 // The solve keeps 4: 2 KB less LDS per workgroup.
 constexpr int kTMaskW = kWR + 1;
 
+// 32 samples' bits of a row mask that was written whole
+typedef uint32_t __attribute__((may_alias)) MaskHalf;
+
 template <int TW>
 __device__ __forceinline__ void gather_positions(const SeriesDev& sd, const uint64_t* kmask,
                                                  const int* kpre, const int* kcnt, int s, int type,
@@ -749,7 +752,7 @@ __device__ __forceinline__ void gather_positions(const SeriesDev& sd, const uint
             for (int q0 = 8 * xa; q0 <= 8 * xb; q0 += kWave) {
                 const int x = (q0 + lane) >> 3, sub = lane & 7;
                 const bool in = x <= xb;
-                uint32_t m = in ? ((const uint32_t*)tmask[in ? x : 0])[sub] : 0u;
+                uint32_t m = in ? ((const MaskHalf*)tmask[in ? x : 0])[sub] : 0u;
                 int before = __popc(m);
                 int gi = (in ? tpre[in ? x : 0] : 0) - before;
                 const int s1 = dpp_row_i<0x111, 0xF>(before, 0);
