@@ -658,10 +658,6 @@ __global__ __launch_bounds__(kThreads) void k_knot_prefix_w(SeriesDev sd, KnotsD
     }
 }
 
-// ------------------------------------------------------------- stage init
-
-// ---------------------------------------------------------------- sift pass
-
 // ------------------------------------------------------- windowed spline solve
 
 // Positions of knots [glo, ghi) of (series s, type) into LDS (sp index =
@@ -1238,7 +1234,6 @@ struct WTile {
 // appended to a.ovf_segs for a second launch with the full table, and the
 // tile after it takes h_new of its left neighbour from its own knots.
 //
-//
 // The pass is bound by the number of instructions of all kinds: VALU, scalar
 // and memory pipes were each about 58 % busy, and more than six waves per SIMD
 // changed nothing.
@@ -1356,7 +1351,6 @@ __device__ __forceinline__ void sift_segment(const SiftArgs<real>& a, const Segm
 #pragma unroll
         for (int ty = 0; ty < 2; ++ty) {
             if constexpr (Lay<real>::kQuad) {
-                // the lane's bits to the top, then out one by one (bit 3 first)
                 quad_masks(cur.mk[ty], lane, bm[ty]);
             } else {
 #pragma unroll

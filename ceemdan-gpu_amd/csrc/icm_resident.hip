@@ -779,9 +779,10 @@ hipError_t launch_stage(const StageArgs<real>& args, const StageGeom& g, hipStre
     const unsigned grid = (unsigned)g.grid;
     if (g.nwv == 4 && g.hold) launch_one<real, 4, true>(a, grid, g.lds, st);
     else if (g.nwv == 8 && g.hold) launch_one<real, 8, true>(a, grid, g.lds, st);
-    else if (g.nwv == 8) launch_one<real, 8, false>(a, grid, g.lds, st);
     else if (g.hold) launch_one<real, 16, true>(a, grid, g.lds, st);
-    else launch_one<real, 16, false>(a, grid, g.lds, st);
+    else if (g.nwv == 16) launch_one<real, 16, false>(a, grid, g.lds, st);
+    else if constexpr (sizeof(real) == 4) launch_one<real, 8, false>(a, grid, g.lds, st);   // FP32 only
+    else return hipErrorInvalidValue;
     return hipGetLastError();
 }
 

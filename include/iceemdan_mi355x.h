@@ -211,7 +211,7 @@ int icm_sift_pass(int dtype, const void* d_h, int64_t N, int64_t I, void* d_h_ne
  * harnesses that forbid hipMalloc).  Same arguments, kernels and result bit
  * for bit as icm_sift_pass, which allocates memory for the call only when the
  * series are too long for one workgroup's LDS or d_h_new overlaps d_h (here
- * they must not overlap); every buffer beyond d_h, d_h_new and d_nk is
+ * they are the same or do not overlap); every buffer beyond d_h, d_h_new and d_nk is
  * carved from one file-scope device array of 24 MiB per GPU, held until the
  * process ends.  Limits: I * N <= 2^21 samples and I <= 4096 series, else
  * ICM_ERR_INVALID_ARG.  Calls on one GPU share that GPU's array (it keeps
