@@ -726,25 +726,31 @@ void launch_one(const StageArgs<real>& a, unsigned grid, size_t lds, hipStream_t
 }  // namespace
 
 // Which phases take the stage kernel, and its workgroup.  Measured per pass
-// (us) against the tuned launch-per-step path on EEG-like noise-mode stages
-// (the first four rows: an earlier state of both):
+// (us, the CEEMDAN stages of a replayed decomposition of one EEG-like channel
+// with their sums) against the tuned launch-per-step path:
 //   series x samples    FP32 steps / stage     FP64 steps / stage
-//     50 x   1000           30.9 /  5.7            35.2 /  7.4
-//   4000 x   1000           94.8 / 25.9           118.2 / 44.3
-//     50 x   4000           33.3 /  7.0            37.3 /  9.1
-//   4000 x   4000          147.7 / 84.8           211.6 / 142.6
-//   4000 x   8000          246.3 / 182.4          347.8 / 288.8
-//   3000 x  16000          295.9 / 242.4          434.4 / 363.6
-//    500 x  24000           88.9 / 56.1           126.3 / 87.4
-//   3000 x  24000          410.8 / 334.1          606.2 / 509.0
-//    250 x  32000           70.4 / 39.3            95.6 / 68.6
-//    500 x  32000          108.7 / 76.6           155.0 / 133.5
-//    800 x  32000          153.5 / 144.5          232.0 / 253.1
-//   3000 x  32000          528.6 / 457.4          783.6 / 806.8
+//     50 x   1000           27.6 / 5.2             31.5 / 6.8
+//   4000 x   1000          132.1 / 50.8           152.5 / 67.9
+//     50 x   4000           28.5 / 6.7             34.3 / 9.0
+//   4000 x   4000          179.9 / 102.1          235.0 / 148.3
+//   4000 x   8000          245.8 / 183.5          347.6 / 289.0
+//   3000 x  16000          295.9 / 243.5          433.8 / 363.2
+//      4 x  24000           34.0 / 23.4            39.5 / 34.7
+//     50 x  24000           39.4 / 24.3            47.2 / 37.4
+//    500 x  24000           89.4 / 56.4           126.4 / 87.9
+//   3000 x  24000          411.2 / 335.0          605.2 / 508.0
+//      4 x  32000           34.9 / 30.6            42.0 / 47.7
+//     50 x  32000           41.8 / 32.0            49.1 / 51.8
+//    100 x  32000           46.0 / 35.8            59.9 / 54.3
+//    250 x  32000           70.7 / 39.6            95.3 / 68.7
+//    500 x  32000          108.4 / 77.2           155.1 / 134.9
+//    800 x  32000          153.4 / 145.1          232.0 / 253.1 (an earlier state)
+//   3000 x  32000          527.5 / 459.9          783.6 / 806.8 (an earlier state)
 // A workgroup sifts one series at a time and one fits a CU from about 2000
-// samples on, so its time grows with series / 256 while the launch-per-step
-// path spreads any one pass over the chip: only FP64 series of more than 96
-// tiles lose here, beyond three workgroups per CU.
+// samples on, so its time grows with series / 256 and is flat below 256, while
+// the launch-per-step path spreads any one pass over the chip: FP64 series of
+// more than 96 tiles lose here beyond three workgroups per CU, and the longest
+// where they are few (few_long_series in icm_plan.hip).
 // Waves per workgroup: one tile each as far as 16 waves go (the shortest
 // pass); FP32 series of up to 16 tiles in plans of more series than CUs take
 // 8 waves, so that two workgroups share a CU (500 x 4000: 11.8 against 13.4).
