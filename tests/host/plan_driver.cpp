@@ -234,6 +234,10 @@ bool record_room()
         }
         CHECK(g_prefixes > 0 && g_dirty == 0);   // without scratch: launches per step
         fake_free_bytes = (long long)1 << 40;
+        reset_watch();
+        CHECK(icm_forward(p, k.inp.data(), k.outp.data(), nullptr, nullptr) == ICM_OK);
+        CHECK(icm_backward(p, k.outp.data(), k.inp.data(), nullptr) == ICM_OK);
+        CHECK(g_stages == 0 && g_prefixes > 0 && g_dirty == 0);
         CHECK(device_bytes(p) <= fake_used_bytes && device_bytes(p) >= fake_used_bytes - (64 << 10));
         CHECK(icm_plan_destroy(p) == ICM_OK);
         CHECK(fake_used_bytes == 0);

@@ -115,6 +115,31 @@ def test_more_series_than_workgroups(icm, dev, monkeypatch):
         _same(a, b)
 
 
+@pytest.mark.parametrize("keep", [True, False])
+def test_phases_on_different_paths(icm, dev, monkeypatch, keep):
+    """4 x 32768, I = 20 in FP64: 20 noise-mode series launch step by step,
+    beside 80 series of the CEEMDAN phase in whole stages; replayed with other
+    inputs, forward and adjoint, and equal to launches per step."""
+    import torch
+    lens, I, M, S = [32768] * 4, 20, 4, 5
+    print(f"case: phases on different paths keep={keep}", flush=True)
+    kw = dict(dtype=torch.float64, max_sifts=S, device=dev, keep_records=keep)
+    steps = _plan(icm, monkeypatch, STEPS, lens, I, M, use_graph=False, **kw)
+    monkeypatch.delenv("ICM_WHOLE_STAGES", raising=False)
+    plan = icm.Plan(lens, I, M, **kw)
+    assert plan.tuning_left() == 0
+    rng = np.random.default_rng(8)
+    for seed in range(4):
+        xs = [torch.tensor(_sig().eeg_like(n, seed=900 + 10 * seed + c), device=dev)
+              for c, n in enumerate(lens)]
+        gs = [torch.tensor(rng.standard_normal((M, n)), device=dev) for n in lens]
+        for a, b in zip(plan.forward(xs) + plan.backward(gs), steps.forward(xs) + steps.backward(gs)):
+            _same(a, b)
+    assert plan.graph_status() == 1
+    plan.close()
+    steps.close()
+
+
 @pytest.mark.parametrize("dt", ["f64", "f32"])
 @pytest.mark.parametrize("stop", [0, 1])
 def test_staged_forward_that_changes_path(icm, dev, monkeypatch, dt, stop):
