@@ -737,8 +737,33 @@ bool few_long_series(const icm_config& c, const HostSeries& h)
     return c.stop_mode == ICM_STOP_FIXED ? n < std::min<int64_t>(3 * (ntl - 98), 72) : n < 4 * (ntl - 103);
 }
 
+// Long FP64 series, more than there are CUs, in a decomposition of few rows.
+// From 95 tiles on the knot rows of a dense pass fit LDS no longer, not even
+// their values, so the first stages, the only dense ones, are slow, and the
+// others make up for them from a number of rows on.  One channel, 10 sifts,
+// both phases side by side, stage kernel / tuned launches (1 = as fast):
+//   FIXED      M = 4: 257 series  400   513   768    M = 10: 257  400   513   768
+//     24000 samples   1.07  0.95  1.06  0.96           0.83  0.82  0.90  0.87
+//     24576           1.18  1.04  1.10  1.07           0.87  0.87  0.92  0.92
+//     28000           1.21  1.07  1.15  1.06           0.92  0.89  0.96  0.93
+//     32768           1.35  1.17  1.29  1.18           1.04  0.95  1.03  1.01
+//   RILLING, caps 30 and 40 at 300 and 513 series (100 and 300: within 0.1)
+//                     M = 3            M = 6            M = 10
+//     24576           1.16  1.11       0.96  0.91       0.85  0.83
+//     28000           1.18  1.21       0.99  1.00       0.93  0.94
+//     32768           1.27  1.32       1.06  1.08       0.99  0.99
+// (the ratio falls by about a twentieth per row; just past a multiple of the
+// CUs it is a tenth higher than halfway to the next: the line is between)
+bool few_rows_of_long_series(const icm_config& c, const HostSeries& h)
+{
+    const int64_t ntl = (h.max_len + tile_of(c.dtype) - 1) / tile_of(c.dtype), n = (h.ntiles + ntl - 1) / ntl;
+    if (c.dtype != ICM_DTYPE_F64 || ntl <= 94 || n <= 256) return false;
+    return c.stop_mode == ICM_STOP_FIXED ? 16 * (c.num_imfs - 5) < ntl - 94 : 16 * (c.num_imfs - 3) <= ntl - 94;
+}
+
 // Launch shape of the stage kernel for one phase (ok = false: launches per
-// step).  ICM_WHOLE_STAGES=0 turns it off, 1 takes it for few long series too.
+// step).  ICM_WHOLE_STAGES=0 turns it off, 1 takes it wherever the series'
+// length and number allow.
 StageGeom stage_choice(const icm_config& c, int phase, const HostSeries& h)
 {
     const char* env = std::getenv("ICM_WHOLE_STAGES");
@@ -751,6 +776,7 @@ StageGeom stage_choice(const icm_config& c, int phase, const HostSeries& h)
         g.ok = false;
         g.few = true;
     }
+    if (!env && few_rows_of_long_series(c, h)) g.ok = false;
     return g;
 }
 

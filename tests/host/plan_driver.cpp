@@ -304,6 +304,32 @@ bool few_series()
     return true;
 }
 
+// The same by the number of rows, for more long series than CUs; the launches
+// per step are tuned then.
+bool few_rows()
+{
+    const struct { int dtype, stop, n, I, M; bool whole; } t[] = {
+        {ICM_DTYPE_F64, ICM_STOP_FIXED, 32768, 300, 7, false}, {ICM_DTYPE_F64, ICM_STOP_FIXED, 32768, 300, 8, true},
+        {ICM_DTYPE_F64, ICM_STOP_FIXED, 32768, 256, 3, true},   {ICM_DTYPE_F64, ICM_STOP_FIXED, 24576, 300, 5, false},
+        {ICM_DTYPE_F64, ICM_STOP_FIXED, 24576, 300, 6, true},   {ICM_DTYPE_F64, ICM_STOP_FIXED, 24064, 300, 3, true},
+        {ICM_DTYPE_F64, ICM_STOP_RILLING, 28160, 300, 4, false}, {ICM_DTYPE_F64, ICM_STOP_RILLING, 28160, 300, 5, true},
+        {ICM_DTYPE_F32, ICM_STOP_FIXED, 32768, 300, 3, true},
+    };
+    for (const auto& q : t) {
+        Call k({q.n}, q.I, q.M, q.dtype, q.stop);
+        icm_plan p = nullptr;
+        CHECK(icm_plan_create(&k.c, &p) == ICM_OK);
+        int left = -1;
+        CHECK(icm_get_tuning_left(p, &left) == ICM_OK && (left == 0) == q.whole);
+        reset_watch();
+        CHECK(icm_forward(p, k.inp.data(), k.outp.data(), nullptr, nullptr) == ICM_OK);
+        if ((g_stages > 0) != q.whole) std::printf("dtype %d stop %d %d x %d M %d\n", q.dtype, q.stop, q.I, q.n, q.M);
+        CHECK((g_stages > 0) == q.whole && (g_prefixes > 0) != q.whole);
+        CHECK(icm_plan_destroy(p) == ICM_OK);
+    }
+    return true;
+}
+
 std::vector<FakeLaunch> g_noise;
 std::vector<std::vector<int>> g_noise_len;
 
@@ -365,6 +391,7 @@ int main(int argc, char** argv)
         {"trace_room", trace_room},
         {"tuning_round_trip", tuning_round_trip},
         {"few_series", few_series},
+        {"few_rows", few_rows},
         {"noise_groups", noise_groups},
     };
     for (int i = 1; i < argc; ++i)

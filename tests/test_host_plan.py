@@ -77,5 +77,11 @@ def test_few_long_series_launch_step_by_step(driver):
     driver("few_series")
 
 
+def test_long_series_of_few_rows_launch_step_by_step(driver):
+    """More FP64 series of 95 tiles and up than CUs, in a decomposition whose
+    dense first stages weigh most."""
+    driver("few_rows")
+
+
 def test_noise_of_uneven_lengths_launches_few_idle_workgroups(driver):
     driver("noise_groups")
