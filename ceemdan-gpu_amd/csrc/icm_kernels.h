@@ -129,7 +129,22 @@ struct SiftArgs {
     // per segment): a resident grid of wavefronts takes segments from it one
     // at a time until none is left
     unsigned* queue;
+    bool past_caches;       // samples past the caches (sift_past_caches)
 };
+
+// Whether the sift's samples go past the caches: where the two sample buffers
+// of a phase do not fit the 256 MB one.  Whole decompositions past them and
+// through them, ms, by the size of one buffer:
+//              FP64, 8 channels      FP32, 8 channels      FP64, 1 channel
+//   102 MB       6.49 / 6.21           7.40 / 7.12           9.87 / 9.79 (96 MB)
+//   128          7.67 / 7.61           8.46 / 8.42          12.55 / 12.77
+//   153          8.87 / 8.96           9.89 / 10.02
+//   204         11.40 / 11.52         12.59 / 12.91         18.02 / 18.48 (192 MB)
+// (one channel: both phases are that large and run side by side)
+inline bool sift_past_caches(int64_t samples, size_t size)
+{
+    return samples * (int64_t)size > (int64_t)128 << 20;
+}
 
 template <typename real>
 struct SolveArgs {

@@ -1155,27 +1155,42 @@ struct Lay {
     __device__ __forceinline__ static int at(int q, int lane) { return kQuad ? 4 * lane + q : kWave * q + lane; }
 };
 
-// Samples go past the caches in both directions: a pass reads and writes each
-// once, and what is read again (tables, masks) stays cached (sift launches
-// above with rows: 114.3 -> 112.8 ms FP32, 44.5 -> 42.5 FP64).  A whole tile's
-// samples of the lane, a series may start at any sample.
+// NT: samples go past the caches in both directions, as a pass reads and writes
+// each once; what is read again (tables, masks) stays cached (sift launches
+// above with rows: 114.3 -> 112.8 ms FP32, 44.5 -> 42.5 FP64).  Only where the
+// samples do not fit the caches (sift_past_caches): the passes and knot
+// prefixes of a smaller phase read them there (96 MB of FP64 samples, Rilling
+// rule, 91.1 ms past the caches, 85.2 through them).  A whole tile's samples of
+// the lane, a series may start at any sample.
 typedef float Quad __attribute__((ext_vector_type(4), aligned(4)));
-template <typename real>
+template <bool NT, typename T>
+__device__ __forceinline__ T load_sample(const T* p)
+{
+    if constexpr (NT) return __builtin_nontemporal_load(p);
+    else return *p;
+}
+template <bool NT, typename T>
+__device__ __forceinline__ void store_sample(T v, T* p)
+{
+    if constexpr (NT) __builtin_nontemporal_store(v, p);
+    else *p = v;
+}
+template <bool NT, typename real>
 __device__ __forceinline__ void load_quad(const real* p, real (&v)[kWR])
 {
-    const Quad q = __builtin_nontemporal_load((const Quad*)p);
+    const Quad q = load_sample<NT>((const Quad*)p);
 #pragma unroll
     for (int i = 0; i < kWR; ++i) v[i] = q[i];
 }
-template <typename real>
+template <bool NT, typename real>
 __device__ __forceinline__ void store_tile(real* p, int lane, const real (&v)[kWR])
 {
     if constexpr (Lay<real>::kQuad) {
         const Quad q = {v[0], v[1], v[2], v[3]};
-        __builtin_nontemporal_store(q, (Quad*)(p + 4 * lane));
+        store_sample<NT>(q, (Quad*)(p + 4 * lane));
     } else {
 #pragma unroll
-        for (int r = 0; r < kWR; ++r) __builtin_nontemporal_store(v[r], p + r * kWave + lane);
+        for (int r = 0; r < kWR; ++r) store_sample<NT>(v[r], p + r * kWave + lane);
     }
 }
 
@@ -1237,7 +1252,7 @@ struct WTile {
 // The pass is bound by the number of instructions of all kinds: VALU, scalar
 // and memory pipes were each about 58 % busy, and more than six waves per SIMD
 // changed nothing.
-template <typename real, bool RILL, int KC>
+template <typename real, bool RILL, int KC, bool NT>
 __device__ __forceinline__ void sift_segment(const SiftArgs<real>& a, const Segment* segs, int sid,
                                              int lane, KnotTable<real, KC>& T)
 {
@@ -1268,12 +1283,12 @@ __device__ __forceinline__ void sift_segment(const SiftArgs<real>& a, const Segm
     auto load = [&](int t, const int (&pre)[2], const int (&cnt)[2], WTile<real, KC>& w) {
         const int t0 = t * kWT;
         if (Lay<real>::kQuad && t0 + kWT <= N) {
-            load_quad(h + t0 + 4 * lane, w.h);
+            load_quad<NT>(h + t0 + 4 * lane, w.h);
         } else {
 #pragma unroll
             for (int q = 0; q < kWR; ++q) {
                 const int p = t0 + Lay<real>::at(q, lane);
-                w.h[q] = p < N ? __builtin_nontemporal_load(h + p) : (real)0;
+                w.h[q] = p < N ? load_sample<NT>(h + p) : (real)0;
             }
         }
 #pragma unroll
@@ -1498,7 +1513,7 @@ __device__ __forceinline__ void sift_segment(const SiftArgs<real>& a, const Segm
             auto stores = [&]() {
                 wait_vmem();
                 if (FULL) {
-                    store_tile(hout + t0, lane, hn);
+                    store_tile<NT>(hout + t0, lane, hn);
                 } else {
 #pragma unroll
                     for (int q = 0; q < kWR; ++q) {
@@ -1656,7 +1671,7 @@ __device__ __forceinline__ void sift_segment(const SiftArgs<real>& a, const Segm
 // and 4 43.9, 5 and 4 42.5).
 template <typename real, int KC>
 constexpr int kSiftWaves = sizeof(real) == 4 ? (KC == kWKS ? 6 : 5) : (KC == kWKS ? 5 : 1);
-template <typename real, bool RILL, int KC, bool QUEUE>
+template <typename real, bool RILL, int KC, bool NT, bool QUEUE>
 __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(kSiftWaves<real, KC>)))
 void k_sift_w(SiftArgs<real> a, int nsegs)
 {
@@ -1670,14 +1685,14 @@ void k_sift_w(SiftArgs<real> a, int nsegs)
     if (!QUEUE) {
         const int sid = blockIdx.x * NW + wv;
         if (sid < nsegs)
-            sift_segment<real, RILL, KC>(a, a.segs, sid, lane, s_tab[wv]);
+            sift_segment<real, RILL, KC, NT>(a, a.segs, sid, lane, s_tab[wv]);
         return;
     }
     unsigned got = lane == 0 ? atomicAdd(a.queue, 1u) : 0u;
     int sid = __builtin_amdgcn_readlane((int)got, 0);
     while (sid < nsegs) {
         const unsigned next = lane == 0 ? atomicAdd(a.queue, 1u) : 0u;
-        sift_segment<real, RILL, KC>(a, a.segs, sid, lane, s_tab[wv]);
+        sift_segment<real, RILL, KC, NT>(a, a.segs, sid, lane, s_tab[wv]);
         wave_sync();
         sid = __builtin_amdgcn_readlane((int)next, 0);
     }
@@ -1687,7 +1702,7 @@ void k_sift_w(SiftArgs<real> a, int nsegs)
 // loop: the tiles the small-table launch listed (*a.ovf_count one-tile
 // segments in a.ovf_segs) or, when the pass input had too many over-full
 // tiles for it to run, every segment of the pass.
-template <typename real, bool RILL>
+template <typename real, bool RILL, bool NT>
 __global__ __launch_bounds__(kThreads) void k_sift_list(SiftArgs<real> a, int nsegs)
 {
     constexpr int NW = kThreads / kWave;
@@ -1700,7 +1715,7 @@ __global__ __launch_bounds__(kThreads) void k_sift_list(SiftArgs<real> a, int ns
     SiftArgs<real> b = a;
     b.ovf_segs = nullptr;   // full tables hold every tile
     for (int sid = blockIdx.x * NW + wv; sid < ns; sid += gridDim.x * NW)
-        sift_segment<real, RILL, kWKC>(b, segs, sid, lane, s_tab[wv]);
+        sift_segment<real, RILL, kWKC, NT>(b, segs, sid, lane, s_tab[wv]);
 }
 
 // Stage start for 256-sample tiles: forms x_i and stores its knots as bitmasks.  MODE is ia.mode as a
@@ -2717,24 +2732,24 @@ static dim3 sift_grid(K kernel, const unsigned* queue, int nsegs)
     return dim3((unsigned)std::max<int64_t>(1, std::min<int64_t>(need, resident_groups(kernel))));
 }
 
-template <typename real, bool RILL, int KC>
+template <typename real, bool RILL, int KC, bool NT>
 static void launch_sift_w(const SiftArgs<real>& a, int nsegs, hipStream_t st)
 {
     if (a.queue) {
-        auto k = k_sift_w<real, RILL, KC, true>;
+        // (past 2^32 work-items the samples never fit the caches)
+        auto k = k_sift_w<real, RILL, KC, true, true>;
         hipLaunchKernelGGL(k, sift_grid(k, a.queue, nsegs), dim3(kThreads), 0, st, a, nsegs);
     } else {
-        auto k = k_sift_w<real, RILL, KC, false>;
+        auto k = k_sift_w<real, RILL, KC, NT, false>;
         hipLaunchKernelGGL(k, sift_grid(k, a.queue, nsegs), dim3(kThreads), 0, st, a, nsegs);
     }
 }
 
-template <typename real>
-hipError_t launch_sift(const SiftArgs<real>& a, int nsegs, hipStream_t st)
+template <typename real, bool RILL, bool NT>
+static hipError_t launch_sift_as(const SiftArgs<real>& a, int nsegs, hipStream_t st)
 {
     if (!a.ovf_segs) {
-        if (a.sx_cnt) launch_sift_w<real, true, kWKC>(a, nsegs, st);
-        else launch_sift_w<real, false, kWKC>(a, nsegs, st);
+        launch_sift_w<real, RILL, kWKC, NT>(a, nsegs, st);
         return hipGetLastError();
     }
     // sparse pass: if few tiles of the input overflow the small knot tables
@@ -2744,14 +2759,19 @@ hipError_t launch_sift(const SiftArgs<real>& a, int nsegs, hipStream_t st)
     // Its grid is what the full-table kernel keeps resident (four
     // workgroups per CU), so it costs little when it has nothing to do.
     const dim3 lgrid(std::min<unsigned>(blocks_for(nsegs, kThreads / kWave), 1024u));
-    if (a.sx_cnt) {
-        launch_sift_w<real, true, kWKS>(a, nsegs, st);
-        hipLaunchKernelGGL((k_sift_list<real, true>), lgrid, dim3(kThreads), 0, st, a, nsegs);
-    } else {
-        launch_sift_w<real, false, kWKS>(a, nsegs, st);
-        hipLaunchKernelGGL((k_sift_list<real, false>), lgrid, dim3(kThreads), 0, st, a, nsegs);
-    }
+    launch_sift_w<real, RILL, kWKS, NT>(a, nsegs, st);
+    hipLaunchKernelGGL((k_sift_list<real, RILL, NT>), lgrid, dim3(kThreads), 0, st, a, nsegs);
     return hipGetLastError();
+}
+
+template <typename real>
+hipError_t launch_sift(const SiftArgs<real>& a, int nsegs, hipStream_t st)
+{
+    if (a.sx_cnt)
+        return a.past_caches ? launch_sift_as<real, true, true>(a, nsegs, st)
+                             : launch_sift_as<real, true, false>(a, nsegs, st);
+    return a.past_caches ? launch_sift_as<real, false, true>(a, nsegs, st)
+                         : launch_sift_as<real, false, false>(a, nsegs, st);
 }
 
 template <typename real>

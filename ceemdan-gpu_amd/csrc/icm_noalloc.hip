@@ -224,6 +224,7 @@ int sift_steps(const Tables<real>& t, const real* h, int N, int I, real* h_new, 
     a.emit = 0;
     a.pc = ctl(2);
     a.queue = nullptr;   // one wavefront per segment (the grid is small here)
+    a.past_caches = sift_past_caches((int64_t)I * N, sizeof(real));
     if (launch_sift<real>(a, I * nseg_s, st) != hipSuccess) return ICM_ERR_HIP;
     if (d_nk && launch_copy<float>((float*)d_nk, (const float*)k.n, 2 * (int64_t)I, st) != hipSuccess)
         return ICM_ERR_HIP;

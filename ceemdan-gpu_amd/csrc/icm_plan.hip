@@ -1114,6 +1114,7 @@ struct Plan : PlanBase {
         // 2^32 work-items: then the work-queue instance on a resident grid
         const bool queue = sift_queue || (int64_t)d.nsegs[l] * 64 >= ((int64_t)1 << 32);
         a.queue = queue ? L.squeue + e : nullptr;
+        a.past_caches = sift_past_caches(d.samples, sizeof(real));
         if (small) sparse_pass(a, L, d, e_in, e);
         int rc;
         if ((rc = prof_begin(2, bytes, st))) return rc;

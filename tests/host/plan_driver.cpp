@@ -330,6 +330,40 @@ bool few_rows()
     return true;
 }
 
+int g_past, g_through;
+
+void watch_sift(const FakeLaunch& l)
+{
+    if (!is(l, "k_sift_w")) return;
+    const bool f64 = is(l, "k_sift_wId");
+    const bool past = f64 ? ((const SiftArgs<double>*)l.args[0])->past_caches
+                          : ((const SiftArgs<float>*)l.args[0])->past_caches;
+    ++(past ? g_past : g_through);
+}
+
+// Samples go past the caches where a phase's two buffers exceed 256 MB, each
+// phase by its own size.
+bool past_caches()
+{
+    const struct { int dtype, I, channels, past, through; } t[] = {
+        {ICM_DTYPE_F64, 68, 1, 0, 2}, {ICM_DTYPE_F64, 69, 1, 2, 0}, {ICM_DTYPE_F64, 35, 2, 1, 1},
+        {ICM_DTYPE_F32, 137, 1, 0, 2}, {ICM_DTYPE_F32, 138, 1, 2, 0},
+    };
+    for (const auto& q : t) {
+        Call k(std::vector<int64_t>(q.channels, 244032), q.I, 2, q.dtype);
+        k.c.max_sifts = k.c.noise_max_sifts = 1;
+        icm_plan p = nullptr;
+        CHECK(icm_plan_create(&k.c, &p) == ICM_OK);
+        CHECK(icm_set_autotune(p, 0) == ICM_OK);
+        g_past = g_through = 0;
+        fake_on_launch = watch_sift;
+        CHECK(icm_forward(p, k.inp.data(), k.outp.data(), nullptr, nullptr) == ICM_OK);
+        CHECK(g_past == q.past && g_through == q.through);
+        CHECK(icm_plan_destroy(p) == ICM_OK);
+    }
+    return true;
+}
+
 std::vector<FakeLaunch> g_noise;
 std::vector<std::vector<int>> g_noise_len;
 
@@ -393,6 +427,7 @@ int main(int argc, char** argv)
         {"few_series", few_series},
         {"few_rows", few_rows},
         {"noise_groups", noise_groups},
+        {"past_caches", past_caches},
     };
     for (int i = 1; i < argc; ++i)
         for (const auto& t : all)

@@ -274,3 +274,25 @@ def test_allocation_free_pass_in_place(icm, dev, dt, rows, n):
     assert icm.lib().icm_sift_pass_static(icm._dtype_code(dtype), C.c_void_p(h.data_ptr()), n, rows,
                                           C.c_void_p(h.data_ptr()), C.c_void_p(k2.data_ptr()), st) == 0
     assert torch.equal(h, ref) and torch.equal(k2, nk)
+
+
+@pytest.mark.parametrize("dt,C", [("f64", 8), ("f32", 16)])
+@pytest.mark.parametrize("stop", [0, 1])
+def test_samples_past_the_caches(icm, dev, dt, C, stop):
+    """8 x 70 k FP64 (16 FP32) channels, I = 32: 143 MB a buffer, sifted past the
+    caches; each of two channels alone, 18 (9) MB, through them.  The same bits."""
+    import torch
+    dtype = torch.float64 if dt == "f64" else torch.float32
+    lens, I, M = [70001 - 3 * c for c in range(C)], 32, 3
+    print(f"case: past the caches {dt} stop={stop}", flush=True)
+    kw = dict(dtype=dtype, stop_mode=stop, max_sifts=4 if stop == 0 else 12,
+              noise_max_sifts=4 if stop == 0 else 20, use_graph=False, device=dev)
+    xs = _inputs(dtype, lens)
+    plan = icm.Plan(lens, I, M, **kw)
+    assert plan.info()["signal_samples"] * xs[0].element_size() > 128 << 20
+    got = [o.clone() for o in plan.forward(xs)]
+    plan.close()
+    for c in (0, C - 1):
+        alone = icm.Plan([lens[c]], I, M, **kw)
+        _same(alone.forward([xs[c]])[0], got[c])
+        alone.close()

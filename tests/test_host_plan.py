@@ -85,3 +85,7 @@ def test_long_series_of_few_rows_launch_step_by_step(driver):
 
 def test_noise_of_uneven_lengths_launches_few_idle_workgroups(driver):
     driver("noise_groups")
+
+
+def test_samples_past_the_caches_only_where_they_do_not_fit(driver):
+    driver("past_caches")
