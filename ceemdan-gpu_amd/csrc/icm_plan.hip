@@ -710,43 +710,43 @@ void layout(PlanBase& P)
     P.cap = T / 2 + 2;   // strict extrema are never adjacent, plus the two ends
 }
 
-// Series that a workgroup each takes longer for than launches per step that
-// spread one pass over the chip: long FP64 ones, while they are few.  A
-// decomposition of one channel, M = 6, in ms, launches (default geometry) /
-// stage kernel, both phases side by side where FIXED:
-//   FIXED, 10 sifts    series  16          32          48          64          80
-//     26000 samples        2.42/2.70   2.68/2.84   3.05/2.94   3.35/2.97   3.54/3.01
-//     28000                2.61/2.91   2.86/3.05   3.12/3.10   3.39/3.14   3.73/3.20
-//     30000                2.60/3.08   2.89/3.25   3.22/3.37   3.47/3.40   3.89/3.46
-//     32768                2.65/3.41   2.95/3.61   3.30/3.68   3.62/3.72   4.01/3.77
-//   RILLING, caps 100 and 2000, 16, 40 and 80 series
-//     26000                39.6/36.6   44.1/40.8   51.7/44.8
-//     28000                37.3/38.2   44.1/42.9   51.5/47.6
-//     30000                44.0/45.9   52.5/52.9   59.8/57.1
-//     32768                48.1/54.6   59.8/66.9   70.2/73.4
-// (another run had the launches at 16 series up to 0.3 ms slower: the line
-// keeps to the stage kernel where the two runs disagree.)  Up to 98 tiles the
-// stage kernel is not behind at any number, nor in FP32 at any length it takes
-// (4 series of 32768: 2.43 / 2.02).  Series of other lengths in the plan count
-// by their tiles: 20 of 32768 and 400 of 300 samples 2.75 / 3.22, 400 of 3000
-// 3.04 / 3.30.
-bool few_long_series(const icm_config& c, const HostSeries& h)
+// Where launches per step are ahead of the stage kernel although the series'
+// length and number allow it.  A workgroup takes as long for one series as for
+// 128 of them (both phases then fill the CUs), while launches spread each pass
+// over the chip; and the first stages are dense, of FP64 series from 95 tiles
+// on so dense that not even their knots' values fit LDS, which the later
+// stages make up for the sooner the more rows there are.  The lines were fitted
+// to kept and one-shot decompositions of one channel of 5000 to 32768
+// samples, 4 to 110 series, M = 2 to 12: what they choose is 0.1 % slower on
+// average than the faster side (one-shot 0.8 %, RILLING 0.7 %), 16 % at worst.
+// Stage kernel / launches (default geometry), kept, FP64, FIXED, 10 sifts:
+//              M = 3: 4 series  60   110    M = 6: 4    60   110    M = 12: 4    60
+//   16384 samples    1.26  1.01  0.81
+//   20000            1.35  1.02  0.85         0.91  0.76  0.67          0.65  0.64
+//   24576            1.85  1.34  1.05         1.11  0.93  0.79          0.90  0.74
+//   32768            2.35  1.54  1.20         1.41  1.12  0.92          1.01  0.81
+// At 32768, 4 and 60 series: FP32 M = 3 1.40 1.12, M = 4 1.21 1.04; FP64,
+// RILLING, caps 100 and 300, M = 3 1.93 1.52, M = 8 1.39 1.16.  Launches of
+// M = 3 take 0.98, 1.71 and 2.29 ms at 32768, the stage kernel 2.29 to 2.75.
+// Such phases are not tuned: the default geometry is as fast there, and two
+// timing forwards cost 7.5 ms each.
+bool few_long_series(const icm_config& c, int64_t ntl, int64_t n)
 {
-    if (c.dtype != ICM_DTYPE_F64) return false;
-    const int64_t ntl = (h.max_len + tile_of(c.dtype) - 1) / tile_of(c.dtype), n = (h.ntiles + ntl - 1) / ntl;
-    return c.stop_mode == ICM_STOP_FIXED ? n < std::min<int64_t>(3 * (ntl - 98), 72) : n < 4 * (ntl - 103);
+    if (n > 128) return false;
+    const int64_t m = c.num_imfs - 1, t = 1000 * ntl, nt = n * ntl;
+    const bool f64 = c.dtype == ICM_DTYPE_F64;
+    if (c.stop_mode == ICM_STOP_RILLING)
+        return f64 ? 2 * t > 112000 + 15000 * m + 5 * nt : t > 100000 + 10000 * m + 3 * nt;
+    return f64 ? t + (ntl > 94 ? 10000 : 0) > 31000 + 12000 * m + 4 * nt : t > 72000 + 16000 * m + nt;
 }
 
-// Long FP64 series, more than there are CUs, in a decomposition of few rows.
-// From 95 tiles on the knot rows of a dense pass fit LDS no longer, not even
-// their values, so the first stages, the only dense ones, are slow, and the
-// others make up for them from a number of rows on.  One channel, 10 sifts,
-// both phases side by side, stage kernel / tuned launches (1 = as fast):
+// The same beyond, for dense FP64 stages and few rows (tuned launches):
 //   FIXED      M = 4: 257 series  400   513   768    M = 10: 257  400   513   768
 //     24000 samples   1.07  0.95  1.06  0.96           0.83  0.82  0.90  0.87
 //     24576           1.18  1.04  1.10  1.07           0.87  0.87  0.92  0.92
 //     28000           1.21  1.07  1.15  1.06           0.92  0.89  0.96  0.93
 //     32768           1.35  1.17  1.29  1.18           1.04  0.95  1.03  1.01
+//     (M = 3 at 150 and 200 series: 24576 1.11 0.95, 32768 1.20 1.04)
 //   RILLING, caps 30 and 40 at 300 and 513 series (100 and 300: within 0.1)
 //                     M = 3            M = 6            M = 10
 //     24576           1.16  1.11       0.96  0.91       0.85  0.83
@@ -754,11 +754,11 @@ bool few_long_series(const icm_config& c, const HostSeries& h)
 //     32768           1.27  1.32       1.06  1.08       0.99  0.99
 // (the ratio falls by about a twentieth per row; just past a multiple of the
 // CUs it is a tenth higher than halfway to the next: the line is between)
-bool few_rows_of_long_series(const icm_config& c, const HostSeries& h)
+bool few_rows_of_long_series(const icm_config& c, int64_t ntl, int64_t n)
 {
-    const int64_t ntl = (h.max_len + tile_of(c.dtype) - 1) / tile_of(c.dtype), n = (h.ntiles + ntl - 1) / ntl;
-    if (c.dtype != ICM_DTYPE_F64 || ntl <= 94 || n <= 256) return false;
-    return c.stop_mode == ICM_STOP_FIXED ? 16 * (c.num_imfs - 5) < ntl - 94 : 16 * (c.num_imfs - 3) <= ntl - 94;
+    if (c.dtype != ICM_DTYPE_F64 || ntl <= 94 || n <= 128) return false;
+    if (c.stop_mode == ICM_STOP_FIXED) return 16 * (c.num_imfs - (n > 256 ? 5 : 2)) < ntl - 94;
+    return n > 256 && 16 * (c.num_imfs - 3) <= ntl - 94;
 }
 
 // Launch shape of the stage kernel for one phase (ok = false: launches per
@@ -772,11 +772,11 @@ StageGeom stage_choice(const icm_config& c, int phase, const HostSeries& h)
     // a stage of a few passes does not repay the allocation
     const int passes = phase == ICM_PHASE_NOISE ? c.noise_max_sifts : c.max_sifts;
     if (g.slot && passes < 4) g.ok = false;
-    if (g.ok && !env && few_long_series(c, h)) {
-        g.ok = false;
-        g.few = true;
-    }
-    if (!env && few_rows_of_long_series(c, h)) g.ok = false;
+    if (!g.ok || env) return g;
+    // series of other lengths than the longest count by their tiles
+    const int64_t ntl = (h.max_len + tile_of(c.dtype) - 1) / tile_of(c.dtype), n = (h.ntiles + ntl - 1) / ntl;
+    g.few = few_long_series(c, ntl, n);
+    g.ok = !g.few && !few_rows_of_long_series(c, ntl, n);
     return g;
 }
 

@@ -749,8 +749,8 @@ void launch_one(const StageArgs<real>& a, unsigned grid, size_t lds, hipStream_t
 // A workgroup sifts one series at a time and one fits a CU from about 2000
 // samples on, so its time grows with series / 256 and is flat below 256, while
 // the launch-per-step path spreads any one pass over the chip: FP64 series of
-// more than 96 tiles lose here beyond three workgroups per CU, and the longest
-// where they are few (few_long_series in icm_plan.hip).
+// more than 96 tiles lose here beyond three workgroups per CU, and long ones
+// where they or their rows are few (few_long_series in icm_plan.hip).
 // Waves per workgroup: one tile each as far as 16 waves go (the shortest
 // pass); FP32 series of up to 16 tiles in plans of more series than CUs take
 // 8 waves, so that two workgroups share a CU (500 x 4000: 11.8 against 13.4).

@@ -272,24 +272,29 @@ bool tuning_round_trip()
     return true;
 }
 
-// Which path a plan takes by its series' length and number.
+// Which path a plan takes by its series' length and number and its rows:
+// both sides of the lines.
 bool few_series()
 {
+    const int F = ICM_STOP_FIXED, R = ICM_STOP_RILLING;
     // (`more` channels of 300 samples beside the one)
-    const struct { int dtype, stop, n, I; bool whole; int more; } t[] = {
-        {ICM_DTYPE_F64, ICM_STOP_FIXED, 32768, 4, false},  {ICM_DTYPE_F64, ICM_STOP_FIXED, 32768, 71, false},
-        {ICM_DTYPE_F64, ICM_STOP_FIXED, 32768, 72, true},  {ICM_DTYPE_F64, ICM_STOP_FIXED, 28160, 35, false},
-        {ICM_DTYPE_F64, ICM_STOP_FIXED, 28160, 36, true},  {ICM_DTYPE_F64, ICM_STOP_FIXED, 25088, 1, true},
-        {ICM_DTYPE_F64, ICM_STOP_RILLING, 32768, 99, false}, {ICM_DTYPE_F64, ICM_STOP_RILLING, 32768, 100, true},
-        {ICM_DTYPE_F64, ICM_STOP_RILLING, 26368, 1, true}, {ICM_DTYPE_F32, ICM_STOP_FIXED, 32768, 1, true},
-        {ICM_DTYPE_F32, ICM_STOP_RILLING, 32768, 1, true}, {ICM_DTYPE_F64, ICM_STOP_FIXED, 1000, 1, true},
-        {ICM_DTYPE_F64, ICM_STOP_FIXED, 32768, 20, false, 20}, {ICM_DTYPE_F64, ICM_STOP_FIXED, 32768, 70, true, 9},
-        {ICM_DTYPE_F32, ICM_STOP_FIXED, 32768, 20, true, 20},
+    const struct { int dtype, stop, n, I, M; bool whole; int more; } t[] = {
+        {ICM_DTYPE_F64, F, 32768, 4, 6, false},  {ICM_DTYPE_F64, F, 32768, 91, 6, false},
+        {ICM_DTYPE_F64, F, 32768, 92, 6, true},  {ICM_DTYPE_F64, F, 28160, 65, 6, false},
+        {ICM_DTYPE_F64, F, 28160, 66, 6, true},  {ICM_DTYPE_F64, F, 24064, 1, 6, false},
+        {ICM_DTYPE_F64, F, 24064, 1, 7, true},   {ICM_DTYPE_F64, F, 14336, 1, 3, false},
+        {ICM_DTYPE_F64, F, 14080, 1, 4, true},   {ICM_DTYPE_F64, F, 32768, 1, 12, true},
+        {ICM_DTYPE_F64, R, 32768, 107, 6, false}, {ICM_DTYPE_F64, R, 32768, 108, 6, true},
+        {ICM_DTYPE_F64, R, 24064, 4, 6, true},   {ICM_DTYPE_F32, F, 32768, 1, 4, false},
+        {ICM_DTYPE_F32, F, 32768, 1, 5, true},   {ICM_DTYPE_F32, R, 32768, 1, 3, false},
+        {ICM_DTYPE_F32, R, 32768, 1, 4, true},   {ICM_DTYPE_F64, F, 1000, 1, 2, true},
+        {ICM_DTYPE_F64, F, 32768, 20, 6, false, 20}, {ICM_DTYPE_F64, F, 32768, 90, 6, true, 7},
+        {ICM_DTYPE_F32, F, 32768, 20, 6, true, 20},
     };
     for (const auto& q : t) {
         std::vector<int64_t> lens(1 + q.more, 300);
         lens[0] = q.n;
-        Call k(lens, q.I, 2, q.dtype, q.stop);
+        Call k(lens, q.I, q.M, q.dtype, q.stop);
         icm_plan p = nullptr;
         CHECK(icm_plan_create(&k.c, &p) == ICM_OK);
         int left = -1;
@@ -297,20 +302,20 @@ bool few_series()
         reset_watch();
         CHECK(icm_forward(p, k.inp.data(), k.outp.data(), nullptr, nullptr) == ICM_OK);
         if ((g_stages > 0) != q.whole || (g_prefixes > 0) == q.whole)
-            std::printf("dtype %d stop %d %d x %d\n", q.dtype, q.stop, q.I, q.n);
+            std::printf("dtype %d stop %d %d x %d M %d\n", q.dtype, q.stop, q.I, q.n, q.M);
         CHECK((g_stages > 0) == q.whole && (g_prefixes > 0) != q.whole);
         CHECK(icm_plan_destroy(p) == ICM_OK);
     }
     return true;
 }
 
-// The same by the number of rows, for more long series than CUs; the launches
-// per step are tuned then.
+// The same for more than 128 series; the launches per step are tuned then.
 bool few_rows()
 {
     const struct { int dtype, stop, n, I, M; bool whole; } t[] = {
         {ICM_DTYPE_F64, ICM_STOP_FIXED, 32768, 300, 7, false}, {ICM_DTYPE_F64, ICM_STOP_FIXED, 32768, 300, 8, true},
-        {ICM_DTYPE_F64, ICM_STOP_FIXED, 32768, 256, 3, true},   {ICM_DTYPE_F64, ICM_STOP_FIXED, 24576, 300, 5, false},
+        {ICM_DTYPE_F64, ICM_STOP_FIXED, 32768, 256, 5, true},   {ICM_DTYPE_F64, ICM_STOP_FIXED, 32768, 256, 4, false},
+        {ICM_DTYPE_F64, ICM_STOP_FIXED, 24576, 300, 5, false},
         {ICM_DTYPE_F64, ICM_STOP_FIXED, 24576, 300, 6, true},   {ICM_DTYPE_F64, ICM_STOP_FIXED, 24064, 300, 3, true},
         {ICM_DTYPE_F64, ICM_STOP_RILLING, 28160, 300, 4, false}, {ICM_DTYPE_F64, ICM_STOP_RILLING, 28160, 300, 5, true},
         {ICM_DTYPE_F32, ICM_STOP_FIXED, 32768, 300, 3, true},

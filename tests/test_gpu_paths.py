@@ -117,11 +117,11 @@ def test_more_series_than_workgroups(icm, dev, monkeypatch):
 
 @pytest.mark.parametrize("keep", [True, False])
 def test_phases_on_different_paths(icm, dev, monkeypatch, keep):
-    """4 x 32768, I = 20 in FP64: 20 noise-mode series launch step by step,
-    beside 80 series of the CEEMDAN phase in whole stages; replayed with other
+    """4 x 32768, I = 23, M = 6 in FP64: 23 noise-mode series launch step by step,
+    beside 92 series of the CEEMDAN phase in whole stages; replayed with other
     inputs, forward and adjoint, and equal to launches per step."""
     import torch
-    lens, I, M, S = [32768] * 4, 20, 4, 5
+    lens, I, M, S = [32768] * 4, 23, 6, 5
     print(f"case: phases on different paths keep={keep}", flush=True)
     kw = dict(dtype=torch.float64, max_sifts=S, device=dev, keep_records=keep)
     steps = _plan(icm, monkeypatch, STEPS, lens, I, M, use_graph=False, **kw)

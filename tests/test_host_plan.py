@@ -72,14 +72,14 @@ def test_default_tuning_given_back_keeps_the_stage_kernel(driver):
 
 
 def test_few_long_series_launch_step_by_step(driver):
-    """FP64 series of about 100 to 128 tiles, too few to fill the chip with a
-    workgroup each; nothing is tuned on either path."""
+    """Series of 56 tiles and up, too few for a workgroup each to be ahead at
+    their number of rows; nothing is tuned on either path."""
     driver("few_series")
 
 
 def test_long_series_of_few_rows_launch_step_by_step(driver):
-    """More FP64 series of 95 tiles and up than CUs, in a decomposition whose
-    dense first stages weigh most."""
+    """FP64 series of 95 tiles and up, too many for launches without tuning, in
+    a decomposition whose dense first stages weigh most."""
     driver("few_rows")
 
 
